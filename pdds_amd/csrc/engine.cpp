@@ -37,7 +37,10 @@ pdds_status fail(pdds_engine *e, pdds_status s, const std::string &msg) {
 // device address on each device comes from hipGetSymbolAddress (noalloc_scratch_of), and only
 // that address is ever handed to kernels or copies.
 // ---------------------------------------------------------------------------
-static __device__ __align__(256) unsigned char scratch[PDDS_NOALLOC_SCRATCH_BYTES];
+// Beside the bytes that callers may plan with, room for what a call's launch-side tables hold beyond
+// kKnotDescQuota (at most some 40,000 knots fit a call).
+static constexpr size_t kScratchSpare = (size_t)8 << 20;
+static __device__ __align__(256) unsigned char scratch[PDDS_NOALLOC_SCRATCH_BYTES + kScratchSpare];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -149,7 +152,7 @@ static void host_sigma(const pdds_problem *p, const PdeParams &pp, double x, dou
         case PDE_HELMHOLTZ: pde_coef<PDE_HELMHOLTZ, double>(x, y, hp, co); break;
         default: pde_coef<PDE_TABLE, double>(x, y, hp, co); break;
     }
-    s[0] = co.s00; s[1] = co.s01; s[2] = co.s10; s[3] = co.s11;
+    s[0] = co.s00; s[1] = 0.0; s[2] = 0.0; s[3] = co.s11;
 }
 
 // Step of a knot's paths: the run's h, or with adaptive_h the distance rule of
@@ -315,6 +318,14 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
                              tabs[t]->e1, tabs[t]->e2, tabs[t]->ipsi};
     TableDesc *dtab;
     if ((st = upload(e, B_TABLES, tdesc, &dtab))) return st;
+    // the global rectangle's centre and half-sides as rect_dist forms them, or the disc's radius
+    double gc[4] = {glob[2], 0.0, 0.0, 0.0};
+    if (geom != GeomDisc) {
+        gc[0] = 0.5 * (glob[0] + glob[2]);
+        gc[1] = 0.5 * (glob[1] + glob[3]);
+        gc[2] = glob[2] - gc[0];
+        gc[3] = glob[3] - gc[1];
+    }
     double kernel_ms = 0.0, reduce_ms = 0.0;
     int grid_used = 0, Pmax_all = 0;
     int64_t items_all = 0;
@@ -343,6 +354,9 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             kd[q].k2 = k.has_k2 ? k.k2 : pp.k2;
             kd[q].h = k.h > 0.0 ? k.h : knot_step(prob, pp, r, geom, sd.rect, sd.geo, k.x0, k.y0);
             kd[q].sqrth = std::sqrt(kd[q].h);
+            for (int i = 0; i < 6; ++i) kd[q].dom[i] = geom == GeomDisc ? sd.geo[i] : i < 4 ? sd.rect[i] : 0.0;
+            kd[q].gmask = sd.gmask;
+            kd[q].pad = 0;
             kd[q].item_begin = (int64_t)items.size();
             for (int64_t p0 = 0; p0 < k.n; p0 += P) {
                 ItemDesc it;
@@ -366,8 +380,17 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         const size_t shmem = reduce_lds_bytes(ne_cap, nnz_cap, S);
         if (shmem > 160 * 1024 || S > 65535)
             return fail(e, PDDS_ERR_UNSUPPORTED, "stencil or sub-batch too large for the LDS reduction buffers");
-        KnotDesc *dk; ItemDesc *dit;
+        // blocks of 2^kshift paths, about two per knot, each with its first path's knot (find_knot)
+        int kshift = 6;
+        while ((tot >> kshift) > std::max<int64_t>(64, 2 * (int64_t)nk)) ++kshift;
+        std::vector<int32_t> kblk((size_t)((tot - 1) >> kshift) + 2, nk - 1);
+        for (size_t b = 0, q = 0; b + 1 < kblk.size(); ++b) {
+            while ((int)q + 1 < nk && kd[q + 1].path_off <= (int64_t)b << kshift) ++q;
+            kblk[b] = (int32_t)q;
+        }
+        KnotDesc *dk; ItemDesc *dit; int32_t *dkblk;
         if ((st = upload(e, B_KNOTS, kd, &dk))) return st;
+        if ((st = upload(e, B_KBLK, kblk, &dkblk))) return st;
         if ((st = upload(e, B_ITEMS, items, &dit))) return st;
         Records rec;
         if ((st = dbuf(e, B_REC, (size_t)tot * sizeof(ExitRec), &p))) return st; rec.r = (ExitRec *)p;
@@ -408,30 +431,56 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         const size_t nctr = std::max<size_t>(kMaxQueues, patches.size());
         PatchDesc *dpatch = nullptr;
         if (tiled && (st = upload(e, B_PATCH, patches, &dpatch))) return st;
-        if ((st = dbuf(e, B_COUNTER, nctr * sizeof(unsigned long long), &p))) return st; dctr = (unsigned long long *)p;
-        HIPCHK(launch_fill_u64(dctr, (int64_t)nctr, 0ULL, e->stream));
+        if ((st = dbuf(e, B_COUNTER, nctr * kQueueStride * sizeof(unsigned long long), &p))) return st;
+        dctr = (unsigned long long *)p;
+        HIPCHK(launch_fill_u64(dctr, (int64_t)nctr * kQueueStride, 0ULL, e->stream));
         // path kernel
         PathKernelArgs pa;
         std::memset(&pa, 0, sizeof(pa));
         pa.knots = dk; pa.n_knots = nk; pa.tables = dtab; pa.total = tot; pa.base = 0; pa.counter = dctr; pa.rec = rec;
-        for (int i = 0; i < 4; ++i) pa.glob[i] = glob[i];
+        pa.kshift = kshift; pa.kblk = dkblk;
+        for (int i = 0; i < 4; ++i) pa.gc[i] = gc[i];
         pa.h = r->h; pa.sqrth = std::sqrt(r->h); pa.beta = r->beta;
-        pa.seed = r->seed; pa.stream = r->stream; pa.max_steps = max_steps; pa.pp = pp;
+        pa.seed = r->seed; pa.stream = r->stream; pa.max_steps = (uint32_t)max_steps; pa.pp = pp;
         pa.pool_chunk = 64 * (int64_t)(r->paths_per_lane > 0 ? r->paths_per_lane : 4);
-        int grid;
-        if (persistent) {
-            grid = r->grid_wgs > 0 ? r->grid_wgs : e->path_wgs_per_cu * e->n_cu;
-            grid = (int)std::max<int64_t>(1, std::min<int64_t>(grid, (tot + wg - 1) / wg));
-        } else {
-            grid = (int)std::min<int64_t>((tot + wg - 1) / wg, (int64_t)1 << 30);
-        }
-        pa.n_queues = persistent ? std::min(kMaxQueues, grid) : 1;
         pa.patches = dpatch;
         pa.n_patches = (int32_t)patches.size();
-        const int twg = path_tiled_wg(r->precision, r->step, geom);
+        const bool fp64 = r->precision == PDDS_FP64;
+        auto launch = [&](const PathLaunch &l) -> hipError_t {
+            return fp64 ? launch_path_f64(prob->pde, geom, persistent, mixed, l, pa)
+                        : launch_path_f32(prob->pde, geom, persistent, mixed, l, pa);
+        };
+        auto launched = [&](hipError_t lr) {
+            return lr == hipSuccess ? PDDS_OK : fail(e, PDDS_ERR_DEVICE, std::string("path launch: ") + hipGetErrorString(lr));
+        };
+        int grid;
+        pa.n_queues = 1;
         if (tiled) {
+            const int twg = path_tiled_wg(r->precision, r->step, geom);
             grid = r->grid_wgs > 0 ? r->grid_wgs
                                    : (int)std::max<int64_t>(1, std::min<int64_t>(e->n_cu, (tot + 8 * twg - 1) / (8 * twg)));
+        } else if (persistent) {
+            // one wave per SIMD as far as the paths fill it; more, up to what the card holds at once,
+            // while every lane has four paths one after another (lanes without a path cost as much as
+            // the others until the wave's last one ends)
+            int per_cu = 0;
+            if ((st = launched(launch(PathLaunch{0, wg, e->stream, &per_cu})))) return st;
+            const int64_t slots = 64;      // paths a wave carries at once
+            const int64_t per_wg = slots * (wg / 64), held = (int64_t)e->n_cu * std::max(1, per_cu);
+            const int64_t one = ((int64_t)e->n_cu * 4 + wg / 64 - 1) / (wg / 64);
+            const int64_t want = std::min(held, std::max(one, tot / (4 * per_wg)));
+            grid = (int)std::max<int64_t>(1, std::min<int64_t>(r->grid_wgs > 0 ? r->grid_wgs : want, (tot + per_wg - 1) / per_wg));
+            // the first paths of every wave are its own -- unless not all waves run at once, when
+            // these would wait for others to end -- and the rest goes out in chunks of a sixteenth
+            // of an even share
+            const int64_t share = tot / ((int64_t)grid * (wg / 64));
+            pa.n_queues = std::min(kMaxQueues, grid);
+            pa.queue_len = (tot + pa.n_queues - 1) / pa.n_queues;
+            pa.pool_first = grid <= held ? (int32_t)slots : 0;
+            pa.pool_chunk = r->paths_per_lane > 0 ? slots * r->paths_per_lane
+                                                  : std::max<int64_t>(std::min<int64_t>(slots, 16), std::min<int64_t>(256, share / 16));
+        } else {
+            grid = (int)std::min<int64_t>((tot + wg - 1) / wg, (int64_t)1 << 30);
         }
         grid_used = std::max(grid_used, grid);
         HIPCHK(hipEventRecord(e->ev[0], e->stream));
@@ -444,9 +493,8 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
                 lr = r->precision == PDDS_FP64 ? launch_path_tiled_f64(geom, mixed, g, lds_bytes, e->stream, pa)
                                                : launch_path_tiled_f32(geom, mixed, g, lds_bytes, e->stream, pa);
             else
-                lr = r->precision == PDDS_FP64 ? launch_path_f64(prob->pde, geom, persistent, mixed, g, wg, e->stream, pa)
-                                               : launch_path_f32(prob->pde, geom, persistent, mixed, g, wg, e->stream, pa);
-            if (lr != hipSuccess) return fail(e, PDDS_ERR_DEVICE, std::string("path launch: ") + hipGetErrorString(lr));
+                lr = launch(PathLaunch{g, wg, e->stream, nullptr});
+            if ((st = launched(lr))) return st;
         }
         HIPCHK(hipEventRecord(e->ev[1], e->stream));
         // reduction + finalize
@@ -459,14 +507,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         // exit sides: FP32 records carry them; FP64 exits are classified as write_exit does, on
         // the global rectangle's centre and half-sides (rect_dist's) or the disc's radius
         ra.side_mode = r->precision != PDDS_FP64 ? SIDE_BITS : geom == GeomDisc ? SIDE_DISC : SIDE_RECT;
-        if (geom == GeomDisc) {
-            ra.gc[0] = glob[2];
-        } else {
-            ra.gc[0] = 0.5 * (glob[0] + glob[2]);
-            ra.gc[1] = 0.5 * (glob[1] + glob[3]);
-            ra.gc[2] = glob[2] - ra.gc[0];
-            ra.gc[3] = glob[3] - ra.gc[1];
-        }
+        for (int i = 0; i < 4; ++i) ra.gc[i] = gc[i];
         const int64_t nit = (int64_t)items.size();
         for (int64_t base = 0; base < nit; base += (int64_t)1 << 30) {
             ra.item_base = base;
@@ -1352,7 +1393,7 @@ static pdds_status point_eval_locked(pdds_engine *e, const pdds_problem *p, cons
         // most 17 of them, P >= N / 16, each with its descriptor and statistics), with room for
         // alignment
         const int64_t need = paths * (int64_t)sizeof(ExitRec) +
-                             (int64_t)knots.size() * (int64_t)(sizeof(KnotDesc) + sizeof(KnotStat) + 16 +
+                             (int64_t)knots.size() * (int64_t)(kKnotDescQuota + sizeof(KnotStat) + 16 +
                                                                 17 * (sizeof(ItemDesc) + sizeof(ItemStat))) +
                              ((int64_t)1 << 16);
         if (need > (int64_t)PDDS_NOALLOC_SCRATCH_BYTES)
@@ -1370,7 +1411,7 @@ static pdds_status point_eval_locked(pdds_engine *e, const pdds_problem *p, cons
     if (noalloc) {
         Arena arena;
         arena.base = e->scratch;
-        arena.cap = PDDS_NOALLOC_SCRATCH_BYTES;
+        arena.cap = PDDS_NOALLOC_SCRATCH_BYTES + kScratchSpare;
         struct Scope {
             pdds_engine *e;
             ~Scope() { e->arena = nullptr; }

@@ -11,48 +11,38 @@ namespace pdds {
 __constant__ double kExp2TabDev[64] = PDDS_EXP2_TAB;   // 2^(j/64), j = 0..63
 
 template <int PDE, int GEOM, int FAM>
-static hipError_t path_f64_gf(bool persistent, bool mixed, int grid, int wg, hipStream_t s, const PathKernelArgs &a) {
-    if (!persistent)
-        hipLaunchKernelGGL((plain_kernel<double, PDE, GEOM, FAM>), dim3(grid), dim3(wg), 0, s, a);
-    else if (mixed)
-        hipLaunchKernelGGL((path_kernel<double, PDE, true, GEOM, FAM>), dim3(grid), dim3(wg), 0, s, a);
-    else
-        hipLaunchKernelGGL((path_kernel<double, PDE, false, GEOM, FAM>), dim3(grid), dim3(wg), 0, s, a);
-    return hipGetLastError();
+static hipError_t path_f64_gf(bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
+    if (!persistent) return l.go(plain_kernel<double, PDE, GEOM, FAM>, a);
+    return mixed ? l.go(path_kernel<double, PDE, true, GEOM, FAM>, a) : l.go(path_kernel<double, PDE, false, GEOM, FAM>, a);
 }
 
 // the default control-variate step has kernels of its own, without a family test in the loop
 template <int PDE, int GEOM>
-static hipError_t path_f64_g(bool persistent, bool mixed, int grid, int wg, hipStream_t s, const PathKernelArgs &a) {
-    return a.pp.step == STEP_CV ? path_f64_gf<PDE, GEOM, STEP_CV>(persistent, mixed, grid, wg, s, a)
-                                : path_f64_gf<PDE, GEOM, STEP_ANY>(persistent, mixed, grid, wg, s, a);
+static hipError_t path_f64_g(bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
+    if (a.pp.step != STEP_CV) return path_f64_gf<PDE, GEOM, STEP_ANY>(persistent, mixed, l, a);
+    return path_f64_gf<PDE, GEOM, STEP_CV>(persistent, mixed, l, a);
 }
 
 template <int PDE>
-static hipError_t path_f64(int geom, bool persistent, bool mixed, int grid, int wg, hipStream_t s,
-                          const PathKernelArgs &a) {
+static hipError_t path_f64(int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
     if (a.pp.refl) {
         // reflecting sides: rectangles, one stream and k2 per launch, every step family
         if (mixed || geom != GeomRect) return hipErrorInvalidValue;
-        if (!persistent)
-            hipLaunchKernelGGL((plain_kernel<double, PDE, GeomRect, STEP_ANY, true>), dim3(grid), dim3(wg), 0, s, a);
-        else
-            hipLaunchKernelGGL((path_kernel<double, PDE, false, GeomRect, STEP_ANY, true>), dim3(grid), dim3(wg), 0, s, a);
-        return hipGetLastError();
+        return persistent ? l.go(path_kernel<double, PDE, false, GeomRect, STEP_ANY, true>, a)
+                          : l.go(plain_kernel<double, PDE, GeomRect, STEP_ANY, true>, a);
     }
-    return geom == GeomDisc ? path_f64_g<PDE, GeomDisc>(persistent, mixed, grid, wg, s, a)
-                            : path_f64_g<PDE, GeomRect>(persistent, mixed, grid, wg, s, a);
+    return geom == GeomDisc ? path_f64_g<PDE, GeomDisc>(persistent, mixed, l, a)
+                            : path_f64_g<PDE, GeomRect>(persistent, mixed, l, a);
 }
 
-hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, int grid, int wg, hipStream_t s,
-                           const PathKernelArgs &a) {
+hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
     switch (pde) {
-        case PDE_MONEGROS: return path_f64<PDE_MONEGROS>(geom, persistent, mixed, grid, wg, s, a);
-        case PDE_SINSIN: return path_f64<PDE_SINSIN>(geom, persistent, mixed, grid, wg, s, a);
-        case PDE_VARCOEF: return path_f64<PDE_VARCOEF>(geom, persistent, mixed, grid, wg, s, a);
-        case PDE_VARCOEF_LUT: return path_f64<PDE_VARCOEF_LUT>(geom, persistent, mixed, grid, wg, s, a);
-        case PDE_HELMHOLTZ: return path_f64<PDE_HELMHOLTZ>(geom, persistent, mixed, grid, wg, s, a);
-        case PDE_TABLE: return path_f64<PDE_TABLE>(geom, persistent, mixed, grid, wg, s, a);
+        case PDE_MONEGROS: return path_f64<PDE_MONEGROS>(geom, persistent, mixed, l, a);
+        case PDE_SINSIN: return path_f64<PDE_SINSIN>(geom, persistent, mixed, l, a);
+        case PDE_VARCOEF: return path_f64<PDE_VARCOEF>(geom, persistent, mixed, l, a);
+        case PDE_VARCOEF_LUT: return path_f64<PDE_VARCOEF_LUT>(geom, persistent, mixed, l, a);
+        case PDE_HELMHOLTZ: return path_f64<PDE_HELMHOLTZ>(geom, persistent, mixed, l, a);
+        case PDE_TABLE: return path_f64<PDE_TABLE>(geom, persistent, mixed, l, a);
         default: return hipErrorInvalidValue;
     }
 }

@@ -58,9 +58,12 @@ PDDS_HD int classify_coord(const double rect[4], const double glob[4], double x,
 // |y - cy| - hy) inside the rectangle (its tie rule picks between equal values) and positive
 // outside, where that maximum is positive too, so for finite coordinates the global test is the
 // same comparison without the projection.
-PDDS_HD int classify_coord_c(const double rect[4], const double gc[4], double x, double y) {
+PDDS_HD bool classify_global_c(const double gc[4], double x, double y) {
     const double ax = __builtin_fabs(x - gc[0]) - gc[2], ay = __builtin_fabs(y - gc[1]) - gc[3];
-    if (__builtin_fmax(ax, ay) >= -1e-8) return 4;
+    return __builtin_fmax(ax, ay) >= -1e-8;
+}
+PDDS_HD int classify_coord_c(const double rect[4], const double gc[4], double x, double y) {
+    if (classify_global_c(gc, x, y)) return 4;
     if (__builtin_fabs(y - rect[1]) < 1e-8) return 1;
     if (__builtin_fabs(y - rect[3]) < 1e-8) return 0;
     if (__builtin_fabs(x - rect[0]) < 1e-8) return 3;
@@ -142,15 +145,40 @@ template <class R> struct PathState {
 // Y += c Y h + Y mu . dW and the drift of X loses sigma mu.
 // LT: the step carries local-time terms lz = psi Y L and ly = varphi Y L of a reflecting side
 // (Integrators/FKACIntegrator.hpp:156-158: Z += f Y h + psi Y L, Y += c Y h + varphi Y L).
-template <class R, int FAM, bool LT = false>
+// the move b h + s i of one coordinate (FP32: the drift's product fused into the sum)
+__device__ __forceinline__ double em_move(double b, double h, double s, double i) { return b * h + s * i; }
+__device__ __forceinline__ float em_move(float b, float h, float s, float i) { return __builtin_fmaf(b, h, s * i); }
+// a i + b j (FP32: the first product fused into the sum)
+__device__ __forceinline__ double em_dot(double a, double i, double b, double j) { return a * i + b * j; }
+__device__ __forceinline__ float em_dot(float a, float i, float b, float j) { return __builtin_fmaf(a, i, b * j); }
+// FP32 kernels compiled from the general form with sigma's off-diagonal zeros written out: the
+// run-time step families, reflecting sides and the Monegros problem.  Which products the compiler
+// fuses in FP32 follows from the shape of the expressions, and a path's values from that; these
+// keep the shape they had, while the control-variate step of the other problems is written with
+// its fused products and without the zeros.
+template <class R, int PDE, int FAM, bool REFL> constexpr bool zero_terms() {
+    return sizeof(R) == 4 && (FAM != STEP_CV || REFL || PDE == PDE_MONEGROS);
+}
+
+template <class R, int PDE, int FAM, bool LT = false>
 __device__ __forceinline__ void em_step(PathState<R> &s, const Coef<R> &co, R h, R sqrth, R n1, R n2, int fam,
                                         R lz = (R)0, R ly = (R)0) {
+    constexpr bool zeros = zero_terms<R, PDE, FAM, LT>();
+    constexpr R s01 = (R)0, s10 = (R)0;
     R i0 = sqrth * n1, i1 = sqrth * n2;
     const bool vrcv = FAM != STEP_CV && fam == STEP_VRCV;
-    R v0 = -(co.s00 * co.g0 + co.s10 * co.g1);
-    R v1 = -(co.s01 * co.g0 + co.s11 * co.g1);
+    R v0, v1;
+    if constexpr (zeros) {
+        v0 = -(co.s00 * co.g0 + s10 * co.g1);
+        v1 = -(s01 * co.g0 + co.s11 * co.g1);
+    } else {
+        v0 = -(co.s00 * co.g0);
+        v1 = -(co.s11 * co.g1);
+    }
     if (vrcv) { v0 = co.F0; v1 = co.F1; }
-    R dxi = s.Y * (v0 * i0 + v1 * i1);
+    R dxi;
+    if constexpr (zeros) dxi = s.Y * (v0 * i0 + v1 * i1);
+    else dxi = s.Y * em_dot(v1, i1, v0, i0);
     R dz = co.f * s.Y * h;
     if constexpr (LT) dz = dz + lz;
     const bool vr = FAM != STEP_CV && fam == STEP_VR;
@@ -170,17 +198,59 @@ __device__ __forceinline__ void em_step(PathState<R> &s, const Coef<R> &co, R h,
         R dy = co.c * Yold * h + (vrcv ? Yold * (m0 * i0 + m1 * i1) : dxi);
         if constexpr (LT) dy = dy + ly;
         s.Y = Yold + dy;
-        b0 = b0 - (co.s00 * m0 + co.s01 * m1);
-        b1 = b1 - (co.s10 * m0 + co.s11 * m1);
+        if constexpr (zeros) {
+            b0 = b0 - (co.s00 * m0 + s01 * m1);
+            b1 = b1 - (s10 * m0 + co.s11 * m1);
+        } else {
+            b0 = b0 - co.s00 * m0;
+            b1 = b1 - co.s11 * m1;
+        }
     } else {
         R dy = co.c * Yold * h;
         if constexpr (LT) dy = dy + ly;
         s.Y = Yold + dy;
     }
-    R nx = s.x + (b0 * h + (co.s00 * i0 + co.s01 * i1));
-    R ny = s.y + (b1 * h + (co.s10 * i0 + co.s11 * i1));
-    s.x = nx;
-    s.y = ny;
+    if constexpr (zeros) {
+        R nx = s.x + (b0 * h + (co.s00 * i0 + s01 * i1));
+        R ny = s.y + (b1 * h + (s10 * i0 + co.s11 * i1));
+        s.x = nx;
+        s.y = ny;
+    } else {
+        s.x = s.x + em_move(b0, h, co.s00, i0);
+        s.y = s.y + em_move(b1, h, co.s11, i1);
+    }
+}
+
+// |N^T sigma| for an outward normal (nx, ny)
+template <class R, int PDE, int FAM, bool REFL> __device__ __forceinline__ R normal_sigma(R nx, R ny, const Coef<R> &co) {
+    if constexpr (zero_terms<R, PDE, FAM, REFL>()) {
+        constexpr R s01 = (R)0, s10 = (R)0;
+        const R ga = nx * co.s00 + ny * s10;
+        const R gb = nx * s01 + ny * co.s11;
+        return RM<R>::sqrt(ga * ga + gb * gb);
+    } else {
+        const R ga = nx * co.s00, gb = ny * co.s11;
+        return RM<R>::sqrt(em_dot(ga, ga, gb, gb));
+    }
+}
+
+// The FP32 normals of steps 2 call and 2 call + 1 of a path (n[0], n[1] and n[2], n[3]).
+__device__ __forceinline__ void normals4_f32(uint32_t call, uint32_t path, uint32_t knot, uint32_t seed,
+                                             uint32_t stream, float n[4]) {
+    Philox4 w = philox4x32_10(call, path, knot, 0u, seed, stream);
+    // u = (k + 1/2) 2^-24 as one fma (one rounding of the same exact value as k + 1/2);
+    // -2 ln u = (-2 ln 2) log2 u with the hardware log2
+    const float sc = 5.9604644775390625e-08f, half = 2.98023223876953125e-08f;
+    float u1 = __builtin_fmaf((float)(w.v[0] >> 8), sc, half);
+    float u2 = __builtin_fmaf((float)(w.v[1] >> 8), sc, half);
+    float u3 = __builtin_fmaf((float)(w.v[2] >> 8), sc, half);
+    float u4 = __builtin_fmaf((float)(w.v[3] >> 8), sc, half);
+    float r1 = RM<float>::sqrt(__builtin_amdgcn_logf(u1) * -1.3862943611198906f);
+    float r2 = RM<float>::sqrt(__builtin_amdgcn_logf(u3) * -1.3862943611198906f);
+    n[0] = r1 * __builtin_amdgcn_cosf(u2);
+    n[1] = r1 * __builtin_amdgcn_sinf(u2);
+    n[2] = r2 * __builtin_amdgcn_cosf(u4);
+    n[3] = r2 * __builtin_amdgcn_sinf(u4);
 }
 
 // Normal pair of step s.st for this lane's path.  FP32: one Philox call per even step gives
@@ -197,21 +267,10 @@ __device__ __forceinline__ void draw_normals(PathState<R> &s, uint32_t seed, uin
         n1 = a; n2 = b;
     } else {
         if (even) {
-            const uint32_t call = s.st >> 1;
-            Philox4 w = philox4x32_10(call, s.path, knot, 0u, seed, stream);
-            // u = (k + 1/2) 2^-24 as one fma (one rounding of the same exact value as k + 1/2);
-            // -2 ln u = (-2 ln 2) log2 u with the hardware log2
-            const float sc = 5.9604644775390625e-08f, half = 2.98023223876953125e-08f;
-            float u1 = __builtin_fmaf((float)(w.v[0] >> 8), sc, half);
-            float u2 = __builtin_fmaf((float)(w.v[1] >> 8), sc, half);
-            float u3 = __builtin_fmaf((float)(w.v[2] >> 8), sc, half);
-            float u4 = __builtin_fmaf((float)(w.v[3] >> 8), sc, half);
-            float r1 = RM<float>::sqrt(__builtin_amdgcn_logf(u1) * -1.3862943611198906f);
-            float r2 = RM<float>::sqrt(__builtin_amdgcn_logf(u3) * -1.3862943611198906f);
-            n1 = r1 * __builtin_amdgcn_cosf(u2);
-            n2 = r1 * __builtin_amdgcn_sinf(u2);
-            s.pn1 = r2 * __builtin_amdgcn_cosf(u4);
-            s.pn2 = r2 * __builtin_amdgcn_sinf(u4);
+            float n[4];
+            normals4_f32(s.st >> 1, s.path, knot, seed, stream, n);
+            n1 = n[0]; n2 = n[1];
+            s.pn1 = n[2]; s.pn2 = n[3];
         } else {
             n1 = s.pn1;
             n2 = s.pn2;
@@ -260,7 +319,8 @@ __device__ __forceinline__ void refl_step(PathState<R> &s, const Coef<R> &co, co
     R L = (R)0;
     if (lep) {
         const R i0 = sqrth * n1, i1 = sqrth * n2;
-        const R ga = nx * co.s00 + ny * co.s10, gb = nx * co.s01 + ny * co.s11;
+        constexpr R s01 = (R)0, s10 = (R)0;
+        const R ga = nx * co.s00 + ny * s10, gb = nx * s01 + ny * co.s11;
         const R uc = (ga * i0 + gb * i1) + (nx * co.b0 + ny * co.b1) * h;
         const R M = (R)0.5 * (uc + RM<R>::sqrt((ga * ga + gb * gb) * (((R)2.0 * h) * E) + uc * uc));
         L = RM<R>::fmax((R)0, M + d);
@@ -276,12 +336,17 @@ __device__ __forceinline__ void refl_step(PathState<R> &s, const Coef<R> &co, co
         lz = (psi * s.Y) * w;
         ly = (phi * s.Y) * w;
     }
-    em_step<R, FAM, true>(s, co, h, sqrth, n1, n2, fam, lz, ly);
+    em_step<R, PDE, FAM, true>(s, co, h, sqrth, n1, n2, fam, lz, ly);
     if (lep) {
         s.x = s.x - L * nx;
         s.y = s.y - L * ny;
     }
 }
+
+// The value is in its register here.  After a branch that loads, a wait for the loads at the first
+// use behind it would wait for the exit records just stored as well (one counter), on every pass,
+// also those that load nothing; with the use inside the branch only the passes that load wait.
+template <class T> __device__ __forceinline__ void loaded(T &v) { __asm__ volatile("" : "+v"(v)); }
 
 // Wave iterations on which a lane may start a path: FP32 paths start only on odd iterations,
 // so that a stepping lane's step count has the parity of the iteration; FP64 paths any time.
@@ -296,11 +361,12 @@ __device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v) 
 }
 
 // Knot of global path g: the last knot whose first path is <= g.
-__device__ __forceinline__ int find_knot(const KnotDesc *knots, int n_knots, int64_t g) {
-    int lo = 0, hi = n_knots;
+__device__ __forceinline__ int find_knot(const PathKernelArgs &a, int64_t g) {
+    const int b = (int)(g >> a.kshift);
+    int lo = a.kblk[b], hi = a.kblk[b + 1] + 1;
     while (hi - lo > 1) {
         int mid = (lo + hi) >> 1;
-        if (knots[mid].path_off <= g) lo = mid;
+        if (a.knots[mid].path_off <= g) lo = mid;
         else hi = mid;
     }
     return lo;
@@ -309,13 +375,18 @@ __device__ __forceinline__ int find_knot(const KnotDesc *knots, int n_knots, int
 // Exit record of a stopped path at batch slot g: the exit projection, Y and the score
 // (Z + xi, plus Y g(X) for a global-boundary exit, Reduce_Analytic
 // Solvers/EMFKACSolver.hpp:559-566); FP32 paths also put their exit side in Y's low bits.
+// (an FP64 path's side is found again by the reduction: here only whether the exit is global
+// matters, classify_coord's and classify_sector's first test)
 template <class R, int PDE, int GEOM>
-__device__ __forceinline__ void write_exit(const PathKernelArgs &a, uint32_t g, const PathState<R> &s,
-                                           const R *dom, int gmask, R ex, R ey, int kind) {
-    int side;
+__device__ __forceinline__ void write_exit(const PathKernelArgs &a, uint32_t g, const PathState<R> &s, int gmask, R ex,
+                                           R ey, int kind) {
+    int side = 4;
     if constexpr (sizeof(R) == 8) {
-        if constexpr (GEOM == GeomDisc) side = classify_sector(dom, a.glob[2], (double)ex, (double)ey);
-        else side = classify_coord(dom, a.glob, (double)ex, (double)ey);
+        const double x = (double)ex, y = (double)ey;
+        bool global;
+        if constexpr (GEOM == GeomDisc) global = __builtin_sqrt(x * x + y * y) >= a.gc[0] - 1e-8;
+        else global = classify_global_c(a.gc, x, y);
+        if (!global) side = 0;
     } else {
         side = classify_kind(kind, gmask);
     }
@@ -343,7 +414,7 @@ struct KnotSteps {
     unsigned long long st;    // steps
     uint32_t cap;             // paths stopped by the step cap while inside
 
-    __device__ __forceinline__ void init() { k = 0; st = 0ULL; cap = 0u; }
+    __device__ __forceinline__ void init() { k = -1; st = 0ULL; cap = 0u; }
     __device__ __forceinline__ void flush(const PathKernelArgs &a) {
         if (st) {
             atomicAdd(a.rec.kacc + 2 * (int64_t)k, st);
@@ -352,12 +423,10 @@ struct KnotSteps {
             cap = 0u;
         }
     }
-    // the lane takes a path of knot kn
+    // the lane goes on to paths of knot kn
     __device__ __forceinline__ void enter(const PathKernelArgs &a, int kn) {
-        if (kn != k) {
-            flush(a);
-            k = kn;
-        }
+        flush(a);
+        k = kn;
     }
 };
 
@@ -366,10 +435,6 @@ template <class R, int GEOM>
 __device__ __forceinline__ R domain_dist(const R *dom, R x, R y, R &ex, R &ey, R &nx, R &ny, int &kind) {
     if constexpr (GEOM == GeomDisc) return sector_dist<R>(dom, x, y, ex, ey, nx, ny, kind);
     else return rect_dist<R>(dom, x, y, ex, ey, nx, ny, kind);
-}
-template <int GEOM> __device__ __forceinline__ const double *domain_of(const StencilDesc &sd) {
-    if constexpr (GEOM == GeomDisc) return sd.geo;
-    else return sd.rect;
 }
 template <int GEOM> constexpr int domain_len() { return GEOM == GeomDisc ? 6 : 4; }
 
@@ -384,13 +449,20 @@ template <int GEOM> constexpr int domain_len() { return GEOM == GeomDisc ? 6 : 4
 // side reflects; only absorbing sides stop it.
 template <class R, int PDE, bool MIXED, int GEOM, int FAM, bool REFL = false>
 struct Walker {
+    // rectangles without reflecting sides: the stopping test without branches, the exit projection
+    // and side formed by the stopping lanes alone; fast: also lanes that are not stepping kept out by
+    // what they hold (below) instead of a select per state variable
+    static constexpr bool fast = GEOM == GeomRect && !REFL && !zero_terms<R, PDE, FAM, REFL>();
+    static constexpr bool branchless = GEOM == GeomRect && !REFL && !fast;   // its distance alone
     PathState<R> s;
     Coef<R> co;            // coefficients at the current X
     R pn1, pn2;            // normals of step s.st (the next step)
-    R rect[domain_len<GEOM>()];   // stopping domain in path precision (FP64 classifies on it)
+    R x0, y0;              // start point of the lane's knot
+    R dom[domain_len<GEOM>()];    // stopping domain in path precision; fast: its RectC
     uint32_t kid;
     int gmask;
     uint32_t g;            // batch path index (record slot; a batch holds fewer than 2^32 paths)
+    uint32_t poff;         // batch index of the knot's first path
     uint32_t kstream;      // Philox key word 1 of the path's knot
     R k2;                  // Helmholtz parameter of the path's knot
     R hk, sqhk;            // step of the path's knot and its square root
@@ -399,48 +471,68 @@ struct Walker {
     // local time
     int rmask, rk;
     R rd, rnx, rny, lt;
-    KnotSteps ks;          // steps of the lane's stopped paths not yet added to their knot's counters
+    KnotSteps ks;          // the lane's knot, and the steps of its stopped paths not yet added to its counters
 
     __device__ __forceinline__ void init() {
-        pn1 = 0; pn2 = 0; kid = 0; kstream = 0; gmask = 0; g = 0; k2 = 0; hk = 0; sqhk = 0;
+        // (a lane's first step, with zero coefficients, still takes the normals: they must be finite)
+        pn1 = 0; pn2 = 0; s.pn1 = 0; s.pn2 = 0; kid = 0; kstream = 0; gmask = 0; g = 0; poff = 0; k2 = 0; hk = 0; sqhk = 0;
         active = false; fresh = false;
         rmask = 0; rk = 0; rd = 0; rnx = 0; rny = 0; lt = 0;
         ks.init();
     }
 
-    // take path gg of the batch; k is its knot
+    // take path gg of the batch; k is its knot.  A lane's next path is mostly one of the same knot,
+    // whose data the lane still holds: the start then reads no memory.
     __device__ __forceinline__ void start(const PathKernelArgs &a, int64_t gg, int k) {
-        ks.enter(a, k);
-        const KnotDesc &kd = a.knots[k];
-        const StencilDesc &sd = a.tables[kd.table].sten[kd.stencil];
-        const double *dom = domain_of<GEOM>(sd);
-        for (int q = 0; q < domain_len<GEOM>(); ++q) rect[q] = (R)dom[q];
-        gmask = sd.gmask;
-        kid = kd.knot_id;
-        if constexpr (MIXED) {
-            kstream = kd.stream;
-            k2 = (R)kd.k2;
-            hk = (R)kd.h;
-            sqhk = (R)kd.sqrth;
+        if (k != ks.k) {
+            ks.enter(a, k);
+            const KnotDesc &kd = a.knots[k];
+            R d[domain_len<GEOM>()];
+            for (int q = 0; q < domain_len<GEOM>(); ++q) d[q] = (R)kd.dom[q];
+            if constexpr (fast) {
+                const RectC<R> c = rect_centre<R>(d);
+                dom[0] = c.cx; dom[1] = c.cy; dom[2] = c.hx; dom[3] = c.hy;
+            } else {
+                for (int q = 0; q < domain_len<GEOM>(); ++q) dom[q] = d[q];
+            }
+            gmask = kd.gmask;
+            kid = kd.knot_id;
+            poff = (uint32_t)kd.path_off;
+            x0 = (R)kd.x0; y0 = (R)kd.y0;
+            if constexpr (MIXED) {
+                kstream = kd.stream;
+                k2 = (R)kd.k2;
+                hk = (R)kd.h;
+                sqhk = (R)kd.sqrth;
+            }
+            if constexpr (REFL) rmask = kd.gmask & a.pp.refl;   // stencil sides on reflecting global sides
+            loaded(x0); loaded(y0); loaded(poff); loaded(kid); loaded(gmask);
+            for (int q = 0; q < domain_len<GEOM>(); ++q) loaded(dom[q]);
+            if constexpr (MIXED) { loaded(kstream); loaded(k2); loaded(hk); loaded(sqhk); }
         }
-        if constexpr (REFL) {
-            rmask = sd.gmask & a.pp.refl;   // stencil sides on reflecting global sides
-            lt = (R)0;
-        }
+        if constexpr (REFL) lt = (R)0;
         g = (uint32_t)gg;
-        s.path = (uint32_t)(gg - kd.path_off);
-        s.x = (R)kd.x0; s.y = (R)kd.y0;
+        s.path = g - poff;
+        s.x = x0; s.y = y0;
         s.Y = (R)1; s.Z = (R)0; s.xi = (R)0; s.zc = (R)0; s.xc = (R)0;
-        s.st = 0;
         active = true;
-        fresh = true;
+        if constexpr (fast) {
+            // the first iteration only evaluates the coefficients at X0: a step with zero
+            // coefficients adds exact zeros and takes the step count from -1 to 0
+            co = Coef<R>{};
+            s.st = ~0u;
+        } else {
+            s.st = 0;
+            fresh = true;
+        }
     }
 
     // One step for every lane, as one straight-line block (a lane that is not stepping
     // computes and discards), so the LUT loads of the new X are issued together and overlap
     // the next step's normal draw, which does not depend on X.  Inactive lanes hold stale or
-    // unset state: they touch no memory except the LUT, whose coordinates are clamped into
-    // the table.  A lane whose path stops writes its exit record and goes inactive.
+    // unset state and, on rectangles, go on moving with it: they touch no memory except the LUT,
+    // whose coordinates are clamped into the table, and start() sets whatever a path needs.  A lane
+    // whose path stops writes its exit record and goes inactive.
     // DRAW_FIRST: draw this step's normals at its start instead of overlapping the next
     // step's draw with the LUT reads (for LDS-resident LUT tiles, whose reads are short).
     // it: the wave's iteration count (stepping lanes have s.st of its parity)
@@ -449,9 +541,13 @@ struct Walker {
         const R h = MIXED ? hk : (R)a.h, sqrth = MIXED ? sqhk : (R)a.sqrth, beta = (R)a.beta;
         const uint32_t strm = MIXED ? kstream : a.stream;
         const R kk2 = MIXED ? k2 : (R)a.pp.k2;
-        const bool stepping = active && !fresh;
+        bool stepping = active && !fresh;
         if constexpr (DRAW_FIRST) draw_normals<R>(s, a.seed, strm, kid, pn1, pn2, (it & 1) == 0);
-        {
+        if constexpr (fast) {
+            em_step<R, PDE, FAM>(s, co, h, sqrth, pn1, pn2, a.pp.step);
+            s.st += 1u;
+            stepping = active && s.st != 0u;
+        } else {
             PathState<R> t = s;
             if constexpr (REFL) {
                 // the nearest side at the current X reflects: the Lepingle step within rho of it
@@ -461,7 +557,7 @@ struct Walker {
                 if (stepping && lep) E = draw_exponential<R>(s.st, s.path, a.seed, strm, kid);
                 refl_step<R, PDE, FAM>(t, co, a.pp, h, sqrth, pn1, pn2, a.pp.step, lep, E, rnx, rny, rd, lt);
             } else {
-                em_step<R, FAM>(t, co, h, sqrth, pn1, pn2, a.pp.step);
+                em_step<R, PDE, FAM>(t, co, h, sqrth, pn1, pn2, a.pp.step);
             }
             s.x = stepping ? t.x : s.x;
             s.y = stepping ? t.y : s.y;
@@ -472,18 +568,21 @@ struct Walker {
                 s.zc = stepping ? t.zc : s.zc;
                 s.xc = stepping ? t.xc : s.xc;
             }
-            s.st += stepping ? 1 : 0;
+            s.st += stepping ? 1u : 0u;
         }
         R ex, ey, nx, ny;
         int kind = 0;
-        // the stopping test needs only the distance and the nearest side's normal; on a rectangle
-        // without reflecting sides those come without branches, and the exit projection and side
-        // are formed below for the stopping lanes alone
-        constexpr bool fast = GEOM == GeomRect && !REFL;
         R d;
-        if constexpr (fast) d = rect_dist_inside<R>(rect, s.x, s.y, nx, ny);
-        else d = domain_dist<R, GEOM>(rect, s.x, s.y, ex, ey, nx, ny, kind);
-        bool rnow = false;
+        bool xside = false, rnow = false;
+        RectC<R> rc{};
+        if constexpr (fast) {
+            rc = RectC<R>{dom[0], dom[1], dom[2], dom[3]};
+            d = rect_dist_inside<R>(rc, s.x, s.y, xside);
+        } else if constexpr (branchless) {
+            d = rect_dist_inside<R>(dom, s.x, s.y, nx, ny);
+        } else {
+            d = domain_dist<R, GEOM>(dom, s.x, s.y, ex, ey, nx, ny, kind);
+        }
         if constexpr (REFL) {
             // past a reflecting side: back onto it, the distance becoming local time for the next
             // step (Inside's reflect outcome, Integrators/FKACIntegrator.hpp:189-207)
@@ -493,25 +592,29 @@ struct Walker {
                 lt = d;
                 s.x = ex;
                 s.y = ey;
-                d = domain_dist<R, GEOM>(rect, s.x, s.y, ex, ey, nx, ny, kind);
+                d = domain_dist<R, GEOM>(dom, s.x, s.y, ex, ey, nx, ny, kind);
                 rnow = refl_kind(kind, rmask);
             }
             rd = d; rk = kind; rnx = nx; rny = ny;
         }
-        pde_coef_t<PDE, R, TILED, FAM>(s.x, s.y, a.pp, T, kk2, co);
+        pde_coef_t<PDE, R, TILED, FAM>(s.x, s.y, a.pp, T, kk2, co, active);
         if constexpr (!DRAW_FIRST) draw_normals<R>(s, a.seed, strm, kid, pn1, pn2, (it & 1) != 0);
-        const R ga = nx * co.s00 + ny * co.s10;
-        const R gb = nx * co.s01 + ny * co.s11;
-        const R nrm = RM<R>::sqrt(ga * ga + gb * gb);
+        R nrm;
+        if constexpr (fast) {
+            nrm = side_norm(xside, co.s00, co.s11);
+        } else {
+            nrm = normal_sigma<R, PDE, FAM, REFL>(nx, ny, co);
+        }
         // a reflecting nearest side never stops the path
         const bool go = rnow || d < beta * nrm * sqrth;
-        const bool capped = (int64_t)s.st >= a.max_steps;
+        const bool capped = s.st >= a.max_steps;
         if (stepping && (!go || capped)) {
-            if constexpr (fast) {
+            if constexpr (fast) rect_exit<R>(rc, s.x, s.y, ex, ey, kind);
+            if constexpr (branchless) {
                 R tx, ty;
-                (void)rect_dist<R>(rect, s.x, s.y, ex, ey, tx, ty, kind);
+                (void)rect_dist<R>(dom, s.x, s.y, ex, ey, tx, ty, kind);
             }
-            write_exit<R, PDE, GEOM>(a, g, s, rect, gmask, ex, ey, kind);
+            write_exit<R, PDE, GEOM>(a, g, s, gmask, ex, ey, kind);
             ks.st += s.st;
             ks.cap += capped && go ? 1u : 0u;
             active = false;
@@ -520,8 +623,8 @@ struct Walker {
     }
 };
 
-// Wave-private pool of consecutive paths [next, end) taken a.pool_chunk at a time from one
-// queue (one atomic per a.pool_chunk paths: 64 lanes x the run's paths per lane).  With it, the knot of the pool's first path and
+// Wave-private pool of consecutive paths [next, end), taken a.pool_chunk at a time from one queue
+// (one atomic per chunk).  With it, the knot of the pool's first path and
 // where that knot ends, found once per chunk with wave-uniform values; a lane whose path
 // lies past that knot searches for its own.
 struct WavePool {
@@ -529,22 +632,24 @@ struct WavePool {
     int ck = 0;
     int64_t ck_end = 0;
 
+    // the paths [s0, s0 + n) cut at qe
+    __device__ __forceinline__ bool set(const PathKernelArgs &a, int64_t s0, int64_t n, int64_t qe) {
+        if (s0 >= qe) return false;
+        next = s0;
+        end = s0 + n < qe ? s0 + n : qe;
+        ck = find_knot(a, s0);
+        ck_end = ck + 1 < a.n_knots ? a.knots[ck + 1].path_off : a.total;
+        return true;
+    }
     // a fresh chunk from counter over [qb, qe); false if that queue is drained
     __device__ __forceinline__ bool take(const PathKernelArgs &a, unsigned long long *counter, int64_t qb,
                                          int64_t qe, int lane) {
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd(counter, (unsigned long long)a.pool_chunk);
-        base = uniform_u64(base);
-        const int64_t s0 = qb + (int64_t)base;
-        if (s0 >= qe) return false;
-        next = s0;
-        end = s0 + a.pool_chunk < qe ? s0 + a.pool_chunk : qe;
-        ck = find_knot(a.knots, a.n_knots, s0);
-        ck_end = ck + 1 < a.n_knots ? a.knots[ck + 1].path_off : a.total;
-        return true;
+        return set(a, qb + (int64_t)uniform_u64(base), a.pool_chunk, qe);
     }
     __device__ __forceinline__ int knot_of(const PathKernelArgs &a, int64_t gg) const {
-        return gg < ck_end ? ck : find_knot(a.knots, a.n_knots, gg);
+        return gg < ck_end ? ck : find_knot(a, gg);
     }
     // start paths on the lanes that need one; lanes left without a path once `drained`
     // is set are marked done
@@ -566,6 +671,39 @@ struct WavePool {
     }
 };
 
+// The queues of a persistent launch as one wave sees them (PathKernelArgs).
+struct PathQueues {
+    WavePool pool;
+    int q, tried = 0;
+    bool drained = false;
+
+    __device__ __forceinline__ int64_t begin(const PathKernelArgs &a, int i) const { return (int64_t)i * a.queue_len; }
+    __device__ __forceinline__ int64_t finish(const PathKernelArgs &a, int i) const {
+        const int64_t e = (int64_t)(i + 1) * a.queue_len;
+        return e < a.total ? e : a.total;
+    }
+    // the wave's own first paths
+    __device__ __forceinline__ void init(const PathKernelArgs &a) {
+        q = (int)(blockIdx.x % (unsigned)a.n_queues);
+        const int w = (int)(blockIdx.x / (unsigned)a.n_queues) * (int)(blockDim.x >> 6) +
+                      __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        (void)pool.set(a, begin(a, q) + (int64_t)w * a.pool_first, a.pool_first, finish(a, q));
+    }
+    // a chunk for an empty pool, from the wave's queue or the next one with paths left
+    __device__ __forceinline__ void refill(const PathKernelArgs &a, int lane) {
+        while (pool.next >= pool.end && !drained) {
+            const int wgs = (int)((gridDim.x + (unsigned)a.n_queues - 1u - (unsigned)q) / (unsigned)a.n_queues);
+            const int64_t qb = begin(a, q) + (int64_t)wgs * (int)(blockDim.x >> 6) * a.pool_first;
+            unsigned long long *c = a.counter + q * kQueueStride;
+            // (a drained queue is seen without an atomic)
+            const unsigned long long taken = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (qb + (int64_t)uniform_u64(taken) < finish(a, q) && pool.take(a, c, qb, finish(a, q), lane)) break;
+            if (++tried >= a.n_queues) drained = true;
+            else q = q + 1 == a.n_queues ? 0 : q + 1;
+        }
+    }
+};
+
 // ----------------------------------------------------------------------------
 // Persistent path kernel: one path per lane, lanes refilled from XCD-local queues
 // ----------------------------------------------------------------------------
@@ -584,22 +722,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(path_w
     bool done = false;
     // The wave starts on its XCD's queue, so the paths (and LUT texels) of one XCD's L2
     // stay in one contiguous range of knots; a drained queue sends the wave on to the next.
-    WavePool pool;
-    bool drained = false;
-    int q = (int)(blockIdx.x % (unsigned)a.n_queues);
-    int tried = 0;
+    PathQueues qs;
+    qs.init(a);
     for (int it = 1;; ++it) {
         const bool can_start = may_start<R>(it);
         if (can_start) {
             const bool need = !w.active && !done;
             const unsigned long long m = __ballot(need);
             if (m) {
-                while (pool.next >= pool.end && !drained) {
-                    if (pool.take(a, a.counter + q, a.total * q / a.n_queues, a.total * (q + 1) / a.n_queues, lane)) break;
-                    if (++tried >= a.n_queues) drained = true;
-                    else q = q + 1 == a.n_queues ? 0 : q + 1;
-                }
-                pool.hand_out(a, w, need, m, drained, done, lane);
+                qs.refill(a, lane);
+                qs.pool.hand_out(a, w, need, m, qs.drained, done, lane);
             }
         }
         if (!__any(w.active)) {
@@ -628,14 +760,12 @@ template <class R, int PDE, int GEOM, int FAM, bool REFL = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_waves<R, FAM>()))) plain_kernel(PathKernelArgs a) {
     const int64_t gg = a.base + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gg >= a.total) return;
-    const int kn = find_knot(a.knots, a.n_knots, gg);
+    const int kn = find_knot(a, gg);
     const KnotDesc &kd = a.knots[kn];
-    const StencilDesc &sd = a.tables[kd.table].sten[kd.stencil];
     const LutTile none{nullptr, 0, 0, 0, 0};
     const R h = (R)kd.h, sqrth = (R)kd.sqrth, beta = (R)a.beta, k2 = (R)kd.k2;
     R rect[domain_len<GEOM>()];
-    const double *dom = domain_of<GEOM>(sd);
-    for (int q = 0; q < domain_len<GEOM>(); ++q) rect[q] = (R)dom[q];
+    for (int q = 0; q < domain_len<GEOM>(); ++q) rect[q] = (R)kd.dom[q];
     PathState<R> s;
     s.path = (uint32_t)(gg - kd.path_off);
     s.x = (R)kd.x0; s.y = (R)kd.y0;
@@ -647,7 +777,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
     int kind;
     // REFL: reflecting sides, the nearest side at the current X and the pending local time (as
     // in Walker::step)
-    const int rmask = REFL ? (sd.gmask & a.pp.refl) : 0;
+    const int rmask = REFL ? (kd.gmask & a.pp.refl) : 0;
     R rd = (R)0, rnx = (R)0, rny = (R)0, lt = (R)0;
     int rk = 0;
     if constexpr (REFL) rd = domain_dist<R, GEOM>(rect, s.x, s.y, ex, ey, rnx, rny, rk);
@@ -660,7 +790,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
             const R E = lep ? draw_exponential<R>(s.st, s.path, a.seed, kd.stream, kd.knot_id) : (R)0;
             refl_step<R, PDE, FAM>(s, co, a.pp, h, sqrth, n1, n2, a.pp.step, lep, E, rnx, rny, rd, lt);
         } else {
-            em_step<R, FAM>(s, co, h, sqrth, n1, n2, a.pp.step);
+            em_step<R, PDE, FAM>(s, co, h, sqrth, n1, n2, a.pp.step);
         }
         s.st += 1;
         R d = domain_dist<R, GEOM>(rect, s.x, s.y, ex, ey, nx, ny, kind);
@@ -678,13 +808,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
             rd = d; rk = kind; rnx = nx; rny = ny;
         }
         pde_coef_t<PDE, R, false, FAM>(s.x, s.y, a.pp, none, k2, co);
-        const R ga = nx * co.s00 + ny * co.s10;
-        const R gb = nx * co.s01 + ny * co.s11;
-        const R nrm = RM<R>::sqrt(ga * ga + gb * gb);
+        const R nrm = normal_sigma<R, PDE, FAM, REFL>(nx, ny, co);
         go = rnow || d < beta * nrm * sqrth;
-        capped = (int64_t)s.st >= a.max_steps;
+        capped = s.st >= a.max_steps;
     } while (go && !capped);
-    write_exit<R, PDE, GEOM>(a, (uint32_t)gg, s, rect, sd.gmask, ex, ey, kind);
+    write_exit<R, PDE, GEOM>(a, (uint32_t)gg, s, kd.gmask, ex, ey, kind);
     // steps and step-cap stops into the knot's counters: one wave sum and one atomic per counter
     // when all 64 lanes hold paths of one knot, else an atomic per lane
     const bool cap = capped && go;
@@ -741,15 +869,26 @@ path_kernel_tiled(PathKernelArgs a) {
     // first patch: the one holding this work-group's share of the batch's path range
     int p = find_patch(a.patches, a.n_patches, (int64_t)blockIdx.x * a.total / (int64_t)gridDim.x);
     while (true) {
-        if (threadIdx.x == 0) {
+        if (threadIdx.x < 64) {
+            // the next patch with paths left, 64 counters at a time
             int pick = -1;
-            for (int k = 0; k < a.n_patches; ++k) {
-                const int c = p + k < a.n_patches ? p + k : p + k - a.n_patches;
-                const PatchDesc &pd = a.patches[c];
-                const unsigned long long taken = __hip_atomic_load(a.counter + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((int64_t)taken < pd.pend - pd.pbeg) { pick = c; break; }
+            for (int k0 = 0; k0 < a.n_patches && pick < 0; k0 += 64) {
+                const int k = k0 + lane;
+                int c = p + k;
+                c = c < a.n_patches ? c : c - a.n_patches;
+                bool left = false;
+                if (k < a.n_patches) {
+                    const unsigned long long taken =
+                        __hip_atomic_load(a.counter + c * kQueueStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    left = (int64_t)taken < a.patches[c].pend - a.patches[c].pbeg;
+                }
+                const unsigned long long m = __ballot(left);
+                if (m) {
+                    pick = p + k0 + __builtin_ctzll(m);
+                    pick = pick < a.n_patches ? pick : pick - a.n_patches;
+                }
             }
-            s_patch = pick;
+            if (lane == 0) s_patch = pick;
         }
         __syncthreads();
         p = __builtin_amdgcn_readfirstlane(s_patch);   // uniform: the patch, its tile and queue stay scalar
@@ -773,7 +912,7 @@ path_kernel_tiled(PathKernelArgs a) {
                 const unsigned long long m = __ballot(need);
                 if (m) {
                     if (pool.next >= pool.end && !drained)
-                        if (!pool.take(a, a.counter + p, pd.pbeg, pd.pend, lane)) drained = true;
+                        if (!pool.take(a, a.counter + p * kQueueStride, pd.pbeg, pd.pend, lane)) drained = true;
                     pool.hand_out(a, w, need, m, drained, done, lane);
                 }
             }
@@ -833,7 +972,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) p
                 const R E = lep ? draw_exponential<R>(s.st, s.path, a.seed, a.stream, a.knot) : (R)0;
                 refl_step<R, PDE, FAM>(s, co, a.pp, h, sqrth, n1, n2, a.pp.step, lep, E, rnx, rny, rd, lt);
             } else {
-                em_step<R, FAM>(s, co, h, sqrth, n1, n2, a.pp.step);
+                em_step<R, PDE, FAM>(s, co, h, sqrth, n1, n2, a.pp.step);
             }
             s.st += 1;
             R d = rect_dist<R>(rect, s.x, s.y, ex, ey, nx, ny, kind);
@@ -851,9 +990,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) p
                 rd = d; rk = kind; rnx = nx; rny = ny;
             }
             pde_coef<PDE, R, FAM>(s.x, s.y, a.pp, co);
-            R ga = nx * co.s00 + ny * co.s10;
-            R gb = nx * co.s01 + ny * co.s11;
-            R nrm = RM<R>::sqrt(ga * ga + gb * gb);
+            R nrm = normal_sigma<R, PDE, FAM, REFL>(nx, ny, co);
             go = (rnow || d < beta * nrm * sqrth) && ((int64_t)(s.st - st0) < a.max_steps);
         }
         double *o[5];

@@ -22,6 +22,9 @@ inline size_t reduce_lds_bytes(int ne_cap, int nnz_cap, int S) {
 // Y: a float widened to double leaves the low 29 bits of its mantissa zero.
 constexpr uint64_t kSideBitsMask = 7ULL;
 constexpr int kMaxQueues = 8;              // path queues: one per XCD of an MI355X (8 XCDs x 32 CUs)
+// 64-bit words between two queue counters: atomics of one cache line wait for each other across the
+// XCDs (about 130 ns each)
+constexpr int kQueueStride = 32;
 
 // One Monte Carlo knot of an assembly batch.
 struct KnotDesc {
@@ -37,6 +40,11 @@ struct KnotDesc {
     int64_t item_count;
     double k2;              // Helmholtz parameter of the knot's problem
     double h, sqrth;        // Euler-Maruyama step of the knot's paths (the run's, or its adaptive h)
+    // the knot's stopping domain and the sides of it on the global boundary, copied from its
+    // stencil (StencilDesc rect or geo, gmask): a lane starts a path with one load instead of three
+    // that wait for each other
+    double dom[6];
+    int32_t gmask, pad;
 };
 
 // One distinct stencil: stopping rectangle, four side lists (N,S,E,W), Psi^-1 per side,
@@ -86,6 +94,11 @@ struct KnotStat {
     unsigned long long cnt[6];
 };
 
+// Bytes of a knot's descriptor where a call's device memory is estimated ahead of it (serving
+// admission, pdds_point_eval_noalloc).  What a descriptor has beyond them and the block table of the
+// knots are launch-side copies of a few dozen bytes a knot and stay out of these limits.
+constexpr int64_t kKnotDescQuota = 96;
+
 // Per-path exit records, indexed by global path index: the FP64 exit values as one aligned
 // 32-byte record (a lane stores it with two 16-byte writes when its path stops, so a record
 // reaches memory as one 32-byte piece).  The exit side is not stored for FP64 paths: the
@@ -113,23 +126,31 @@ struct PatchDesc {
 struct PathKernelArgs {
     const KnotDesc *knots;
     int32_t n_knots;
+    // knot of the first path of every block of 2^kshift paths, and of the last path at the end:
+    // bounds of the search for a path's knot
+    int32_t kshift;
+    const int32_t *kblk;
     const TableDesc *tables;
     int64_t total;          // paths in the batch
     int64_t base;           // plain launches: first path of this launch
-    // persistent launches: queue q serves paths [q*total/n_queues, (q+1)*total/n_queues)
-    // through counter[q]; work-group b starts on queue b % n_queues (the XCD it is
-    // dispatched to) and moves to the next queue when its own is drained
+    // persistent launches: queue q serves paths [q queue_len, (q + 1) queue_len) of the batch;
+    // work-group b starts on queue b % n_queues (the XCD it is dispatched to) and moves to the next
+    // queue when its own is drained.  The first pool_first paths of each wave of a queue are its own
+    // (no atomic where a launch starts, with every wave at once); those behind them are handed out
+    // pool_chunk at a time through counter[q kQueueStride].
     unsigned long long *counter;
     int32_t n_queues;
-    int64_t pool_chunk;     // paths a wave takes from a queue at once (64 x paths per lane)
-    // LDS-tiled launches: one queue per patch (counter[p] counts paths handed out of patch p)
+    int32_t pool_first;
+    int64_t queue_len;
+    int64_t pool_chunk;     // paths a wave takes from a queue at once
+    // LDS-tiled launches: one queue per patch (counter[p kQueueStride] counts paths handed out of patch p)
     const struct PatchDesc *patches;
     int32_t n_patches;
     Records rec;
-    double glob[4];
+    double gc[4];           // the global rectangle's centre and half-sides, or the disc's radius
     double h, sqrth, beta;
     uint32_t seed, stream;
-    int64_t max_steps;
+    uint32_t max_steps;     // below 2^27
     PdeParams pp;
 };
 
@@ -185,14 +206,25 @@ struct PathsArgs {
     int64_t *steps2;
 };
 
+// A path launch: with per_cu set nothing is launched, and the work-groups of the kernel that a CU
+// holds at once are put there (a persistent grid is sized by them).
+struct PathLaunch {
+    int grid, wg;
+    hipStream_t stream;
+    int *per_cu;
+    template <class K> hipError_t go(K kernel, const PathKernelArgs &a) const {
+        if (per_cu) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, kernel, wg, 0);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), 0, stream, a);
+        return hipGetLastError();
+    }
+};
+
 // Launchers (defined in engine_f64.hip / engine_f32.hip)
 hipError_t launch_path_tiled_f64(int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
 hipError_t launch_path_tiled_f32(int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
 int path_tiled_wg(int precision, int step, int geom);   // block size of the LDS-tiled kernel
-hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, int grid, int wg, hipStream_t s,
-                           const PathKernelArgs &a);
-hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, int grid, int wg, hipStream_t s,
-                           const PathKernelArgs &a);
+hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
+hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_reduce(int grid, int wg, size_t shmem, hipStream_t s, const ReduceArgs &a);
 hipError_t launch_paths_f64(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);
 hipError_t launch_paths_f32(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);

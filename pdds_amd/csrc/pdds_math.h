@@ -110,7 +110,43 @@ PDDS_HD double dexp_core(double x) {
     const double k = __builtin_floor(x * kLog2e + 0.5);
     double r = __builtin_fma(-k, kLn2Hi, x);
     r = __builtin_fma(-k, kLn2Lo, r);
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_ldexp(exp_poly(r), (int)k);   // one v_ldexp_f64
+#else
     return exp_poly(r) * pow2i((int)k);
+#endif
+}
+
+// a / b for |b| in [1, 4] and a = 0 or 2^-100 < |a| < 4: the correctly rounded quotient from the
+// reciprocal, two Newton steps and the remainder -- the compiler's own division without the operand
+// scaling and special cases that such operands do not need (8 instructions instead of 12)
+PDDS_HD double div_near1(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+#else
+    return a / b;
+#endif
+}
+
+// sqrt(x) for x = 0 or 2^-700 < x < 2^700, correctly rounded: the compiler's own iteration from the
+// reciprocal square root without its rescaling of tiny arguments (11 instructions instead of 17; the
+// bound on the start value keeps x = 0 out of 0 * infinity)
+PDDS_HD double sqrt_mid(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_fmin(__builtin_amdgcn_rsq(__builtin_fabs(x)), 0x1p+400);
+    double g = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+#else
+    return __builtin_sqrt(x);
+#endif
 }
 
 // dexp(x) bit for bit: the short path where the result is normal, a branch to dexp elsewhere
@@ -214,10 +250,13 @@ PDDS_HD double dexprel(double x) { return x == 0.0 ? 1.0 : dexpm1(x) / x; }
 // their logs take this path directly, without dlog's special-case tests.
 PDDS_HD double dlog_core(double x, int sub) {
     const uint64_t b = f64_bits(x);
-    int e = (int)((b >> 52) & 0x7ff) + sub - 1023;
-    double m = f64_from((b & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
-    if (m > 1.4142135623730951) { m *= 0.5; e += 1; }
-    double s = (m - 1.0) / (m + 1.0);
+    const uint32_t hi = (uint32_t)(b >> 32);
+    uint32_t mh = (hi & 0x000fffffu) | 0x3ff00000u;
+    const bool big = f64_from(((uint64_t)mh << 32) | (uint32_t)b) > 1.4142135623730951;
+    mh -= big ? 0x00100000u : 0u;                        // m / 2
+    const int e = (int)(hi >> 20) + sub - (big ? 1022 : 1023);
+    const double m = f64_from(((uint64_t)mh << 32) | (uint32_t)b);
+    double s = div_near1(m - 1.0, m + 1.0);
     double s2 = s * s;
     // s^2 <= 0.0295: the atanh series terms past s^23 are below 1e-2 ulp
     // (Horner steps through fma_k: one instruction each, the coefficient from scalar registers)
@@ -270,17 +309,18 @@ PDDS_HD void sincospi_kernel(double r, double &s, double &c) {
     c = fma_k(pc, y2, 1.0);
 }
 
-// sin(pi x), cos(pi x); |x| < 2^52 assumed (path coordinates and uniforms)
+// sin(pi x), cos(pi x); |x| < 2^50 assumed (path coordinates and uniforms)
 PDDS_HD void dsincospi(double x, double &sp, double &cp) {
     double k = __builtin_floor(2.0 * x + 0.5);
     double r = x - 0.5 * k;
     double s, c;
     sincospi_kernel(r, s, c);
-    int q = ((int)(int64_t)k) & 3;
-    double a = (q & 1) ? c : s;
-    double b = (q & 1) ? -s : c;
-    sp = (q & 2) ? -a : a;
-    cp = (q & 2) ? -b : b;
+    // k mod 4 from the low bits of k + 1.5 2^52; quadrants swap s and c and flip their signs
+    const uint32_t q = (uint32_t)f64_bits(k + 0x1.8p+52);
+    const bool odd = (q & 1u) != 0u;
+    const uint64_t a = f64_bits(odd ? c : s), b = f64_bits(odd ? s : c);
+    sp = f64_from(a ^ ((uint64_t)((q << 30) & 0x80000000u) << 32));
+    cp = f64_from(b ^ ((uint64_t)(((q + 1u) << 30) & 0x80000000u) << 32));
 }
 PDDS_HD double x_over_pi(double x) { return __builtin_fma(x, kInvPiHi, x * kInvPiLo); }
 PDDS_HD void dsincos(double x, double &s, double &c) { dsincospi(x_over_pi(x), s, c); }
@@ -372,9 +412,11 @@ PDDS_HD Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3
     return o;
 }
 
+// (m + 1/2) 2^-53 of the 53-bit m = a 2^21 + (b >> 11): the fused form rounds the same exact value
+// once, as the conversion of m, the sum and the scaling by a power of two do
 PDDS_HD double u01_53(uint32_t a, uint32_t b) {
-    uint64_t m = ((uint64_t)a << 21) | (uint64_t)(b >> 11);
-    return ((double)m + 0.5) * 1.1102230246251565e-16;
+    const double lo = __builtin_fma((double)(b >> 11), 0x1p-53, 0x1p-54);   // exact
+    return __builtin_fma((double)a, 0x1p-32, lo);
 }
 
 // FP64 normal pair for one step: one Philox draw, Box-Muller on 53-bit uniforms.
@@ -383,7 +425,7 @@ PDDS_HD void normals_f64(uint32_t seed, uint32_t stream, uint32_t knot, uint32_t
     Philox4 w = philox4x32_10((uint32_t)step, path, knot, (uint32_t)(step >> 32), seed, stream);
     double u1 = u01_53(w.v[0], w.v[1]);
     double u2 = u01_53(w.v[2], w.v[3]);
-    double r = __builtin_sqrt(-2.0 * dlog_core(u1, 0));
+    double r = sqrt_mid(-2.0 * dlog_core(u1, 0));   // 0 or within [2^-53, 75]
     double s, c;
     dsincospi(2.0 * u2, s, c);
     n1 = r * c;
@@ -432,10 +474,27 @@ PDDS_HD R rect_dist(const R p[4], R x, R y, R &ex, R &ey, R &nx, R &ny, int &kin
     return dy - hy;
 }
 
+// A rectangle by its centre and half-sides, rect_dist's own cx = 0.5 (x0 + x1), hx = x1 - cx.
+template <class R> struct RectC { R cx, cy, hx, hy; };
+template <class R> PDDS_HD RectC<R> rect_centre(const R p[4]) {
+    RectC<R> c;
+    c.cx = (R)0.5 * (p[0] + p[2]); c.cy = (R)0.5 * (p[1] + p[3]);
+    c.hx = p[2] - c.cx; c.hy = p[3] - c.cy;
+    return c;
+}
+
 // What the stopping test needs of rect_dist, without branches: inside the rectangle its signed
-// distance and outward normal, bit for bit (same operations, same tie rule); outside a positive
-// distance (the largest side excess, which is not rect_dist's corner distance) -- a point there
-// stops whatever its value, and the exit projection comes from rect_dist itself.
+// distance and whether the nearest side is one of constant x, bit for bit (same operations, same tie
+// rule); outside a positive distance (the largest side excess, which is not rect_dist's corner
+// distance) -- a point there stops whatever its value, and the exit projection comes from rect_exit.
+template <class R> PDDS_HD R rect_dist_inside(const RectC<R> &p, R x, R y, bool &xside) {
+    const R ax = RM<R>::fabs(x - p.cx) - p.hx, ay = RM<R>::fabs(y - p.cy) - p.hy;
+    xside = ax > ay;
+    return xside ? ax : ay;
+}
+
+// The same with the outward normal of that side, for the kernels that step with zero terms
+// (zero_terms in engine_kernels.h).
 template <class R>
 PDDS_HD R rect_dist_inside(const R p[4], R x, R y, R &nx, R &ny) {
     const R cx = (R)0.5 * (p[0] + p[2]), cy = (R)0.5 * (p[1] + p[3]);
@@ -447,6 +506,32 @@ PDDS_HD R rect_dist_inside(const R p[4], R x, R y, R &nx, R &ny) {
     nx = xside ? sxs : (R)0;
     ny = xside ? (R)0 : sys;
     return xside ? ax : ay;
+}
+
+// |N^T sigma| of a diagonal sigma at the nearest side: |s00| or |s11| in FP64, where the square root
+// of the rounded square is the value itself; FP32 keeps the square and the hardware root.  The other
+// entry enters with weight 0, so that a coefficient that is not finite still gives NaN.
+PDDS_HD double side_norm(bool xside, double s00, double s11) {
+    const double wx = f64_from((uint64_t)(xside ? 0x3ff00000u : 0u) << 32);
+    const double wy = f64_from((uint64_t)(xside ? 0u : 0x3ff00000u) << 32);
+    return __builtin_fabs(__builtin_fma(s11, wy, s00 * wx));
+}
+__device__ __forceinline__ float side_norm(bool xside, float s00, float s11) {
+    const float t = __builtin_fmaf(s11, xside ? 0.0f : 1.0f, s00 * (xside ? 1.0f : 0.0f));
+    return RM<float>::sqrt(t * t);
+}
+
+// rect_dist's projection and side of a point on the rectangle p
+template <class R> PDDS_HD void rect_exit(const RectC<R> &p, R x, R y, R &ex, R &ey, int &kind) {
+    const R dx = RM<R>::fabs(x - p.cx), dy = RM<R>::fabs(y - p.cy);
+    const bool right = x > p.cx, top = y > p.cy;
+    const R px = right ? p.hx + p.cx : (R)-1 * p.hx + p.cx, py = top ? p.hy + p.cy : (R)-1 * p.hy + p.cy;
+    const bool corner = dx > p.hx && dy > p.hy;
+    const bool inside = dx <= p.hx && dy <= p.hy;
+    const bool xside = inside ? dx - p.hx > dy - p.hy : dx > p.hx;
+    ex = corner || xside ? px : x;
+    ey = corner || !xside ? py : y;
+    kind = corner ? (top ? (right ? 4 : 5) : (right ? 6 : 7)) : xside ? (right ? 2 : 3) : (top ? 0 : 1);
 }
 
 // Signed distance to the annular sector g = {r0, r1, cos a, sin a, cos b, sin b}: radii
@@ -615,11 +700,12 @@ PDDS_HD void lut_accum(const LutView &L, const LutTile &T, lds_float4 *tp, bool 
 //   sum_b wy_b * sum_a wx_a * C[clamp(j-1+b)][clamp(i-1+a)][f]
 // With TILED, a lane whose 4x4 taps lie inside the tile reads fields 0..3 from LDS (one
 // 16-byte LDS read per tap) and the others read them from plane a; the values, and the
-// order of the fused multiply-adds, are the same either way.  A wave whose lanes are all
+// order of the fused multiply-adds, are the same either way.  A wave whose live lanes are all
 // inside the tile takes a path with LDS reads only, so no LDS read waits for the wave's
 // global loads.
 template <class R, int NF, bool TILED>
-PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF]) {
+PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF], bool live = true) {
+    (void)live;
     static_assert(NF <= 8, "at most 8 fields per texel");
     R t = (x - (R)L.ox) * (R)L.sx;
     R v = (y - (R)L.oy) * (R)L.sy;
@@ -638,7 +724,7 @@ PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF])
         const bool in = lc >= 0 && lr >= 0 && lc + 3 < T.tw && lr + 3 < T.th;
         lds_float4 *tp = T.lds + (in ? lr * T.pitch + lc : 0);
 #if defined(__HIP_DEVICE_COMPILE__)
-        if (__all(in)) lut_accum<NF, 1>(L, T, tp, in, t0, wx, wy, acc);
+        if (__all(in || !live)) lut_accum<NF, 1>(L, T, tp, in, t0, wx, wy, acc);
         else lut_accum<NF, 2>(L, T, tp, in, t0, wx, wy, acc);
 #else
         lut_accum<NF, 2>(L, T, tp, in, t0, wx, wy, acc);

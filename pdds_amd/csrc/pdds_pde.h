@@ -16,7 +16,7 @@ enum PdeId { PDE_MONEGROS = 0, PDE_SINSIN = 1, PDE_VARCOEF = 2, PDE_VARCOEF_LUT 
 enum StepFamily { STEP_ANY = -1, STEP_CV = 0, STEP_PLAIN = 1, STEP_VR = 2, STEP_VRCV = 3 };
 
 template <class R> struct Coef {
-    R s00, s01, s10, s11;  // sigma, row-major
+    R s00, s11;            // sigma = diag(s00, s11)
     R b0, b1;
     R c, f;
     R g0, g1;              // grad u
@@ -62,21 +62,22 @@ template <int PDE, class R> PDDS_HD R pde_g(R x, R y, const PdeParams &P);
 
 // TILED: the coefficient LUT's fields 0..3 are read from the LDS tile T where it covers X.
 // k2: the Helmholtz parameter of this path's problem (per knot, so one launch can carry
-// requests with different k^2).
+// requests with different k^2).  live: whether the caller uses this lane's values.
 template <int PDE, class R, bool TILED, int FAM = STEP_CV>
-PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Coef<R> &co) {
+PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Coef<R> &co, bool live = true) {
     (void)T;
+    (void)live;
     if constexpr (PDE == PDE_MONEGROS) {
         R u, gx, gy, lap;
         monegros<R>(x, y, u, gx, gy, lap);
-        co.s00 = (R)1.41421356237; co.s01 = 0; co.s10 = 0; co.s11 = (R)1.41421356237;
+        co.s00 = (R)1.41421356237; co.s11 = (R)1.41421356237;
         co.b0 = 0; co.b1 = 0; co.c = (R)-0.0; co.f = -lap;
         co.g0 = gx; co.g1 = gy;
     } else if constexpr (PDE == PDE_SINSIN || PDE == PDE_HELMHOLTZ) {
         R sx, cx, sy, cy;
         RM<R>::sincospi(x, sx, cx);
         RM<R>::sincospi(y, sy, cy);
-        co.s00 = (R)1.4142135623730951; co.s01 = 0; co.s10 = 0; co.s11 = (R)1.4142135623730951;
+        co.s00 = (R)1.4142135623730951; co.s11 = (R)1.4142135623730951;
         co.b0 = 0; co.b1 = 0;
         co.g0 = (R)3.141592653589793 * cx * sy + (R)2.0 * x;
         co.g1 = (R)3.141592653589793 * sx * cy + (R)2.0 * y;
@@ -93,7 +94,7 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
         // from its samples alone
         R v[8];
         lut_eval<R, 8>(P.lut, x, y, v);
-        co.s00 = v[0]; co.s01 = 0; co.s10 = 0; co.s11 = v[1];
+        co.s00 = v[0]; co.s11 = v[1];
         co.b0 = v[2]; co.b1 = v[3]; co.c = v[4]; co.f = v[5];
         co.g0 = v[6]; co.g1 = v[7];
     } else {  // VARCOEF, VARCOEF_LUT
@@ -110,14 +111,14 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
         co.f = -fcfg;
         co.g0 = uu; co.g1 = uy;
         if constexpr (PDE == PDE_VARCOEF) {
-            co.s00 = s1; co.s01 = 0; co.s10 = 0; co.s11 = s2;
+            co.s00 = s1; co.s11 = s2;
             co.b0 = (R)0.2 * y + (R)0.3 * s1 * cxn;
             co.b1 = (R)-0.2 * x - (R)0.3 * s2 * syn;
             co.c = -((R)1.0 + x * x);
         } else {
             R v[5];
-            lut_eval_t<R, 5, TILED>(P.lut, T, x, y, v);
-            co.s00 = v[0]; co.s01 = 0; co.s10 = 0; co.s11 = v[1];
+            lut_eval_t<R, 5, TILED>(P.lut, T, x, y, v, live);
+            co.s00 = v[0]; co.s11 = v[1];
             co.b0 = v[2]; co.b1 = v[3]; co.c = v[4];
         }
     }

@@ -36,7 +36,7 @@ constexpr int64_t kRecordBytes = (int64_t)sizeof(ExitRec);
 // device bytes per work item of a knot besides its records and partials: the item's descriptor
 // and statistics, and (counted per item, an over-estimate) the knot's descriptor, statistics and
 // step counters
-constexpr int64_t kKnotBytes = (int64_t)(sizeof(KnotDesc) + sizeof(KnotStat) + 2 * sizeof(unsigned long long) +
+constexpr int64_t kKnotBytes = kKnotDescQuota + (int64_t)(sizeof(KnotStat) + 2 * sizeof(unsigned long long) +
                                          sizeof(ItemDesc) + sizeof(ItemStat));
 
 struct SrvReq {
