@@ -251,6 +251,19 @@ void lut_tile_of(const LutView &L, const double rect[4], int &c0, int &r0, int &
     span(rect[1], rect[3], L.oy, L.sy, L.ny, py, r0, th);
 }
 
+// Lanes that carry one path of a launch of the group kernel.  One lane is the cheapest per step (the
+// step-ordered sums are repeated by every lane of a group), 16 finish a path soonest.  With one lane
+// a card holds 1024 to 2048 paths per CU; it pays once every lane has several paths one after
+// another, and below that a launch lasts as long as its longest path.  Measured on 256 CUs:
+// FP32 Helmholtz server burst (15.5 M paths) 83 ms with one lane, 119 with four; FP32 Poisson
+// assembly (0.6 M) 3.4 and 3.5; FP64 Helmholtz assembly (1.9 M) 2.5 and 3.1, FP64 recorded run
+// (0.77 M) 4.0 and 3.6; with four and sixteen lanes: 140 k FP32 paths 1.25 and 1.16 ms, 5000 FP64
+// paths 0.73 and 0.58, 4000 0.34 and 0.29.
+static int group_lanes(int n_cu, bool fp64, int64_t tot) {
+    if (tot >= (int64_t)n_cu * (fp64 ? 4096 : 2048)) return 1;
+    return tot > (int64_t)n_cu * 32 ? 4 : 16;
+}
+
 pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const double glob[4],
                          const std::vector<const DevTables *> &tabs, const std::vector<AsmKnot> &knots,
                          int64_t n_vals, double *G_host, double *Gvar_host, AsmOut &out, const double *W_host) {
@@ -446,13 +459,17 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         pa.patches = dpatch;
         pa.n_patches = (int32_t)patches.size();
         const bool fp64 = r->precision == PDDS_FP64;
+        const int lanes = persistent && geom == GeomRect && pp.refl == 0 && pp.step == STEP_CV && group_pde(prob->pde, r->precision)
+                              ? group_lanes(e->n_cu, fp64, tot) : 0;
         auto launch = [&](const PathLaunch &l) -> hipError_t {
+            if (lanes) return fp64 ? launch_group_f64(prob->pde, mixed, lanes, l, pa) : launch_group_f32(prob->pde, mixed, lanes, l, pa);
             return fp64 ? launch_path_f64(prob->pde, geom, persistent, mixed, l, pa)
                         : launch_path_f32(prob->pde, geom, persistent, mixed, l, pa);
         };
         auto launched = [&](hipError_t lr) {
             return lr == hipSuccess ? PDDS_OK : fail(e, PDDS_ERR_DEVICE, std::string("path launch: ") + hipGetErrorString(lr));
         };
+        const int kwg = lanes ? 256 : wg;   // work-group of the path kernel (not the tiled one)
         int grid;
         pa.n_queues = 1;
         if (tiled) {
@@ -464,16 +481,16 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             // while every lane has four paths one after another (lanes without a path cost as much as
             // the others until the wave's last one ends)
             int per_cu = 0;
-            if ((st = launched(launch(PathLaunch{0, wg, e->stream, &per_cu})))) return st;
-            const int64_t slots = 64;      // paths a wave carries at once
-            const int64_t per_wg = slots * (wg / 64), held = (int64_t)e->n_cu * std::max(1, per_cu);
-            const int64_t one = ((int64_t)e->n_cu * 4 + wg / 64 - 1) / (wg / 64);
+            if ((st = launched(launch(PathLaunch{0, kwg, e->stream, &per_cu})))) return st;
+            const int64_t slots = lanes ? 64 / lanes : 64;      // paths a wave carries at once
+            const int64_t per_wg = slots * (kwg / 64), held = (int64_t)e->n_cu * std::max(1, per_cu);
+            const int64_t one = ((int64_t)e->n_cu * 4 + kwg / 64 - 1) / (kwg / 64);
             const int64_t want = std::min(held, std::max(one, tot / (4 * per_wg)));
             grid = (int)std::max<int64_t>(1, std::min<int64_t>(r->grid_wgs > 0 ? r->grid_wgs : want, (tot + per_wg - 1) / per_wg));
             // the first paths of every wave are its own -- unless not all waves run at once, when
             // these would wait for others to end -- and the rest goes out in chunks of a sixteenth
             // of an even share
-            const int64_t share = tot / ((int64_t)grid * (wg / 64));
+            const int64_t share = tot / ((int64_t)grid * (kwg / 64));
             pa.n_queues = std::min(kMaxQueues, grid);
             pa.queue_len = (tot + pa.n_queues - 1) / pa.n_queues;
             pa.pool_first = grid <= held ? (int32_t)slots : 0;
@@ -493,7 +510,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
                 lr = r->precision == PDDS_FP64 ? launch_path_tiled_f64(geom, mixed, g, lds_bytes, e->stream, pa)
                                                : launch_path_tiled_f32(geom, mixed, g, lds_bytes, e->stream, pa);
             else
-                lr = launch(PathLaunch{g, wg, e->stream, nullptr});
+                lr = launch(PathLaunch{g, kwg, e->stream, nullptr});
             if ((st = launched(lr))) return st;
         }
         HIPCHK(hipEventRecord(e->ev[1], e->stream));

@@ -151,6 +151,10 @@ __device__ __forceinline__ float em_move(float b, float h, float s, float i) { r
 // a i + b j (FP32: the first product fused into the sum)
 __device__ __forceinline__ double em_dot(double a, double i, double b, double j) { return a * i + b * j; }
 __device__ __forceinline__ float em_dot(float a, float i, float b, float j) { return __builtin_fmaf(a, i, b * j); }
+// s i rounded by itself (FP32: not fused into the sum that takes it)
+__device__ __forceinline__ double em_scale(double s, double i) { return s * i; }
+__device__ __forceinline__ float em_scale(float s, float i) { return __builtin_fmaf(s, i, 0.0f); }
+
 // FP32 kernels compiled from the general form with sigma's off-diagonal zeros written out: the
 // run-time step families, reflecting sides and the Monegros problem.  Which products the compiler
 // fuses in FP32 follows from the shape of the expressions, and a path's values from that; these

@@ -225,6 +225,10 @@ hipError_t launch_path_tiled_f32(int geom, bool mixed, int grid, size_t lds, hip
 int path_tiled_wg(int precision, int step, int geom);   // block size of the LDS-tiled kernel
 hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
+// const-motion problems on rectangles, control-variate step: `lanes` (1, 4 or 16) lanes per path
+bool group_pde(int pde, int precision);
+hipError_t launch_group_f64(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a);
+hipError_t launch_group_f32(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_reduce(int grid, int wg, size_t shmem, hipStream_t s, const ReduceArgs &a);
 hipError_t launch_paths_f64(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);
 hipError_t launch_paths_f32(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);
