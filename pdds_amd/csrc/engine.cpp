@@ -251,17 +251,24 @@ void lut_tile_of(const LutView &L, const double rect[4], int &c0, int &r0, int &
     span(rect[1], rect[3], L.oy, L.sy, L.ny, py, r0, th);
 }
 
-// Lanes that carry one path of a launch of the group kernel.  One lane is the cheapest per step (the
-// step-ordered sums are repeated by every lane of a group), 16 finish a path soonest.  With one lane
-// a card holds 1024 to 2048 paths per CU; it pays once every lane has several paths one after
-// another, and below that a launch lasts as long as its longest path.  Measured on 256 CUs:
-// FP32 Helmholtz server burst (15.5 M paths) 83 ms with one lane, 119 with four; FP32 Poisson
-// assembly (0.6 M) 3.4 and 3.5; FP64 Helmholtz assembly (1.9 M) 2.5 and 3.1, FP64 recorded run
-// (0.77 M) 4.0 and 3.6; with four and sixteen lanes: 140 k FP32 paths 1.25 and 1.16 ms, 5000 FP64
-// paths 0.73 and 0.58, 4000 0.34 and 0.29.
-static int group_lanes(int n_cu, bool fp64, int64_t tot) {
-    if (tot >= (int64_t)n_cu * (fp64 ? 4096 : 2048)) return 1;
-    return tot > (int64_t)n_cu * 32 ? 4 : 16;
+// Grid of a persistent path launch of `tot` paths whose waves carry `slots` of them at once, and its
+// queues (PathKernelArgs); per_cu: work-groups a CU holds; grid_wgs, ppl: the run's own choices, or 0.
+static int path_grid(int n_cu, int per_cu, int wg, int64_t slots, int64_t tot, int grid_wgs, int ppl, PathKernelArgs &pa) {
+    // one wave per SIMD as far as the paths fill it; more, up to what the card holds at once, while
+    // every lane has four paths one after another (lanes without a path cost as much as the others
+    // until the wave's last one ends)
+    const int64_t waves = wg / 64, per_wg = slots * waves, held = (int64_t)n_cu * std::max(1, per_cu);
+    const int64_t one = ((int64_t)n_cu * 4 + waves - 1) / waves;
+    const int64_t want = std::min(held, std::max(one, tot / (4 * per_wg)));
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(grid_wgs > 0 ? grid_wgs : want, (tot + per_wg - 1) / per_wg));
+    // the first paths of every wave are its own -- unless not all waves run at once, when these would
+    // wait for others to end -- and the rest goes out in chunks of a sixteenth of an even share
+    const int64_t share = tot / (grid * waves);
+    pa.n_queues = std::min(kMaxQueues, grid);
+    pa.queue_len = (tot + pa.n_queues - 1) / pa.n_queues;
+    pa.pool_first = grid <= held ? (int32_t)slots : 0;
+    pa.pool_chunk = ppl > 0 ? slots * ppl : std::max<int64_t>(std::min<int64_t>(slots, 16), std::min<int64_t>(256, share / 16));
+    return grid;
 }
 
 pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const double glob[4],
@@ -459,8 +466,9 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         pa.patches = dpatch;
         pa.n_patches = (int32_t)patches.size();
         const bool fp64 = r->precision == PDDS_FP64;
-        const int lanes = persistent && geom == GeomRect && pp.refl == 0 && pp.step == STEP_CV && group_pde(prob->pde, r->precision)
-                              ? group_lanes(e->n_cu, fp64, tot) : 0;
+        const int lanes = persistent && geom == GeomRect && pp.step == STEP_CV
+                              ? group_lanes(prob->pde, r->precision, pp.refl != 0, e->n_cu, tot) : 0;
+        const bool use_tiles = tiled && !lanes;
         auto launch = [&](const PathLaunch &l) -> hipError_t {
             if (lanes) return fp64 ? launch_group_f64(prob->pde, mixed, lanes, l, pa) : launch_group_f32(prob->pde, mixed, lanes, l, pa);
             return fp64 ? launch_path_f64(prob->pde, geom, persistent, mixed, l, pa)
@@ -472,30 +480,14 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         const int kwg = lanes ? 256 : wg;   // work-group of the path kernel (not the tiled one)
         int grid;
         pa.n_queues = 1;
-        if (tiled) {
+        if (use_tiles) {
             const int twg = path_tiled_wg(r->precision, r->step, geom);
             grid = r->grid_wgs > 0 ? r->grid_wgs
                                    : (int)std::max<int64_t>(1, std::min<int64_t>(e->n_cu, (tot + 8 * twg - 1) / (8 * twg)));
         } else if (persistent) {
-            // one wave per SIMD as far as the paths fill it; more, up to what the card holds at once,
-            // while every lane has four paths one after another (lanes without a path cost as much as
-            // the others until the wave's last one ends)
             int per_cu = 0;
             if ((st = launched(launch(PathLaunch{0, kwg, e->stream, &per_cu})))) return st;
-            const int64_t slots = lanes ? 64 / lanes : 64;      // paths a wave carries at once
-            const int64_t per_wg = slots * (kwg / 64), held = (int64_t)e->n_cu * std::max(1, per_cu);
-            const int64_t one = ((int64_t)e->n_cu * 4 + kwg / 64 - 1) / (kwg / 64);
-            const int64_t want = std::min(held, std::max(one, tot / (4 * per_wg)));
-            grid = (int)std::max<int64_t>(1, std::min<int64_t>(r->grid_wgs > 0 ? r->grid_wgs : want, (tot + per_wg - 1) / per_wg));
-            // the first paths of every wave are its own -- unless not all waves run at once, when
-            // these would wait for others to end -- and the rest goes out in chunks of a sixteenth
-            // of an even share
-            const int64_t share = tot / ((int64_t)grid * (kwg / 64));
-            pa.n_queues = std::min(kMaxQueues, grid);
-            pa.queue_len = (tot + pa.n_queues - 1) / pa.n_queues;
-            pa.pool_first = grid <= held ? (int32_t)slots : 0;
-            pa.pool_chunk = r->paths_per_lane > 0 ? slots * r->paths_per_lane
-                                                  : std::max<int64_t>(std::min<int64_t>(slots, 16), std::min<int64_t>(256, share / 16));
+            grid = path_grid(e->n_cu, per_cu, kwg, lanes ? 64 / lanes : 64, tot, r->grid_wgs, r->paths_per_lane, pa);
         } else {
             grid = (int)std::min<int64_t>((tot + wg - 1) / wg, (int64_t)1 << 30);
         }
@@ -506,7 +498,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             pa.base = base;
             const int g = persistent ? grid : (int)std::min<int64_t>(grid, (tot - base + wg - 1) / wg);
             hipError_t lr;
-            if (tiled)
+            if (use_tiles)
                 lr = r->precision == PDDS_FP64 ? launch_path_tiled_f64(geom, mixed, g, lds_bytes, e->stream, pa)
                                                : launch_path_tiled_f32(geom, mixed, g, lds_bytes, e->stream, pa);
             else
@@ -1529,12 +1521,53 @@ pdds_status pdds_paths(pdds_engine *e, const pdds_problem *p, const pdds_run *r,
         if ((st = dbuf(e, B_P11, (size_t)n * 8, &ps2))) return st;
         a.steps2 = (int64_t *)ps2;
     }
-    const int wg = r->wg_size > 0 ? r->wg_size : 256;
-    const int64_t grid = (n + wg - 1) / wg;
-    HIPCHK(hipEventRecord(e->ev[0], e->stream));
-    hipError_t lr = r->precision == PDDS_FP64 ? launch_paths_f64(p->pde, (int)grid, wg, e->stream, a)
-                                              : launch_paths_f32(p->pde, (int)grid, wg, e->stream, a);
-    if (lr != hipSuccess) return fail(e, PDDS_ERR_DEVICE, std::string("paths launch: ") + hipGetErrorString(lr));
+    const bool fp64 = r->precision == PDDS_FP64;
+    int wg = r->wg_size > 0 ? r->wg_size : 256;
+    int64_t grid = (n + wg - 1) / wg;
+    // the control-variate step as a group launch of one knot, whose lanes take up new paths where one
+    // per lane would wait for its wave's longest; not the FP32 forms that the group kernel lacks (a
+    // second phase starts at any step count, half a Philox call) nor counts past its 32-bit indices
+    const bool group = pp.step == STEP_CV && n < ((int64_t)1 << 32) && a.max_steps < ((int64_t)1 << 27) &&
+                       (fp64 || (!phase2 && !pp.refl && p->pde != PDDS_PDE_MONEGROS));
+    PathKernelArgs ga;
+    PathOut go;
+    std::vector<KnotDesc> gk;       // (uploaded asynchronously: they outlive the copies)
+    std::vector<int32_t> gblk;
+    if (group) {
+        KnotDesc kd;
+        std::memset(&kd, 0, sizeof(kd));
+        kd.x0 = x0; kd.y0 = y0; kd.knot_id = knot; kd.stream = r->stream; kd.n_paths = n;
+        // a path's number is its index less the knot's first path, modulo 2^32
+        kd.path_off = -path0;
+        kd.k2 = pp.k2; kd.h = r->h; kd.sqrth = a.sqrth; kd.gmask = 15;
+        for (int i = 0; i < 4; ++i) kd.dom[i] = rect[i];
+        KnotDesc *dk; int32_t *dkblk; unsigned long long *dctr;
+        gk.assign(1, kd);
+        gblk.assign(2, 0);
+        if ((st = upload(e, B_KNOTS, gk, &dk)) || (st = upload(e, B_KBLK, gblk, &dkblk))) return st;
+        void *pc;
+        if ((st = dbuf(e, B_COUNTER, kMaxQueues * kQueueStride * sizeof(unsigned long long), &pc))) return st;
+        dctr = (unsigned long long *)pc;
+        HIPCHK(launch_fill_u64(dctr, kMaxQueues * kQueueStride, 0ULL, e->stream));
+        std::memset(&ga, 0, sizeof(ga));
+        ga.knots = dk; ga.n_knots = 1; ga.kshift = 32; ga.kblk = dkblk; ga.total = n; ga.counter = dctr;
+        ga.h = r->h; ga.sqrth = a.sqrth; ga.beta = r->beta; ga.seed = r->seed; ga.stream = r->stream;
+        ga.max_steps = (uint32_t)a.max_steps; ga.pp = pp;
+        go = PathOut{{a.xt, a.xt2}, {a.yt, a.yt2}, {a.Y, a.Y2}, {a.Z, a.Z2}, {a.xi, a.xi2}, {a.steps, a.steps2}, a.phase2};
+        wg = 256;
+        auto launch = [&](const PathLaunch &l) {
+            return fp64 ? launch_group_records_f64(p->pde, l, ga, go) : launch_group_records_f32(p->pde, l, ga, go);
+        };
+        int per_cu = 0;
+        HIPCHK(launch(PathLaunch{0, wg, e->stream, &per_cu}));
+        grid = path_grid(e->n_cu, per_cu, wg, 64 / 4, n, 0, 0, ga);
+        HIPCHK(hipEventRecord(e->ev[0], e->stream));
+        HIPCHK(launch(PathLaunch{(int)grid, wg, e->stream, nullptr}));
+    } else {
+        HIPCHK(hipEventRecord(e->ev[0], e->stream));
+        hipError_t lr = fp64 ? launch_paths_f64(p->pde, (int)grid, wg, e->stream, a) : launch_paths_f32(p->pde, (int)grid, wg, e->stream, a);
+        if (lr != hipSuccess) return fail(e, PDDS_ERR_DEVICE, std::string("paths launch: ") + hipGetErrorString(lr));
+    }
     HIPCHK(hipEventRecord(e->ev[1], e->stream));
     for (int i = 0; i < 10; ++i)
         if (*dd[i]) HIPCHK(hipMemcpyAsync(hd[i], *dd[i], (size_t)n * 8, hipMemcpyDeviceToHost, e->stream));

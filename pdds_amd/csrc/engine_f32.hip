@@ -2,7 +2,6 @@
 // Kahan-compensated Z and xi, hardware transcendentals, one Philox draw per
 // two steps; exit records, moments and CSR partials stay in FP64.
 #include "engine_kernels.h"
-#include "engine_group.h"
 
 namespace pdds {
 
@@ -16,7 +15,7 @@ static hipError_t path_f32_gf(bool persistent, bool mixed, const PathLaunch &l, 
 template <int PDE, int GEOM>
 static hipError_t path_f32_g(bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
     if (a.pp.step != STEP_CV) return path_f32_gf<PDE, GEOM, STEP_ANY>(persistent, mixed, l, a);
-    if constexpr (GEOM == GeomRect && (const_motion<PDE>() && PDE != PDE_MONEGROS)) {
+    if constexpr (GEOM == GeomRect && group_only<PDE, float>()) {
         // (its persistent form is the group kernel)
         return persistent ? hipErrorInvalidValue : l.go(plain_kernel<float, PDE, GEOM, STEP_CV>, a);
     } else {
@@ -44,24 +43,6 @@ hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const
         case PDE_VARCOEF_LUT: return path_f32<PDE_VARCOEF_LUT>(geom, persistent, mixed, l, a);
         case PDE_HELMHOLTZ: return path_f32<PDE_HELMHOLTZ>(geom, persistent, mixed, l, a);
         case PDE_TABLE: return path_f32<PDE_TABLE>(geom, persistent, mixed, l, a);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <int PDE, int G> static hipError_t group_f32g(bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
-    return mixed ? l.go(group_kernel<float, PDE, true, G>, a) : l.go(group_kernel<float, PDE, false, G>, a);
-}
-
-template <int PDE>
-static hipError_t group_f32(bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a) {
-    return lanes == 16 ? group_f32g<PDE, 16>(mixed, l, a) : lanes == 4 ? group_f32g<PDE, 4>(mixed, l, a)
-                                                                     : group_f32g<PDE, 1>(mixed, l, a);
-}
-
-hipError_t launch_group_f32(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a) {
-    switch (pde) {
-        case PDE_SINSIN: return group_f32<PDE_SINSIN>(mixed, lanes, l, a);
-        case PDE_HELMHOLTZ: return group_f32<PDE_HELMHOLTZ>(mixed, lanes, l, a);
         default: return hipErrorInvalidValue;
     }
 }

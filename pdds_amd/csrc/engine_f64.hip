@@ -5,7 +5,6 @@
 // FP64 CPU restatement on the same Philox stream.
 #include "../../include/pdds_engine.h"
 #include "engine_kernels.h"
-#include "engine_group.h"
 
 namespace pdds {
 
@@ -21,7 +20,7 @@ static hipError_t path_f64_gf(bool persistent, bool mixed, const PathLaunch &l, 
 template <int PDE, int GEOM>
 static hipError_t path_f64_g(bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
     if (a.pp.step != STEP_CV) return path_f64_gf<PDE, GEOM, STEP_ANY>(persistent, mixed, l, a);
-    if constexpr (GEOM == GeomRect && (const_motion<PDE>())) {
+    if constexpr (GEOM == GeomRect && group_only<PDE, double>()) {
         // (its persistent form is the group kernel)
         return persistent ? hipErrorInvalidValue : l.go(plain_kernel<double, PDE, GEOM, STEP_CV>, a);
     } else {
@@ -49,29 +48,6 @@ hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const
         case PDE_VARCOEF_LUT: return path_f64<PDE_VARCOEF_LUT>(geom, persistent, mixed, l, a);
         case PDE_HELMHOLTZ: return path_f64<PDE_HELMHOLTZ>(geom, persistent, mixed, l, a);
         case PDE_TABLE: return path_f64<PDE_TABLE>(geom, persistent, mixed, l, a);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-bool group_pde(int pde, int precision) {
-    return pde == PDE_SINSIN || pde == PDE_HELMHOLTZ || (pde == PDE_MONEGROS && precision == PDDS_FP64);
-}
-
-template <int PDE, int G> static hipError_t group_f64g(bool mixed, const PathLaunch &l, const PathKernelArgs &a) {
-    return mixed ? l.go(group_kernel<double, PDE, true, G>, a) : l.go(group_kernel<double, PDE, false, G>, a);
-}
-
-template <int PDE>
-static hipError_t group_f64(bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a) {
-    return lanes == 16 ? group_f64g<PDE, 16>(mixed, l, a) : lanes == 4 ? group_f64g<PDE, 4>(mixed, l, a)
-                                                                     : group_f64g<PDE, 1>(mixed, l, a);
-}
-
-hipError_t launch_group_f64(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a) {
-    switch (pde) {
-        case PDE_MONEGROS: return group_f64<PDE_MONEGROS>(mixed, lanes, l, a);
-        case PDE_SINSIN: return group_f64<PDE_SINSIN>(mixed, lanes, l, a);
-        case PDE_HELMHOLTZ: return group_f64<PDE_HELMHOLTZ>(mixed, lanes, l, a);
         default: return hipErrorInvalidValue;
     }
 }

@@ -1,0 +1,71 @@
+// engine_group_f64.hip -- the group path kernel's FP64 instantiations and launchers.
+#include "../../include/pdds_engine.h"
+#include "engine_group.h"
+
+namespace pdds {
+
+// Lanes that carry one path of a launch of the group kernel.  One lane is the cheapest per step (the
+// step-ordered sums are repeated by every lane of a group), 16 finish a path soonest.  With one lane
+// a card holds 1024 to 2048 paths per CU; it pays once every lane has several paths one after
+// another, and below that a launch lasts as long as its longest path.  Measured on 256 CUs:
+// FP32 Helmholtz server burst (15.5 M paths) 83 ms with one lane, 119 with four; FP32 Poisson
+// assembly (0.6 M) 3.4 and 3.5; FP64 Helmholtz assembly (1.9 M) 2.5 and 3.1, FP64 recorded run
+// (0.77 M) 4.0 and 3.6; with four and sixteen lanes: 140 k FP32 paths 1.25 and 1.16 ms, 5000 FP64
+// paths 0.73 and 0.58, 4000 0.34 and 0.29.
+int group_lanes(int pde, int precision, bool refl, int n_cu, int64_t paths) {
+    const bool fp64 = precision == PDDS_FP64;
+    const bool moves = pde == PDE_SINSIN || pde == PDE_HELMHOLTZ || pde == PDE_MONEGROS;   // const_motion
+    if (!fp64 && (refl || pde == PDE_MONEGROS)) return 0;
+    if ((!moves || refl) && paths > (int64_t)n_cu * 2048) return 0;
+    if (!moves) return 4;
+    if (refl) return paths > (int64_t)n_cu * 32 ? 4 : 16;
+    if (paths >= (int64_t)n_cu * (fp64 ? 4096 : 2048)) return 1;
+    return paths > (int64_t)n_cu * 32 ? 4 : 16;
+}
+
+template <int PDE> static hipError_t group_f64(bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a) {
+    if constexpr (const_motion<PDE>()) {
+        if (a.pp.refl)
+            return lanes == 16 ? l.go(group_kernel<double, PDE, false, 16, true>, a, NoOut{})
+                               : l.go(group_kernel<double, PDE, false, 4, true>, a, NoOut{});
+        if (lanes == 16)
+            return mixed ? l.go(group_kernel<double, PDE, true, 16>, a, NoOut{}) : l.go(group_kernel<double, PDE, false, 16>, a, NoOut{});
+        if (lanes == 1)
+            return mixed ? l.go(group_kernel<double, PDE, true, 1>, a, NoOut{}) : l.go(group_kernel<double, PDE, false, 1>, a, NoOut{});
+    } else if (a.pp.refl) {
+        return l.go(group_kernel<double, PDE, false, 4, true>, a, NoOut{});
+    }
+    return mixed ? l.go(group_kernel<double, PDE, true, 4>, a, NoOut{}) : l.go(group_kernel<double, PDE, false, 4>, a, NoOut{});
+}
+
+hipError_t launch_group_f64(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a) {
+    if (mixed && a.pp.refl) return hipErrorInvalidValue;
+    switch (pde) {
+        case PDE_MONEGROS: return group_f64<PDE_MONEGROS>(mixed, lanes, l, a);
+        case PDE_SINSIN: return group_f64<PDE_SINSIN>(mixed, lanes, l, a);
+        case PDE_VARCOEF: return group_f64<PDE_VARCOEF>(mixed, lanes, l, a);
+        case PDE_VARCOEF_LUT: return group_f64<PDE_VARCOEF_LUT>(mixed, lanes, l, a);
+        case PDE_HELMHOLTZ: return group_f64<PDE_HELMHOLTZ>(mixed, lanes, l, a);
+        case PDE_TABLE: return group_f64<PDE_TABLE>(mixed, lanes, l, a);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <int PDE> static hipError_t group_records_f64(const PathLaunch &l, const PathKernelArgs &a, const PathOut &o) {
+    return a.pp.refl ? l.go(group_kernel<double, PDE, false, 4, true, PathOut>, a, o)
+                     : l.go(group_kernel<double, PDE, false, 4, false, PathOut>, a, o);
+}
+
+hipError_t launch_group_records_f64(int pde, const PathLaunch &l, const PathKernelArgs &a, const PathOut &o) {
+    switch (pde) {
+        case PDE_MONEGROS: return group_records_f64<PDE_MONEGROS>(l, a, o);
+        case PDE_SINSIN: return group_records_f64<PDE_SINSIN>(l, a, o);
+        case PDE_VARCOEF: return group_records_f64<PDE_VARCOEF>(l, a, o);
+        case PDE_VARCOEF_LUT: return group_records_f64<PDE_VARCOEF_LUT>(l, a, o);
+        case PDE_HELMHOLTZ: return group_records_f64<PDE_HELMHOLTZ>(l, a, o);
+        case PDE_TABLE: return group_records_f64<PDE_TABLE>(l, a, o);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace pdds

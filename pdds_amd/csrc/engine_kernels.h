@@ -164,6 +164,15 @@ template <class R, int PDE, int FAM, bool REFL> constexpr bool zero_terms() {
     return sizeof(R) == 4 && (FAM != STEP_CV || REFL || PDE == PDE_MONEGROS);
 }
 
+// Problems whose paths move by a constant multiple of the increments (sigma constant and diagonal,
+// no drift): the serial part of a step is one addition per coordinate.
+template <int PDE> constexpr bool const_motion() { return PDE == PDE_SINSIN || PDE == PDE_HELMHOLTZ || PDE == PDE_MONEGROS; }
+// ... whose persistent control-variate launches on rectangles are all the group kernel's
+// (engine_group.h), which has no form with zero terms
+template <int PDE, class R> constexpr bool group_only() {
+    return const_motion<PDE>() && !zero_terms<R, PDE, STEP_CV, false>();
+}
+
 template <class R, int PDE, int FAM, bool LT = false>
 __device__ __forceinline__ void em_step(PathState<R> &s, const Coef<R> &co, R h, R sqrth, R n1, R n2, int fam,
                                         R lz = (R)0, R ly = (R)0) {

@@ -206,15 +206,21 @@ struct PathsArgs {
     int64_t *steps2;
 };
 
+// Where pdds_paths has a path's exit values written (null: not asked for), per phase.
+struct PathOut {
+    double *xt[2], *yt[2], *Y[2], *Z[2], *xi[2];
+    int64_t *steps[2];
+    int32_t phase2;
+};
 // A path launch: with per_cu set nothing is launched, and the work-groups of the kernel that a CU
 // holds at once are put there (a persistent grid is sized by them).
 struct PathLaunch {
     int grid, wg;
     hipStream_t stream;
     int *per_cu;
-    template <class K> hipError_t go(K kernel, const PathKernelArgs &a) const {
+    template <class K, class... A> hipError_t go(K kernel, const A &...args) const {
         if (per_cu) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, kernel, wg, 0);
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), 0, stream, a);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), 0, stream, args...);
         return hipGetLastError();
     }
 };
@@ -225,10 +231,14 @@ hipError_t launch_path_tiled_f32(int geom, bool mixed, int grid, size_t lds, hip
 int path_tiled_wg(int precision, int step, int geom);   // block size of the LDS-tiled kernel
 hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
-// const-motion problems on rectangles, control-variate step: `lanes` (1, 4 or 16) lanes per path
-bool group_pde(int pde, int precision);
+// Group kernel (rectangles, control-variate step): lanes that carry one path of a launch of that many
+// paths, 1, 4 or 16; 0 where the launch is the other path kernels'
+int group_lanes(int pde, int precision, bool refl, int n_cu, int64_t paths);
 hipError_t launch_group_f64(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_group_f32(int pde, bool mixed, int lanes, const PathLaunch &l, const PathKernelArgs &a);
+// ... with each path's exit values written out (4 lanes to a path)
+hipError_t launch_group_records_f64(int pde, const PathLaunch &l, const PathKernelArgs &a, const PathOut &o);
+hipError_t launch_group_records_f32(int pde, const PathLaunch &l, const PathKernelArgs &a, const PathOut &o);
 hipError_t launch_reduce(int grid, int wg, size_t shmem, hipStream_t s, const ReduceArgs &a);
 hipError_t launch_paths_f64(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);
 hipError_t launch_paths_f32(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);

@@ -60,6 +60,13 @@ PDDS_HD void monegros(R x, R y, R &u, R &gx, R &gy, R &lap) {
 
 template <int PDE, class R> PDDS_HD R pde_g(R x, R y, const PdeParams &P);
 
+// a b + c; FP32 with the product fused (written out, so that it does not depend on which other
+// coefficients a kernel forms beside it)
+template <class R> PDDS_HD R fused(R a, R b, R c) {
+    if constexpr (sizeof(R) == 4) return __builtin_fmaf(a, b, c);
+    else return c + a * b;
+}
+
 // TILED: the coefficient LUT's fields 0..3 are read from the LDS tile T where it covers X.
 // k2: the Helmholtz parameter of this path's problem (per knot, so one launch can carry
 // requests with different k^2).  live: whether the caller uses this lane's values.
@@ -112,8 +119,8 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
         co.g0 = uu; co.g1 = uy;
         if constexpr (PDE == PDE_VARCOEF) {
             co.s00 = s1; co.s11 = s2;
-            co.b0 = (R)0.2 * y + (R)0.3 * s1 * cxn;
-            co.b1 = (R)-0.2 * x - (R)0.3 * s2 * syn;
+            co.b0 = fused<R>((R)0.3 * s1, cxn, (R)0.2 * y);
+            co.b1 = fused<R>(-((R)0.3 * s2), syn, (R)-0.2 * x);
             co.c = -((R)1.0 + x * x);
         } else {
             R v[5];

@@ -71,6 +71,51 @@ def test_group_widths_equal_each_other(eng, precision):
         assert np.array_equal(u, out[0][0]) and np.array_equal(v, out[0][1])
 
 
+@pytest.mark.parametrize("case", ["varcoef", "varcoef_lut", "table", "helmholtz-robin", "varcoef-robin"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_group_equals_one_lane_kernels(eng, case, precision):
+    """Problems whose coefficients move the path, and reflecting sides: the same points in a launch
+    small enough for the group kernel and in one that the other path kernels take."""
+    from pdds_amd.engine import bvp, default_run
+    from pdds_amd.workloads import table_problem, varcoef_lut
+    if case.endswith("robin") and precision == "fp32":
+        pytest.skip("FP32 reflecting launches have no group form")
+    pb = {"varcoef": lambda: bvp("varcoef"), "varcoef_lut": lambda: bvp("varcoef_lut", lut=varcoef_lut(eng, 64)),
+          "table": lambda: table_problem(eng, 64), "helmholtz-robin": lambda: bvp("helmholtz", k2=2.0, neumann=10, varphi=-1.0),
+          "varcoef-robin": lambda: bvp("varcoef", neumann=1, varphi=-0.5, rho=0.2)}[case]()
+    cu = eng.info()["n_cu"]
+    x, y, n = np.array([0.1, -0.6, 0.4]), np.array([-0.3, 0.2, 0.9]), np.array([3000, 41, 700])
+    out = []
+    for extra in (0, cu * 2048 - int(n.sum()), cu * 2048):
+        print(case, precision, extra, flush=True)
+        m = 3 + (extra > 0)
+        r = eng.point_eval(pb, default_run(h=0.01, seed=9, precision=precision), GLOB, np.append(x, 0.5)[:m],
+                           np.append(y, 0.5)[:m], np.append(n, extra)[:m])
+        out.append((r["u"][:3], r["u_var"][:3]))
+    for u, v in out[1:]:
+        assert np.array_equal(u, out[0][0]) and np.array_equal(v, out[0][1])
+
+
+@pytest.mark.parametrize("n,path0,cap", [(1, 0, 0), (63, 5, 0), (1000, (1 << 32) - 1000, 0), (700, 0, 7)])
+@pytest.mark.parametrize("refl", [0, 8])
+def test_group_records_equal_oracle(eng, n, path0, cap, refl):
+    """pdds_paths: partly filled waves, the last path numbers, a cap within the first and the second
+    phase's steps; both phases equal the oracle's records."""
+    from oracle import oracle as O
+    from pdds_amd.engine import bvp, default_run
+    rect = np.array([-0.6, -0.9, 0.4, 0.2])
+    print(n, path0, cap, refl, flush=True)
+    got = eng.paths(bvp("helmholtz", k2=2.0, neumann=refl), default_run(h=4e-3, seed=7, max_steps=cap), 0.1, -0.2, rect, 5,
+                    path0, n, phase2=True)
+    run = O.run_params(4e-3, 7, phase2=1, threads=8)
+    if cap:
+        run.max_steps = cap
+    ref = O.simulate(O.problem(O.PDE_HELMHOLTZ, k2=2.0, refl=refl), run, 0.1, -0.2, rect, 5, path0, n, phase2_out=True)
+    for k in ("steps", "xt", "yt", "Y", "Z", "xi"):
+        assert np.array_equal(got[k], ref[k]), k
+        assert np.array_equal(got["phase2"][k], ref["phase2"][k]), ("phase2", k)
+
+
 @pytest.mark.parametrize("cap", [1, 2, 15, 16, 17, 33])
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_group_step_cap_equals_plain(eng, precision, cap):
