@@ -361,6 +361,8 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         std::vector<ItemDesc> items;
         int64_t part = 0, off = 0;
         int ne_cap = 1, nnz_cap = 1;
+        struct { int ne = 1, nnz = 1; int64_t wgs = 0; } cls[REDUCE_CLASSES];   // the reduction's launches
+        std::vector<uint8_t> kcls(nk);
         for (int q = 0; q < nk; ++q) {
             const AsmKnot &k = knots[ord[k0 + q]];
             const StencilDesc &sd = host_sd(k);
@@ -368,6 +370,11 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             Pmax_all = std::max(Pmax_all, P);
             ne_cap = std::max(ne_cap, sd.msz[0] + sd.msz[1] + sd.msz[2] + sd.msz[3]);
             nnz_cap = std::max(nnz_cap, sd.csr_nnz);
+            int ne = 0, tiles = 0;
+            for (int i = 0; i < 4; ++i) { ne += sd.msz[i]; tiles += (sd.msz[i] + 15) / 16; }
+            kcls[q] = !reduce16_fits(ne, tiles, S) ? REDUCE_ANY : tiles <= kSmallTiles ? REDUCE16_SMALL : REDUCE16_LARGE;
+            auto &cl = cls[kcls[q]];
+            cl.ne = std::max(cl.ne, ne); cl.nnz = std::max(cl.nnz, sd.csr_nnz);
             kd[q].x0 = k.x0; kd[q].y0 = k.y0; kd[q].knot_id = k.id; kd[q].stencil = k.stencil;
             kd[q].table = k.table; kd[q].stream = k.has_stream ? k.stream : r->stream;
             kd[q].n_paths = k.n; kd[q].path_off = off; kd[q].out_off = k.out_off;
@@ -384,6 +391,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
                 it.n = (int32_t)std::min<int64_t>(P, k.n - p0);
                 it.p_begin = p0;
                 it.part_off = part;
+                it.span_first = it.span_count = 0;
                 part += 2 * (int64_t)sd.csr_nnz;
                 items.push_back(it);
             }
@@ -400,6 +408,23 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         const size_t shmem = reduce_lds_bytes(ne_cap, nnz_cap, S);
         if (shmem > 160 * 1024 || S > 65535)
             return fail(e, PDDS_ERR_UNSUPPORTED, "stencil or sub-batch too large for the LDS reduction buffers");
+        // spans of items of one knot for the reduction by 16 sub-batches: as many items as fill a
+        // group, while every CU still has three work-groups
+        const int64_t most = std::min<int64_t>(kSpanItems, std::max<int64_t>(1, (int64_t)items.size() / (3 * (int64_t)e->n_cu)));
+        size_t n_spans = 0;
+        for (int c = 0; c < REDUCE_CLASSES; ++c) {
+            const size_t first = n_spans;
+            for (int q = 0; q < nk; ++q) {
+                if (kcls[q] != c) continue;
+                const int64_t i0 = kd[q].item_begin, ni = kd[q].item_count;
+                const int64_t per = c == REDUCE_ANY || ni == 0 ? 1 : std::max<int64_t>(1, std::min<int64_t>(most, kGroup16 / std::max(1, items[i0].n / S)));
+                for (int64_t i = 0; i < ni; i += per) {
+                    items[n_spans].span_first = (int32_t)(i0 + i);
+                    items[n_spans++].span_count = (int32_t)std::min(per, ni - i);
+                }
+            }
+            cls[c].wgs = (int64_t)(n_spans - first);
+        }
         // blocks of 2^kshift paths, about two per knot, each with its first path's knot (find_knot)
         int kshift = 6;
         while ((tot >> kshift) > std::max<int64_t>(64, 2 * (int64_t)nk)) ++kshift;
@@ -510,19 +535,24 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         ReduceArgs ra;
         std::memset(&ra, 0, sizeof(ra));
         ra.knots = dk; ra.tables = dtab; ra.items = dit; ra.rec = rec;
-        ra.stats = dstats; ra.partials = dpart; ra.ne_cap = ne_cap; ra.nnz_cap = nnz_cap; ra.S = S;
+        ra.stats = dstats; ra.partials = dpart; ra.S = S;
         ra.wref = dW;
         ra.side_rbf = geom == GeomRect ? 1 : 0;   // rectangle sides: the chunked recurrence
         // exit sides: FP32 records carry them; FP64 exits are classified as write_exit does, on
         // the global rectangle's centre and half-sides (rect_dist's) or the disc's radius
         ra.side_mode = r->precision != PDDS_FP64 ? SIDE_BITS : geom == GeomDisc ? SIDE_DISC : SIDE_RECT;
         for (int i = 0; i < 4; ++i) ra.gc[i] = gc[i];
-        const int64_t nit = (int64_t)items.size();
-        for (int64_t base = 0; base < nit; base += (int64_t)1 << 30) {
-            ra.item_base = base;
-            hipError_t lr = launch_reduce((int)std::min<int64_t>(nit - base, (int64_t)1 << 30),
-                                          kReduceWG, shmem, e->stream, ra);
-            if (lr != hipSuccess) return fail(e, PDDS_ERR_DEVICE, std::string("reduce launch: ") + hipGetErrorString(lr));
+        for (int c = 0; c < REDUCE_CLASSES; ++c) {
+            ra.ne_cap = cls[c].ne;
+            ra.nnz_cap = cls[c].nnz;
+            for (int64_t base = 0; base < cls[c].wgs; base += (int64_t)1 << 30) {
+                const int ng = (int)std::min<int64_t>(cls[c].wgs - base, (int64_t)1 << 30);
+                hipError_t lr = c == REDUCE_ANY
+                                    ? launch_reduce(ng, kReduceWG, reduce_lds_bytes(ra.ne_cap, ra.nnz_cap, S), e->stream, ra)
+                                    : launch_reduce16(c == REDUCE16_SMALL, ng, reduce16_lds_bytes(ra.ne_cap, S), e->stream, ra);
+                if (lr != hipSuccess) return fail(e, PDDS_ERR_DEVICE, std::string("reduce launch: ") + hipGetErrorString(lr));
+                ra.item_base += ng;
+            }
         }
         FinalizeArgs f;
         f.knots = dk; f.tables = dtab; f.items = dit; f.stats = dstats; f.partials = dpart;
@@ -1403,7 +1433,7 @@ static pdds_status point_eval_locked(pdds_engine *e, const pdds_problem *p, cons
         // alignment
         const int64_t need = paths * (int64_t)sizeof(ExitRec) +
                              (int64_t)knots.size() * (int64_t)(kKnotDescQuota + sizeof(KnotStat) + 16 +
-                                                                17 * (sizeof(ItemDesc) + sizeof(ItemStat))) +
+                                                                17 * (kItemDescQuota + sizeof(ItemStat))) +
                              ((int64_t)1 << 16);
         if (need > (int64_t)PDDS_NOALLOC_SCRATCH_BYTES)
             return fail(e, PDDS_ERR_FULL, std::to_string(paths) + " paths at " + std::to_string(knots.size()) +

@@ -104,6 +104,17 @@ PDDS_HD double rbf_tab(double px, double py, double x, double y, double inv_c2, 
     return dexp_tab_nonpos(-(dx * dx + dy * dy) * inv_c2, T);
 }
 
+// Four of them, their chains side by side
+PDDS_HD void rbf_tab4(double px, double py, const double x[4], const double y[4], double inv_c2, const double *T, double v[4]) {
+    double e[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const double dx = px - x[u], dy = py - y[u];
+        e[u] = -(dx * dx + dy * dy) * inv_c2;
+    }
+    dexp_tab_nonpos4(e, T, v);
+}
+
 // The same Gaussian at exit (x, y) for the kRbfChunk entries from j0 of a straight, uniformly
 // spaced stencil side (px, py; a rectangle side) with step (sx, sy), ss = |s|^2 and
 // q = exp(-2 ss / c^2): entry j0 directly, the others by the two-multiply recurrence
@@ -116,7 +127,7 @@ PDDS_HD void rbf_side_chunk(const double *px, const double *py, int j0, double s
                             double x, double y, double inv_c2, const double *T, double Y, double acc[kRbfChunk]) {
     const double dx = px[j0] - x, dy = py[j0] - y;
     double p = dexp_tab_nonpos(-(dx * dx + dy * dy) * inv_c2, T);
-    double r = dexp_fast(__builtin_fmin(-(2.0 * (dx * sx + dy * sy) + ss) * inv_c2, 700.0));
+    double r = dexp_le700(__builtin_fmin(-(2.0 * (dx * sx + dy * sy) + ss) * inv_c2, 700.0));
     acc[0] = __builtin_fma(Y, p, acc[0]);
 #pragma unroll
     for (int k = 1; k < kRbfChunk; ++k) {

@@ -18,6 +18,25 @@ inline size_t reduce_lds_bytes(int ne_cap, int nnz_cap, int S) {
     b += g * 4 * sizeof(uint16_t);
     return (b + 15) & ~(size_t)15;
 }
+
+// The reduction of groups of 16 sub-batches (reduce16_kernel): its LDS holds Phi [ne_cap][16], the
+// group's x, y, Y [16 S] and score [16 (S + 1)] (FP64) and the path lists (bytes: [16][S], or
+// [16][4][S] where S does not divide 64).  It takes stencils of at most kMaxTiles tiles of 16 side
+// entries, and sub-batches whose group leaves room for two work-groups on a CU; stencils of up to
+// kSmallTiles leave room for three.
+constexpr int kGroup16 = 16;
+constexpr int kSmallTiles = 16, kMaxTiles = 32;
+constexpr int kSpanItems = 16;            // work items of one knot a work-group may take
+inline size_t reduce16_lds_bytes(int ne_cap, int S) {
+    const size_t g = (size_t)kGroup16 * S;
+    const size_t b = ((size_t)kGroup16 * ne_cap + 4 * g + kGroup16) * sizeof(double) + (S <= 64 && 64 % S == 0 ? g : 4 * g);
+    return (b + 15) & ~(size_t)15;
+}
+inline bool reduce16_fits(int ne, int tiles, int S) {
+    return S <= 256 && reduce16_lds_bytes(ne, S) <= 76 * 1024 && tiles <= kMaxTiles;
+}
+// The reduction of a stencil: by reduce16_kernel, of up to kSmallTiles tiles or more, or by reduce_kernel
+enum ReduceClass { REDUCE16_SMALL = 0, REDUCE16_LARGE = 1, REDUCE_ANY = 2, REDUCE_CLASSES = 3 };
 // FP32 exit records carry the exit side + 1 (0 = none, 1..5 = sides -1..4) in the low bits of
 // Y: a float widened to double leaves the low 29 bits of its mantissa zero.
 constexpr uint64_t kSideBitsMask = 7ULL;
@@ -78,6 +97,10 @@ struct ItemDesc {
     int32_t n;              // paths in the item
     int64_t p_begin;        // first path index within the knot
     int64_t part_off;       // 2*nnz partials (sum, sum of squares / n_beta)
+    // the reduction's w-th work-group (of its launches' one after another) takes items span_first ..
+    // + span_count of one knot, as entry w of the item table says: these two are not about the
+    // entry's own item
+    int32_t span_first, span_count;
 };
 
 struct ItemStat {
@@ -98,6 +121,7 @@ struct KnotStat {
 // admission, pdds_point_eval_noalloc).  What a descriptor has beyond them and the block table of the
 // knots are launch-side copies of a few dozen bytes a knot and stay out of these limits.
 constexpr int64_t kKnotDescQuota = 96;
+constexpr int64_t kItemDescQuota = 24;     // of a work item's, in the same estimates
 
 // Per-path exit records, indexed by global path index: the FP64 exit values as one aligned
 // 32-byte record (a lane stores it with two 16-byte writes when its path stops, so a record
@@ -240,6 +264,7 @@ hipError_t launch_group_f32(int pde, bool mixed, int lanes, const PathLaunch &l,
 hipError_t launch_group_records_f64(int pde, const PathLaunch &l, const PathKernelArgs &a, const PathOut &o);
 hipError_t launch_group_records_f32(int pde, const PathLaunch &l, const PathKernelArgs &a, const PathOut &o);
 hipError_t launch_reduce(int grid, int wg, size_t shmem, hipStream_t s, const ReduceArgs &a);
+hipError_t launch_reduce16(bool small, int grid, size_t shmem, hipStream_t s, const ReduceArgs &a);
 hipError_t launch_paths_f64(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);
 hipError_t launch_paths_f32(int pde, int grid, int wg, hipStream_t s, const PathsArgs &a);
 hipError_t launch_finalize(int grid, int wg, hipStream_t s, const FinalizeArgs &f);

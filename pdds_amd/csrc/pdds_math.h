@@ -155,6 +155,20 @@ PDDS_HD double dexp_fast(double x) {
     return dexp(x);
 }
 
+// dexp(x) for x <= 700, bit for bit, without branches (the factors of the RBF recurrence): ldexp
+// rounds a subnormal result once, as dexp's two scalings do
+PDDS_HD double dexp_le700(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double k = __builtin_floor(x * kLog2e + 0.5);
+    double r = __builtin_fma(-k, kLn2Hi, x);
+    r = __builtin_fma(-k, kLn2Lo, r);
+    const double v = __builtin_ldexp(exp_poly_k(r), (int)k);
+    return x < -745.2 ? 0.0 : v;
+#else
+    return dexp(x);
+#endif
+}
+
 // dexp(x) for x <= 0, bit for bit, without branches: the value of dexp's own steps, with the
 // underflow (x < -745.2 -> 0) and subnormal scalings as selects.  The RBF moments of the
 // reduction evaluate one of these per (exit, stencil entry).
@@ -216,6 +230,28 @@ PDDS_HD double dexp_tab_nonpos(double x, const double *T) {
     const double v = __builtin_fma(t, p, t);
     const double y = v * pow2i(ki >> 6);         // ki >> 6 >= -1022
     return x < -708.0 ? 0.0 : y;
+}
+
+// Four of them, step by step: each is a chain of some 25 dependent operations, which one wave alone
+// would wait for
+PDDS_HD void dexp_tab_nonpos4(const double x[4], const double *T, double v[4]) {
+    double xc[4], k[4], r[4], p[4], t[4];
+    int ki[4];
+#define PDDS_X4 _Pragma("unroll") for (int u = 0; u < 4; ++u)
+    PDDS_X4 xc[u] = __builtin_fmax(x[u], -708.0);
+    PDDS_X4 k[u] = __builtin_rint(xc[u] * kInvLn2x64);
+    PDDS_X4 ki[u] = (int)k[u];
+    PDDS_X4 t[u] = T[ki[u] & 63];
+    PDDS_X4 r[u] = __builtin_fma(-k[u], kLn2d64Hi, xc[u]);
+    PDDS_X4 r[u] = __builtin_fma(-k[u], kLn2d64Lo, r[u]);
+    PDDS_X4 p[u] = fma_k(r[u], 0.008333333333333333, 0.041666666666666664);
+    PDDS_X4 p[u] = fma_k(p[u], r[u], 0.16666666666666666);
+    PDDS_X4 p[u] = fma_k(p[u], r[u], 0.5);
+    PDDS_X4 p[u] = fma_k(p[u], r[u], 1.0);
+    PDDS_X4 p[u] = p[u] * r[u];
+    PDDS_X4 p[u] = __builtin_fma(t[u], p[u], t[u]);
+    PDDS_X4 v[u] = x[u] < -708.0 ? 0.0 : p[u] * pow2i(ki[u] >> 6);
+#undef PDDS_X4
 }
 
 PDDS_HD double dexpm1(double x) {

@@ -37,7 +37,7 @@ constexpr int64_t kRecordBytes = (int64_t)sizeof(ExitRec);
 // and statistics, and (counted per item, an over-estimate) the knot's descriptor, statistics and
 // step counters
 constexpr int64_t kKnotBytes = kKnotDescQuota + (int64_t)(sizeof(KnotStat) + 2 * sizeof(unsigned long long) +
-                                         sizeof(ItemDesc) + sizeof(ItemStat));
+                                         kItemDescQuota + sizeof(ItemStat));
 
 struct SrvReq {
     uint64_t ticket = 0;
