@@ -297,8 +297,20 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
     // LDS-tiled form (coefficient LUT with a fifth-field quad plane, persistent launch): knots
     // are grouped into patches of equal tile, tiles that fit in LDS first, in first-seen order;
     // not with reflecting sides, whose steps run in the persistent and plain kernels
+    int64_t all_paths = 0;
+    for (const AsmKnot &k : knots) all_paths += k.n;
+    const bool table = prob->pde == PDDS_PDE_TABLE;
+    // the tabulated problem's tile holds its fields' two planes, and with a VR + CV step that of mu
+    // and F where its grid is the same and there is room; launches that fill the tiled grid, in
+    // rectangles (not the FP32 VR + CV step, whose FP32 rounding follows the persistent kernel's code)
+    const LutView &la = pp.lut, &lv = pp.vlut;
+    const int tile_planes = !table ? 1 : pp.step == STEP_VRCV && la.nx == lv.nx && la.ny == lv.ny && la.px == lv.px &&
+                                                 la.ox == lv.ox && la.oy == lv.oy && la.sx == lv.sx && la.sy == lv.sy ? 3 : 2;
     const bool tiled =
-        persistent && prob->pde == PDDS_PDE_VARCOEF_LUT && r->lut_lds != 0 && pp.lut.nf == 5 && pp.refl == 0;
+        persistent && r->lut_lds != 0 && pp.refl == 0 &&
+        ((prob->pde == PDDS_PDE_VARCOEF_LUT && pp.lut.nf == 5) ||
+         (table && geom == GeomRect && (r->precision == PDDS_FP64 || pp.step != STEP_VRCV) &&
+          all_paths >= kTableTileLane * e->n_cu * (int64_t)path_tiled_wg(prob->pde, r->precision, r->step, geom)));
     const size_t tile_cap = e->lds_max > 1024 ? e->lds_max - 1024 : 0;
     std::vector<size_t> ord(knots.size());
     for (size_t i = 0; i < ord.size(); ++i) ord[i] = i;
@@ -309,7 +321,8 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         for (size_t i = 0; i < knots.size(); ++i) {
             int c0, r0, tw, th;
             lut_tile_of(pp.lut, host_sd(knots[i]).bbox, c0, r0, tw, th);
-            const int fits = (size_t)(tw + r->lut_pad) * th * sizeof(float4) <= tile_cap ? 1 : 0;
+            const size_t plane = (size_t)(tw + r->lut_pad) * th * sizeof(float4);
+            const int fits = plane * tile_planes <= tile_cap ? tile_planes : tile_planes == 3 && plane * 2 <= tile_cap ? 2 : 0;
             tkey[i] = {c0, r0, tw, th, fits};
             const std::array<int, 4> k4 = fits ? std::array<int, 4>{c0, r0, tw, th} : std::array<int, 4>{-1, -1, -1, -1};
             auto it = first.find(k4);
@@ -317,7 +330,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             rank[i] = it->second;
         }
         std::stable_sort(ord.begin(), ord.end(), [&](size_t a, size_t b) { return rank[a] < rank[b]; });
-        out.wg = path_tiled_wg(r->precision, r->step, geom);
+        out.wg = path_tiled_wg(prob->pde, r->precision, r->step, geom);
     }
     // knots are processed in batches whose exit records fit the record budget
     const int64_t rec_bytes = (int64_t)sizeof(ExitRec);
@@ -465,7 +478,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
                     if (tk[4]) {
                         pd.c0 = tk[0]; pd.r0 = tk[1]; pd.tw = tk[2]; pd.th = tk[3];
                         pd.pitch = tk[2] + r->lut_pad;
-                        lds_bytes = std::max(lds_bytes, (size_t)pd.pitch * tk[3] * sizeof(float4));
+                        lds_bytes = std::max(lds_bytes, (size_t)pd.pitch * tk[3] * pd.tiled * sizeof(float4));
                     }
                     patches.push_back(pd);
                 }
@@ -506,7 +519,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         int grid;
         pa.n_queues = 1;
         if (use_tiles) {
-            const int twg = path_tiled_wg(r->precision, r->step, geom);
+            const int twg = path_tiled_wg(prob->pde, r->precision, r->step, geom);
             grid = r->grid_wgs > 0 ? r->grid_wgs
                                    : (int)std::max<int64_t>(1, std::min<int64_t>(e->n_cu, (tot + 8 * twg - 1) / (8 * twg)));
         } else if (persistent) {
@@ -524,8 +537,8 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             const int g = persistent ? grid : (int)std::min<int64_t>(grid, (tot - base + wg - 1) / wg);
             hipError_t lr;
             if (use_tiles)
-                lr = r->precision == PDDS_FP64 ? launch_path_tiled_f64(geom, mixed, g, lds_bytes, e->stream, pa)
-                                               : launch_path_tiled_f32(geom, mixed, g, lds_bytes, e->stream, pa);
+                lr = r->precision == PDDS_FP64 ? launch_path_tiled_f64(prob->pde, geom, mixed, g, lds_bytes, e->stream, pa)
+                                               : launch_path_tiled_f32(prob->pde, geom, mixed, g, lds_bytes, e->stream, pa);
             else
                 lr = launch(PathLaunch{g, kwg, e->stream, nullptr});
             if ((st = launched(lr))) return st;

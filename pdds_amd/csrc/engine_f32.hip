@@ -47,27 +47,31 @@ hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const
     }
 }
 
-template <bool MIXED, int GEOM, int FAM>
+template <int PDE, bool MIXED, int GEOM, int FAM>
 static hipError_t path_tiled_f32_f(int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
     if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void *)path_kernel_tiled<float, MIXED, GEOM, FAM>,
+        hipError_t e = hipFuncSetAttribute((const void *)path_kernel_tiled<float, PDE, MIXED, GEOM, FAM>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((path_kernel_tiled<float, MIXED, GEOM, FAM>), dim3(grid), dim3(tiled_wg<float, FAM, GEOM>()), lds, s, a);
+    hipLaunchKernelGGL((path_kernel_tiled<float, PDE, MIXED, GEOM, FAM>), dim3(grid), dim3(tiled_wg<float, PDE, FAM, GEOM>()), lds, s, a);
     return hipGetLastError();
 }
 
-template <bool MIXED, int GEOM>
+template <int PDE, bool MIXED, int GEOM>
 static hipError_t path_tiled_f32(int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
-    return a.pp.step == STEP_CV ? path_tiled_f32_f<MIXED, GEOM, STEP_CV>(grid, lds, s, a)
-                                : path_tiled_f32_f<MIXED, GEOM, STEP_ANY>(grid, lds, s, a);
+    return a.pp.step == STEP_CV ? path_tiled_f32_f<PDE, MIXED, GEOM, STEP_CV>(grid, lds, s, a)
+                                : path_tiled_f32_f<PDE, MIXED, GEOM, STEP_ANY>(grid, lds, s, a);
 }
 
-hipError_t launch_path_tiled_f32(int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
-    if (geom == GeomDisc)
-        return mixed ? path_tiled_f32<true, GeomDisc>(grid, lds, s, a) : path_tiled_f32<false, GeomDisc>(grid, lds, s, a);
-    return mixed ? path_tiled_f32<true, GeomRect>(grid, lds, s, a) : path_tiled_f32<false, GeomRect>(grid, lds, s, a);
+template <int PDE, int GEOM> static hipError_t path_tiled_f32_m(bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
+    return mixed ? path_tiled_f32<PDE, true, GEOM>(grid, lds, s, a) : path_tiled_f32<PDE, false, GEOM>(grid, lds, s, a);
+}
+
+hipError_t launch_path_tiled_f32(int pde, int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
+    if (pde == PDE_TABLE) return geom == GeomRect ? path_tiled_f32_m<PDE_TABLE, GeomRect>(mixed, grid, lds, s, a) : hipErrorInvalidValue;
+    return geom == GeomDisc ? path_tiled_f32_m<PDE_VARCOEF_LUT, GeomDisc>(mixed, grid, lds, s, a)
+                            : path_tiled_f32_m<PDE_VARCOEF_LUT, GeomRect>(mixed, grid, lds, s, a);
 }
 
 template <int PDE>

@@ -52,37 +52,43 @@ hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const
     }
 }
 
-template <int GEOM> static int path_tiled_wg_g(int precision, int step) {
+template <int PDE, int GEOM> static int path_tiled_wg_g(int precision, int step) {
     if (step == STEP_CV)
-        return precision == PDDS_FP64 ? tiled_wg<double, STEP_CV, GEOM>() : tiled_wg<float, STEP_CV, GEOM>();
-    return precision == PDDS_FP64 ? tiled_wg<double, STEP_ANY, GEOM>() : tiled_wg<float, STEP_ANY, GEOM>();
+        return precision == PDDS_FP64 ? tiled_wg<double, PDE, STEP_CV, GEOM>() : tiled_wg<float, PDE, STEP_CV, GEOM>();
+    return precision == PDDS_FP64 ? tiled_wg<double, PDE, STEP_ANY, GEOM>() : tiled_wg<float, PDE, STEP_ANY, GEOM>();
 }
 
-int path_tiled_wg(int precision, int step, int geom) {
-    return geom == GeomDisc ? path_tiled_wg_g<GeomDisc>(precision, step) : path_tiled_wg_g<GeomRect>(precision, step);
+int path_tiled_wg(int pde, int precision, int step, int geom) {
+    if (pde == PDE_TABLE) return path_tiled_wg_g<PDE_TABLE, GeomRect>(precision, step);
+    return geom == GeomDisc ? path_tiled_wg_g<PDE_VARCOEF_LUT, GeomDisc>(precision, step)
+                            : path_tiled_wg_g<PDE_VARCOEF_LUT, GeomRect>(precision, step);
 }
 
-template <bool MIXED, int GEOM, int FAM>
+template <int PDE, bool MIXED, int GEOM, int FAM>
 static hipError_t path_tiled_f64_f(int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
     if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void *)path_kernel_tiled<double, MIXED, GEOM, FAM>,
+        hipError_t e = hipFuncSetAttribute((const void *)path_kernel_tiled<double, PDE, MIXED, GEOM, FAM>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((path_kernel_tiled<double, MIXED, GEOM, FAM>), dim3(grid), dim3(tiled_wg<double, FAM, GEOM>()), lds, s, a);
+    hipLaunchKernelGGL((path_kernel_tiled<double, PDE, MIXED, GEOM, FAM>), dim3(grid), dim3(tiled_wg<double, PDE, FAM, GEOM>()), lds, s, a);
     return hipGetLastError();
 }
 
-template <bool MIXED, int GEOM>
+template <int PDE, bool MIXED, int GEOM>
 static hipError_t path_tiled_f64(int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
-    return a.pp.step == STEP_CV ? path_tiled_f64_f<MIXED, GEOM, STEP_CV>(grid, lds, s, a)
-                                : path_tiled_f64_f<MIXED, GEOM, STEP_ANY>(grid, lds, s, a);
+    return a.pp.step == STEP_CV ? path_tiled_f64_f<PDE, MIXED, GEOM, STEP_CV>(grid, lds, s, a)
+                                : path_tiled_f64_f<PDE, MIXED, GEOM, STEP_ANY>(grid, lds, s, a);
 }
 
-hipError_t launch_path_tiled_f64(int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
-    if (geom == GeomDisc)
-        return mixed ? path_tiled_f64<true, GeomDisc>(grid, lds, s, a) : path_tiled_f64<false, GeomDisc>(grid, lds, s, a);
-    return mixed ? path_tiled_f64<true, GeomRect>(grid, lds, s, a) : path_tiled_f64<false, GeomRect>(grid, lds, s, a);
+template <int PDE, int GEOM> static hipError_t path_tiled_f64_m(bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
+    return mixed ? path_tiled_f64<PDE, true, GEOM>(grid, lds, s, a) : path_tiled_f64<PDE, false, GEOM>(grid, lds, s, a);
+}
+
+hipError_t launch_path_tiled_f64(int pde, int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a) {
+    if (pde == PDE_TABLE) return geom == GeomRect ? path_tiled_f64_m<PDE_TABLE, GeomRect>(mixed, grid, lds, s, a) : hipErrorInvalidValue;
+    return geom == GeomDisc ? path_tiled_f64_m<PDE_VARCOEF_LUT, GeomDisc>(mixed, grid, lds, s, a)
+                            : path_tiled_f64_m<PDE_VARCOEF_LUT, GeomRect>(mixed, grid, lds, s, a);
 }
 
 template <int PDE>

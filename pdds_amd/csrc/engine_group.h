@@ -106,7 +106,7 @@ struct NoOut {};
 
 // the coefficients that move X and Y (the others are not formed)
 template <class R, int PDE> __device__ __forceinline__ void group_motion(const PathKernelArgs &a, GroupState<R> &p) {
-    const LutTile none{nullptr, 0, 0, 0, 0};
+    const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     Coef<R> co;
     pde_coef_t<PDE, R, false>(p.x, p.y, a.pp, none, p.k2, co);
     p.s00 = co.s00; p.s11 = co.s11; p.b0 = co.b0; p.b1 = co.b1; p.c = co.c;
@@ -152,7 +152,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
     const int lane = __lane_id();
     const int sub = lane & (G - 1);
     const int base = lane & ~(G - 1);
-    const LutTile none{nullptr, 0, 0, 0, 0};
+    const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     const R beta = REC && p.second ? (R)0 : (R)a.beta;
     const R h = p.h, sqrth = p.sqrth;
     R x = p.x, y = p.y, Y = p.Y, Z = p.Z, xi = p.xi, nzc = p.nzc, nxc = p.nxc;

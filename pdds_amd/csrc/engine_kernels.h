@@ -740,7 +740,7 @@ template <class R, int PDE, int FAM> constexpr int path_waves_f() {
 template <class R, int PDE, bool MIXED, int GEOM, int FAM, bool REFL = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(path_waves_f<R, PDE, FAM>()))) path_kernel(PathKernelArgs a) {
     const int lane = __lane_id();
-    const LutTile none{nullptr, 0, 0, 0, 0};
+    const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     Walker<R, PDE, MIXED, GEOM, FAM, REFL> w;
     w.init();
     bool done = false;
@@ -786,7 +786,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
     if (gg >= a.total) return;
     const int kn = find_knot(a, gg);
     const KnotDesc &kd = a.knots[kn];
-    const LutTile none{nullptr, 0, 0, 0, 0};
+    const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     const R h = (R)kd.h, sqrth = (R)kd.sqrth, beta = (R)a.beta, k2 = (R)kd.k2;
     R rect[domain_len<GEOM>()];
     for (int q = 0; q < domain_len<GEOM>(); ++q) rect[q] = (R)kd.dom[q];
@@ -856,21 +856,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
 }
 
 // ----------------------------------------------------------------------------
-// LDS-tiled path kernel (coefficient-LUT problem): one work-group per CU.  The work-group
+// LDS-tiled path kernel (coefficient-LUT and tabulated problems): one work-group per CU.  The work-group
 // works on one patch at a time: it copies the patch's plane-a tile into LDS, its waves take
 // paths from the patch's queue until it is drained, and once every wave is done it moves to
-// the next patch with paths left.  The 16 taps of a step are then LDS reads; only field 4
-// (one 16-byte load per tap row, 4 per step, from its float plane) and taps outside the tile
-// go to the vector L1.
+// the next patch with paths left.  The 16 taps of a step are then LDS reads; only field 4 of the
+// coefficient LUT (one 16-byte load per tap row, 4 per step, from its float plane) and taps
+// outside the tile go to the vector L1.  The tabulated problem holds both planes of its eight
+// fields, and with a VR + CV step that of mu and F if its grid is the same and there is room.
+// Without the tile its step waits for 32 (48) scattered 16-byte reads of the vector L1, about a cache
+// line a cycle: 357 knots, 1.4 10^6 paths, a table of 128 x 128, FP64, h = 5e-4: VR + CV step 15.5 ms
+// persistent, 9.4 ms tiled; control variates 10.0 and 6.4 ms (FP32 9.3 and 5.2).
 // ----------------------------------------------------------------------------
 // one work-group per CU holding every wave the register budget allows (the run-time step-family
 // variants one wave less, as in path_kernel, and so the FP32 annular-sector kernels, whose
 // sector distance needs more registers than three waves per SIMD leave)
-template <class R, int FAM, int GEOM> constexpr int tiled_waves() {
-    return path_waves_f<R, PDE_VARCOEF_LUT, FAM>() -
-           (sizeof(R) == 4 && GEOM == GeomDisc && path_waves_f<R, PDE_VARCOEF_LUT, FAM>() > 2 ? 1 : 0);
+template <class R, int PDE, int FAM, int GEOM> constexpr int tiled_waves() {
+    if (PDE == PDE_TABLE) return 2;
+    return path_waves_f<R, PDE, FAM>() - (sizeof(R) == 4 && GEOM == GeomDisc && path_waves_f<R, PDE, FAM>() > 2 ? 1 : 0);
 }
-template <class R, int FAM, int GEOM> constexpr int tiled_wg() { return 64 * 4 * tiled_waves<R, FAM, GEOM>(); }
+template <class R, int PDE, int FAM, int GEOM> constexpr int tiled_wg() { return 64 * 4 * tiled_waves<R, PDE, FAM, GEOM>(); }
 
 __device__ __forceinline__ int find_patch(const PatchDesc *p, int n, int64_t g) {
     int lo = 0, hi = n;
@@ -882,13 +886,13 @@ __device__ __forceinline__ int find_patch(const PatchDesc *p, int n, int64_t g) 
     return lo;
 }
 
-template <class R, bool MIXED, int GEOM, int FAM>
-__global__ void __launch_bounds__((tiled_wg<R, FAM, GEOM>())) __attribute__((amdgpu_waves_per_eu(tiled_waves<R, FAM, GEOM>())))
+template <class R, int PDE, bool MIXED, int GEOM, int FAM>
+__global__ void __launch_bounds__((tiled_wg<R, PDE, FAM, GEOM>())) __attribute__((amdgpu_waves_per_eu(tiled_waves<R, PDE, FAM, GEOM>())))
 path_kernel_tiled(PathKernelArgs a) {
     extern __shared__ float4 tile[];
     __shared__ int s_patch;
     const int lane = __lane_id();
-    Walker<R, PDE_VARCOEF_LUT, MIXED, GEOM, FAM> w;
+    Walker<R, PDE, MIXED, GEOM, FAM> w;
     w.init();
     // first patch: the one holding this work-group's share of the batch's path range
     int p = find_patch(a.patches, a.n_patches, (int64_t)blockIdx.x * a.total / (int64_t)gridDim.x);
@@ -918,12 +922,19 @@ path_kernel_tiled(PathKernelArgs a) {
         p = __builtin_amdgcn_readfirstlane(s_patch);   // uniform: the patch, its tile and queue stay scalar
         if (p < 0) break;
         const PatchDesc pd = a.patches[p];
-        const LutTile T{(lds_float4 *)tile, pd.c0, pd.r0, pd.tw, pd.tiled ? pd.th : 0, pd.pitch};
+        const int plane = pd.pitch * pd.th;
+        const LutTile T{(lds_float4 *)tile, pd.c0, pd.r0, pd.tw, pd.tiled ? pd.th : 0, pd.pitch, plane,
+                        pd.tiled == 3 ? 2 * plane : 0};
         if (pd.tiled) {
             const int nt = pd.tw * pd.th;
             for (int i = threadIdx.x; i < nt; i += blockDim.x) {
                 const int r = i / pd.tw, c = i - r * pd.tw;
-                tile[r * pd.pitch + c] = a.pp.lut.a[(int64_t)(pd.r0 + r) * a.pp.lut.px + (pd.c0 + c)];
+                const int64_t at = (int64_t)(pd.r0 + r) * a.pp.lut.px + (pd.c0 + c);
+                tile[r * pd.pitch + c] = a.pp.lut.a[at];
+                if constexpr (PDE == PDE_TABLE) {
+                    tile[plane + r * pd.pitch + c] = ((const float4 *)a.pp.lut.b)[at];
+                    if (T.pv) tile[T.pv + r * pd.pitch + c] = a.pp.vlut.a[at];
+                }
             }
         }
         __syncthreads();

@@ -144,7 +144,8 @@ struct Records {
 struct PatchDesc {
     int64_t pbeg, pend;
     int32_t c0, r0, tw, th;
-    int32_t tiled, pitch;   // pitch: texels per LDS tile row (tw plus the run's lut_pad)
+    int32_t tiled, pitch;   // tiled: planes in the tile (coefficient LUT: 1, tabulated problem: 2, or 3
+                            // with mu and F), 0: none; pitch: texels per LDS tile row (tw plus the run's lut_pad)
 };
 
 struct PathKernelArgs {
@@ -250,9 +251,13 @@ struct PathLaunch {
 };
 
 // Launchers (defined in engine_f64.hip / engine_f32.hip)
-hipError_t launch_path_tiled_f64(int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
-hipError_t launch_path_tiled_f32(int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
-int path_tiled_wg(int precision, int step, int geom);   // block size of the LDS-tiled kernel
+hipError_t launch_path_tiled_f64(int pde, int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
+hipError_t launch_path_tiled_f32(int pde, int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
+// The tabulated problem takes the LDS-tiled kernel from this many paths per lane of its grid (357 knots, a
+// table of 128 x 128, FP64, VR step: 285 10^3 paths 4.6 ms, 5.4 without; 1.4 10^6 6.7 ms and 11; at 142 10^3
+// the two are equal, 4.0 ms)
+constexpr int64_t kTableTileLane = 1;
+int path_tiled_wg(int pde, int precision, int step, int geom);   // block size of the LDS-tiled kernel
 hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 // Group kernel (rectangles, control-variate step): lanes that carry one path of a launch of that many

@@ -656,7 +656,8 @@ PDDS_HD const T &lut_at(const void *base, uint32_t byte_off) {
     return *(const T *)((const char *)base + byte_off);
 }
 
-// A rectangle of plane a held in LDS: padded columns [c0, c0 + tw), rows [r0, r0 + th),
+// A rectangle of texels held in LDS: plane a's, and with eight fields plane b's `pb` texels behind it
+// (and a second table's plane a `pv` texels behind it, if pv is not 0): padded columns [c0, c0 + tw), rows [r0, r0 + th),
 // row-major with `pitch` texels per row (pitch >= tw; the spare texels change which LDS banks
 // the rows start on).  th == 0 means no tile.  The pointer is typed in the LDS address space,
 // so tile reads are ds_read_b128 and never merge with the global-memory branch into generic
@@ -670,6 +671,7 @@ struct LutTile {
     lds_float4 *lds;
     int c0, r0, tw, th;
     int pitch;
+    int pb, pv;
 };
 
 // The 16-tap accumulation of lut_eval_t.  SRC 0: plane a from global memory; 1: from the LDS
@@ -710,7 +712,9 @@ PDDS_HD void lut_accum(const LutView &L, const LutTile &T, lds_float4 *tp, bool 
             const float4 q0 = A[a];
             c[0] = q0.x; c[1] = q0.y; c[2] = q0.z; c[3] = q0.w;
             if constexpr (NF > 5) {
-                const float4 q1 = lut_at<float4>(L.b, (r0 + (uint32_t)a) * 16u);
+                float4 q1;
+                if (SRC == 1 || (SRC == 2 && in)) q1 = tp[T.pb + b * T.pitch + a];
+                else q1 = lut_at<float4>(L.b, (r0 + (uint32_t)a) * 16u);
                 c[4] = q1.x; c[5] = q1.y; c[6] = q1.z; c[7] = q1.w;
             }
 #pragma unroll
@@ -734,8 +738,8 @@ PDDS_HD void lut_accum(const LutView &L, const LutTile &T, lds_float4 *tp, bool 
 
 // Evaluate fields [0, NF) (NF <= 8) at (x,y):
 //   sum_b wy_b * sum_a wx_a * C[clamp(j-1+b)][clamp(i-1+a)][f]
-// With TILED, a lane whose 4x4 taps lie inside the tile reads fields 0..3 from LDS (one
-// 16-byte LDS read per tap) and the others read them from plane a; the values, and the
+// With TILED, a lane whose 4x4 taps lie inside the tile reads fields 0..3 (and 4..7 of eight) from
+// LDS (one 16-byte LDS read per tap and plane) and the others read them from the planes; the values, and the
 // order of the fused multiply-adds, are the same either way.  A wave whose live lanes are all
 // inside the tile takes a path with LDS reads only, so no LDS read waits for the wave's
 // global loads.
@@ -774,7 +778,7 @@ PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF],
 
 template <class R, int NF>
 PDDS_HD void lut_eval(const LutView &L, R x, R y, R out[NF]) {
-    const LutTile none{nullptr, 0, 0, 0, 0};
+    const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     lut_eval_t<R, NF, false>(L, none, x, y, out);
 }
 

@@ -67,7 +67,8 @@ template <class R> PDDS_HD R fused(R a, R b, R c) {
     else return c + a * b;
 }
 
-// TILED: the coefficient LUT's fields 0..3 are read from the LDS tile T where it covers X.
+// TILED: the coefficient LUT's fields 0..3 (the tables' eight, and those of mu and F) are read from the
+// LDS tile T where it covers X.
 // k2: the Helmholtz parameter of this path's problem (per knot, so one launch can carry
 // requests with different k^2).  live: whether the caller uses this lane's values.
 template <int PDE, class R, bool TILED, int FAM = STEP_CV>
@@ -100,7 +101,7 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
         // textures, Solvers/MCinCUDA.cu:453-478; here sigma and b as well), so a problem runs
         // from its samples alone
         R v[8];
-        lut_eval<R, 8>(P.lut, x, y, v);
+        lut_eval_t<R, 8, TILED>(P.lut, T, x, y, v, live);
         co.s00 = v[0]; co.s11 = v[1];
         co.b0 = v[2]; co.b1 = v[3]; co.c = v[4]; co.f = v[5];
         co.g0 = v[6]; co.g1 = v[7];
@@ -142,7 +143,17 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
         } else if (P.step == STEP_VRCV) {
             // mu and F from their table (Integrators/FKACIntegrator.hpp:100-112)
             R w[4];
-            lut_eval<R, 4>(P.vlut, x, y, w);
+            if constexpr (PDE == PDE_TABLE && TILED) {
+                if (T.pv) {
+                    LutTile V = T;
+                    V.lds += T.pv;
+                    lut_eval_t<R, 4, true>(P.vlut, V, x, y, w, live);
+                } else {
+                    lut_eval<R, 4>(P.vlut, x, y, w);
+                }
+            } else {
+                lut_eval<R, 4>(P.vlut, x, y, w);
+            }
             co.m0 = w[0]; co.m1 = w[1]; co.F0 = w[2]; co.F1 = w[3];
         }
     }
@@ -150,7 +161,7 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
 
 template <int PDE, class R, int FAM = STEP_CV>
 PDDS_HD void pde_coef(R x, R y, const PdeParams &P, Coef<R> &co) {
-    const LutTile none{nullptr, 0, 0, 0, 0};
+    const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     pde_coef_t<PDE, R, false, FAM>(x, y, P, none, (R)P.k2, co);
 }
 
