@@ -302,14 +302,14 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
     const bool table = prob->pde == PDDS_PDE_TABLE;
     // the tabulated problem's tile holds its fields' two planes, and with a VR + CV step that of mu
     // and F where its grid is the same and there is room; launches that fill the tiled grid, in
-    // rectangles (not the FP32 VR + CV step, whose FP32 rounding follows the persistent kernel's code)
+    // rectangles (not the FP32 VR and VR + CV steps, whose rounding follows the persistent kernel's code)
     const LutView &la = pp.lut, &lv = pp.vlut;
     const int tile_planes = !table ? 1 : pp.step == STEP_VRCV && la.nx == lv.nx && la.ny == lv.ny && la.px == lv.px &&
                                                  la.ox == lv.ox && la.oy == lv.oy && la.sx == lv.sx && la.sy == lv.sy ? 3 : 2;
     const bool tiled =
         persistent && r->lut_lds != 0 && pp.refl == 0 &&
         ((prob->pde == PDDS_PDE_VARCOEF_LUT && pp.lut.nf == 5) ||
-         (table && geom == GeomRect && (r->precision == PDDS_FP64 || pp.step != STEP_VRCV) &&
+         (table && geom == GeomRect && (r->precision == PDDS_FP64 || pp.step == STEP_CV || pp.step == STEP_PLAIN) &&
           all_paths >= kTableTileLane * e->n_cu * (int64_t)path_tiled_wg(prob->pde, r->precision, r->step, geom)));
     const size_t tile_cap = e->lds_max > 1024 ? e->lds_max - 1024 : 0;
     std::vector<size_t> ord(knots.size());

@@ -33,7 +33,7 @@ def _problem(eng, n, nv):
 # 64: every tile fits with three planes; 160: some with three, some with two; 300: some with none
 @pytest.mark.parametrize("n,nv", [(64, 64), (64, 50), (160, 160), (300, 300)])
 @pytest.mark.parametrize("precision,step", [("fp64", 0), ("fp64", 1), ("fp64", 2), ("fp64", 3), ("fp32", 0),
-                                            ("fp32", 1), ("fp32", 3)])
+                                            ("fp32", 1), ("fp32", 2), ("fp32", 3)])
 def test_tiled_equals_persistent_and_oracle(eng, n, nv, precision, step):
     from pdds_amd.engine import Mesh, default_run
     from pdds_amd.workloads import relative_fac
