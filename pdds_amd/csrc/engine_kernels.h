@@ -277,6 +277,14 @@ __device__ __forceinline__ void normals4_f32(uint32_t call, uint32_t path, uint3
     n[3] = r2 * __builtin_amdgcn_sinf(u4);
 }
 
+// A wave-uniform Philox key word as a value of this step: its round keys are then added up in the step,
+// on the scalar unit.  As loop invariants they fill the scalar registers of the FP64 coefficient-LUT
+// kernels and are spilled, a v_readlane each (343 10^6 paths: path kernels 543 ms, 537 so).
+__device__ __forceinline__ uint32_t key_here(uint32_t k) {
+    asm volatile("" : "+s"(k));
+    return k;
+}
+
 // Normal pair of step s.st for this lane's path.  FP32: one Philox call per even step gives
 // the normals of steps st and st + 1; `even` is the parity of st, which the path kernels keep
 // the same for every lane of a wave (paths only start on odd wave iterations), so the draw is a
@@ -563,10 +571,12 @@ struct Walker {
     template <bool TILED, bool DRAW_FIRST>
     __device__ __forceinline__ void step(const PathKernelArgs &a, const LutTile &T, int it) {
         const R h = MIXED ? hk : (R)a.h, sqrth = MIXED ? sqhk : (R)a.sqrth, beta = (R)a.beta;
-        const uint32_t strm = MIXED ? kstream : a.stream;
+        constexpr bool keyed = sizeof(R) == 8 && PDE == PDE_VARCOEF_LUT;
+        const uint32_t seed = keyed ? key_here(a.seed) : a.seed;
+        const uint32_t strm = MIXED ? kstream : keyed ? key_here(a.stream) : a.stream;
         const R kk2 = MIXED ? k2 : (R)a.pp.k2;
         bool stepping = active && !fresh;
-        if constexpr (DRAW_FIRST) draw_normals<R>(s, a.seed, strm, kid, pn1, pn2, (it & 1) == 0);
+        if constexpr (DRAW_FIRST) draw_normals<R>(s, seed, strm, kid, pn1, pn2, (it & 1) == 0);
         if constexpr (fast) {
             em_step<R, PDE, FAM>(s, co, h, sqrth, pn1, pn2, a.pp.step);
             s.st += 1u;
@@ -578,7 +588,7 @@ struct Walker {
                 const bool rside = refl_kind(rk, rmask);
                 const bool lep = rside && (a.pp.rho <= 0.0 || rd > -(R)a.pp.rho);
                 R E = (R)0;
-                if (stepping && lep) E = draw_exponential<R>(s.st, s.path, a.seed, strm, kid);
+                if (stepping && lep) E = draw_exponential<R>(s.st, s.path, seed, strm, kid);
                 refl_step<R, PDE, FAM>(t, co, a.pp, h, sqrth, pn1, pn2, a.pp.step, lep, E, rnx, rny, rd, lt);
             } else {
                 em_step<R, PDE, FAM>(t, co, h, sqrth, pn1, pn2, a.pp.step);
@@ -622,7 +632,7 @@ struct Walker {
             rd = d; rk = kind; rnx = nx; rny = ny;
         }
         pde_coef_t<PDE, R, TILED, FAM>(s.x, s.y, a.pp, T, kk2, co, active);
-        if constexpr (!DRAW_FIRST) draw_normals<R>(s, a.seed, strm, kid, pn1, pn2, (it & 1) != 0);
+        if constexpr (!DRAW_FIRST) draw_normals<R>(s, seed, strm, kid, pn1, pn2, (it & 1) != 0);
         R nrm;
         if constexpr (fast) {
             nrm = side_norm(xside, co.s00, co.s11);
@@ -940,8 +950,14 @@ path_kernel_tiled(PathKernelArgs a) {
         __syncthreads();
         WavePool pool;
         bool drained = false, done = false;
+        // One step per pass, or two where paths start on every other step (may_start) and the registers
+        // hold it: as one step with a count, an FP32 loop copies some 20 values at its head, beside
+        // about 400 vector instructions a step.  (Disc 2.8 -> 2.5 ms, tabulated problem 5.2 -> 4.9 and,
+        // 285 10^3 paths, 3.9 -> 3.4 ms.  The kernels of three waves per SIMD spill with two steps:
+        // 338 ms one step, 357 two; the run-time families' FP32 rounding follows the one-step form.)
+        constexpr bool pairs = sizeof(R) == 4 && FAM == STEP_CV && tiled_waves<R, PDE, FAM, GEOM>() == 2;
         for (int it = 1;; ++it) {
-            const bool can_start = may_start<R>(it);
+            const bool can_start = pairs || may_start<R>(it);
             if (can_start) {
                 const bool need = !w.active && !done;
                 const unsigned long long m = __ballot(need);
@@ -957,7 +973,8 @@ path_kernel_tiled(PathKernelArgs a) {
             }
             // FP64 overlaps the next step's normal draw with the LUT reads; the shorter FP32
             // draw goes first (measured: each order is about 1 % faster in its precision)
-            w.template step<true, sizeof(R) == 4>(a, T, it);
+            w.template step<true, sizeof(R) == 4>(a, T, pairs ? 1 : it);
+            if constexpr (pairs) w.template step<true, true>(a, T, 2);
         }
         __syncthreads();   // every wave is done with this tile
     }
