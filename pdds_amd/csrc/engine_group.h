@@ -22,7 +22,7 @@
 // (group_lanes) and widens where a wave's last paths leave room.  Measured against one path per
 // lane: 4 points x 1000 paths 1.9 -> 0.29 ms, one knot of the recorded run 4.7 -> 0.58, the whole
 // run 8.0 -> 3.6, Poisson FP32 (0.6 M paths) 8.2 -> 3.4, server burst 139 -> 83 ms; per-path records
-// of 1e5 two-phase paths 9.5 -> 5.4, 16 Robin points x 4096 paths 8.5 -> 4.2, 390 k paths of a LUT
+// of 1e5 two-phase paths 9.5 -> 5.4, 16 Robin points x 4096 paths 8.5 -> 4.0, 390 k paths of a LUT
 // assembly 7.3 -> 5.6 (FP64) and 8.9 -> 4.0 ms (FP32).
 #pragma once
 #include <type_traits>
@@ -189,7 +189,18 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
     R pd = 0, pLt = 0, qx = 0, qy = 0, qd = 0, qlt = 0, d = p.rd, lt = p.lt;
     int pk = 0, qk = 0, kind = p.rk;
     R E = 0;
-    if constexpr (REFL) E = draw_exponential<R>(st_l, p.g - p.poff, a.seed, p.strm, p.kid);
+    // constant motion: the root of the lane's own Lepingle step for a side in x and one in y (outside
+    // the rectangle's corners a normal has one component, +-1), which so leaves the serial part
+    // (5 points x 500 paths 2.34 -> 2.13 ms, 20 x 20000 18.9 -> 17.6)
+    R Sx = 0, Sy = 0;
+    if constexpr (REFL) {
+        E = draw_exponential<R>(st_l, p.g - p.poff, a.seed, p.strm, p.kid);
+        if constexpr (!VAR) {
+            const R hE = ((R)2.0 * h) * E;
+            Sx = RM<R>::sqrt((co.s00 * co.s00) * hE + dx[0] * dx[0]);
+            Sy = RM<R>::sqrt((co.s11 * co.s11) * hE + dy[0] * dy[0]);
+        }
+    }
     static_for<G>([&](auto kk) {
         constexpr int K = decltype(kk)::value;
         const bool me = group_lane<G, K>();
@@ -202,19 +213,31 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
             // refl_step's move: the Lepingle step while the nearest side reflects (within rho of it)
             R nx, ny, L = (R)0;
             group_normal<R>(kind, nx, ny);
-            const R j0 = group_bcast<G, K>(i0[0]), j1 = group_bcast<G, K>(i1[0]);
             const bool lep = refl_kind(kind, p.rmask) && (a.pp.rho <= 0.0 || d > -(R)a.pp.rho);
-            if (__any(lep)) {
-                const R ga = nx * co.s00, gb = ny * co.s11;
-                const R uc = (ga * j0 + gb * j1) + (nx * co.b0 + ny * co.b1) * h;
-                const R M = (R)0.5 * (uc + RM<R>::sqrt((ga * ga + gb * gb) * (((R)2.0 * h) * group_bcast<G, K>(E)) + uc * uc));
+            R mx, my;
+            if constexpr (VAR) {
+                const R j0 = group_bcast<G, K>(i0[0]), j1 = group_bcast<G, K>(i1[0]);
+                if (__any(lep)) {
+                    const R ga = nx * co.s00, gb = ny * co.s11;
+                    const R uc = (ga * j0 + gb * j1) + (nx * co.b0 + ny * co.b1) * h;
+                    const R M = (R)0.5 * (uc + RM<R>::sqrt((ga * ga + gb * gb) * (((R)2.0 * h) * group_bcast<G, K>(E)) + uc * uc));
+                    L = lep ? RM<R>::fmax((R)0, M + d) : (R)0;
+                }
+                mx = em_move(co.b0, h, co.s00, j0);
+                my = em_move(co.b1, h, co.s11, j1);
+            } else {
+                mx = group_bcast<G, K>(dx[0]);
+                my = group_bcast<G, K>(dy[0]);
+                const R sx = group_bcast<G, K>(Sx), sy = group_bcast<G, K>(Sy);
+                const R S = nx != (R)0 ? sx : sy;
+                const R M = (R)0.5 * (nx * mx + ny * my + S);
                 L = lep ? RM<R>::fmax((R)0, M + d) : (R)0;
             }
             pd = me ? d : pd;
             pk = me ? kind : pk;
             pLt = me ? L + lt : pLt;
-            x = x + em_move(co.b0, h, co.s00, j0);
-            y = y + em_move(co.b1, h, co.s11, j1);
+            x = x + mx;
+            y = y + my;
             x = lep ? x - L * nx : x;
             y = lep ? y - L * ny : y;
             R ex, ey;

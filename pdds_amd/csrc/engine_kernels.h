@@ -4,16 +4,19 @@
 //
 // Two kernels per assembly batch:
 //  * path_kernel: one path per lane.  In persistent form every lane whose path
-//    has stopped takes the next path of the batch from a device-wide counter
-//    (one atomic per wave per refill), so lanes idle only at the very end of the
-//    batch -- the on-device form of the reference's relaunch-and-refill loop
+//    has stopped takes the next path of the batch from its wave's pool, which is
+//    refilled from one of eight queues (one atomic per chunk), so lanes idle only
+//    at the very end of the batch -- the on-device form of the reference's relaunch-and-refill loop
 //    (Solvers/SolveLoop.cuh:59-74, solveCUDA.cuh:118-168).  Each path is stepped
 //    by the control-variate Euler-Maruyama scheme (Integrators/FKACIntegrator.hpp:46-57),
 //    stopped by the Gobet-shifted test (Integrators/FKACIntegrator.hpp:168-186),
 //    and its exit record (projection, Y, score) is written at its global path
 //    index; steps are summed per knot.  The plain form launches one lane per path,
-//    no refill.
-//  * reduce_kernel: one work-group per work item of P paths of one knot.  Per
+//    no refill; path_kernel_tiled reads its tables from LDS tiles; small launches
+//    and those of constant-motion problems run in engine_group.h's group_kernel,
+//    several lanes per path.
+//  * reduce16_kernel (reduce_kernel for what it does not take): work items of P
+//    paths of one knot per work-group.  Per
 //    sub-batch of S paths it forms the per-side RBF moments Phi_j = sum Y phi_j(X)
 //    (m exps per exit, where Meshes/stencil.cpp:244-307 spends m^2), then
 //    G_beta = -Psi^-T Phi per CSR column, and accumulates sums and sums of squares
