@@ -221,14 +221,15 @@ def summarize_traffic(pmc_dir, out_path):
            "commands": list(TRAFFIC_RUNS.values()) + ["python3 bench.py --summarize-traffic gpurun_out/pmc"]}
     fetch = _counter_rows(pmc_dir, "fetch", "FETCH_SIZE")
     write = _counter_rows(pmc_dir, "write", "WRITE_SIZE")
-    for label, pat in (("path_kernel", "path_kernel"), ("reduce_kernel", "reduce_kernel")):
+    # (the reduction of an assembly is one launch per class of stencils: their sum)
+    for label, pat, of in (("path_kernel", "path_kernel", np.mean), ("reduction", "reduce", np.sum)):
         fk = [v for k, v in fetch if pat in k]
         wk = [v for k, v in write if pat in k]
         if not fk or not wk:
             continue
         rec = {"kernel": [k for k, v in fetch if pat in k][0][:120], "launches": len(fk),
-               "fetch_size_kib": float(np.mean(fk)), "write_size_kib": float(np.mean(wk)),
-               "fetch_bytes": float(np.mean(fk)) * 1024.0 * ff, "write_bytes": float(np.mean(wk)) * 1024.0 * wf}
+               "fetch_size_kib": float(of(fk)), "write_size_kib": float(of(wk)),
+               "fetch_bytes": float(of(fk)) * 1024.0 * ff, "write_bytes": float(of(wk)) * 1024.0 * wf}
         rec["bytes_per_launch"] = rec["fetch_bytes"] + rec["write_bytes"]
         out[label] = rec
     if "path_kernel" in out:

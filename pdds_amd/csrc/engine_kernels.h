@@ -282,7 +282,7 @@ __device__ __forceinline__ void normals4_f32(uint32_t call, uint32_t path, uint3
 
 // A wave-uniform Philox key word as a value of this step: its round keys are then added up in the step,
 // on the scalar unit.  As loop invariants they fill the scalar registers of the FP64 coefficient-LUT
-// kernels and are spilled, a v_readlane each (343 10^6 paths: path kernels 543 ms, 537 so).
+// kernels and are spilled, a v_readlane each (3437 x 100000 paths: an assembly 588 ms, 582 so).
 __device__ __forceinline__ uint32_t key_here(uint32_t k) {
     asm volatile("" : "+s"(k));
     return k;
@@ -878,7 +878,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
 // fields, and with a VR + CV step that of mu and F if its grid is the same and there is room.
 // Without the tile its step waits for 32 (48) scattered 16-byte reads of the vector L1, about a cache
 // line a cycle: 357 knots, 1.4 10^6 paths, a table of 128 x 128, FP64, h = 5e-4: VR + CV step 15.5 ms
-// persistent, 9.4 ms tiled; control variates 10.0 and 6.4 ms (FP32 9.3 and 5.2).
+// persistent, 9.4 ms tiled; control variates 10.0 and 6.4 ms (FP32 9.3 and 4.9).
 // ----------------------------------------------------------------------------
 // one work-group per CU holding every wave the register budget allows (the run-time step-family
 // variants one wave less, as in path_kernel, and so the FP32 annular-sector kernels, whose
