@@ -909,26 +909,39 @@ path_kernel_tiled(PathKernelArgs a) {
     w.init();
     // first patch: the one holding this work-group's share of the batch's path range
     int p = find_patch(a.patches, a.n_patches, (int64_t)blockIdx.x * a.total / (int64_t)gridDim.x);
+    bool first = true;
     while (true) {
         if (threadIdx.x < 64) {
-            // the next patch with paths left, 64 counters at a time
-            int pick = -1;
-            for (int k0 = 0; k0 < a.n_patches && pick < 0; k0 += 64) {
+            // the first patch: the next one of the work-group's share with paths left; then the one with the
+            // most paths left of the next 1024 that have any, 64 counters at a time.  Taken in their
+            // order, work-groups follow each other through patches that are nearly drained, each time
+            // with a tile to stage, thin waves and a longest path to wait for (3437 x 100000 paths: FP64
+            // 541 ms against 509, FP32 298 and 256; a disc's 32 10^6 paths, 385 patches: 33.3 and 27.5);
+            // with the largest taken first as well, all would start on one patch.
+            long long most = 0;
+            int at = -1;
+            for (int k0 = 0; k0 < a.n_patches; k0 += 64) {
                 const int k = k0 + lane;
                 int c = p + k;
                 c = c < a.n_patches ? c : c - a.n_patches;
-                bool left = false;
                 if (k < a.n_patches) {
                     const unsigned long long taken =
                         __hip_atomic_load(a.counter + c * kQueueStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    left = (int64_t)taken < a.patches[c].pend - a.patches[c].pbeg;
+                    const long long left = a.patches[c].pend - a.patches[c].pbeg - (long long)taken;
+                    if (left > most) { most = first ? a.n_patches - k : left; at = c; }
                 }
-                const unsigned long long m = __ballot(left);
-                if (m) {
-                    pick = p + k0 + __builtin_ctzll(m);
-                    pick = pick < a.n_patches ? pick : pick - a.n_patches;
-                }
+                if ((first || (k0 & 960) == 960) && __any(at >= 0)) break;
             }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                const long long l = __shfl_xor(most, off);
+                const int c = __shfl_xor(at, off);
+                const bool more = l > most || (l == most && (unsigned)c < (unsigned)at);
+                most = more ? l : most;
+                at = more ? c : at;
+            }
+            int pick = at;
+            first = false;
             if (lane == 0) s_patch = pick;
         }
         __syncthreads();
