@@ -680,10 +680,10 @@ struct WavePool {
     }
     // a fresh chunk from counter over [qb, qe); false if that queue is drained
     __device__ __forceinline__ bool take(const PathKernelArgs &a, unsigned long long *counter, int64_t qb,
-                                         int64_t qe, int lane) {
+                                         int64_t qe, int lane, int64_t chunk) {
         unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(counter, (unsigned long long)a.pool_chunk);
-        return set(a, qb + (int64_t)uniform_u64(base), a.pool_chunk, qe);
+        if (lane == 0) base = atomicAdd(counter, (unsigned long long)chunk);
+        return set(a, qb + (int64_t)uniform_u64(base), chunk, qe);
     }
     __device__ __forceinline__ int knot_of(const PathKernelArgs &a, int64_t gg) const {
         return gg < ck_end ? ck : find_knot(a, gg);
@@ -734,7 +734,7 @@ struct PathQueues {
             unsigned long long *c = a.counter + q * kQueueStride;
             // (a drained queue is seen without an atomic)
             const unsigned long long taken = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (qb + (int64_t)uniform_u64(taken) < finish(a, q) && pool.take(a, c, qb, finish(a, q), lane)) break;
+            if (qb + (int64_t)uniform_u64(taken) < finish(a, q) && pool.take(a, c, qb, finish(a, q), lane, a.pool_chunk)) break;
             if (++tried >= a.n_queues) drained = true;
             else q = q + 1 == a.n_queues ? 0 : q + 1;
         }
@@ -979,7 +979,14 @@ path_kernel_tiled(PathKernelArgs a) {
                 const unsigned long long m = __ballot(need);
                 if (m) {
                     if (pool.next >= pool.end && !drained)
-                        if (!pool.take(a, a.counter + p * kQueueStride, pd.pbeg, pd.pend, lane)) drained = true;
+                        {
+                        // a wave's first paths of a patch and the patch's last 24 chunks go out 64 at a
+                        // time: a wave that holds four paths a lane when the patch is drained keeps
+                        // its work-group waiting (tabulated problem, 1.4 10^6 paths: FP64 6.3 -> 5.6 ms,
+                        // FP32 4.9 -> 4.1; an FP32 disc 2.5 -> 2.0; 3437 x 100000 paths FP64 549 -> 538)
+                        const int64_t chunk = pool.end > pd.pbeg && pd.pend - pool.end > 24 * a.pool_chunk ? a.pool_chunk : 64;
+                        if (!pool.take(a, a.counter + p * kQueueStride, pd.pbeg, pd.pend, lane, chunk)) drained = true;
+                    }
                     pool.hand_out(a, w, need, m, drained, done, lane);
                 }
             }
