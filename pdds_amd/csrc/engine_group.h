@@ -189,13 +189,17 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
     R pd = 0, pLt = 0, qx = 0, qy = 0, qd = 0, qlt = 0, d = p.rd, lt = p.lt;
     int pk = 0, qk = 0, kind = p.rk;
     R E = 0;
-    // constant motion: the root of the lane's own Lepingle step for a side in x and one in y (outside
-    // the rectangle's corners a normal has one component, +-1), which so leaves the serial part
-    // (5 points x 500 paths 2.34 -> 2.13 ms, 20 x 20000 18.9 -> 17.6)
+    // constant motion: the root of the lane's own Lepingle step for a side in x and one in y (a side's
+    // normal has one component, +-1), which so leaves the serial part (5 points x 500 paths
+    // 2.34 -> 2.13 ms, 20 x 20000 18.9 -> 17.6).  A corner's has two, and its root is formed in place.  A
+    // path steps from a corner only where it starts past one, or was put back onto one (below) and
+    // the projection rounded outwards: corner says whether a path of the wave may do so.
     R Sx = 0, Sy = 0;
+    bool corner = false;
     if constexpr (REFL) {
         E = draw_exponential<R>(st_l, p.g - p.poff, a.seed, p.strm, p.kid);
         if constexpr (!VAR) {
+            corner = __any(p.active && kind > 3);
             const R hE = ((R)2.0 * h) * E;
             Sx = RM<R>::sqrt((co.s00 * co.s00) * hE + dx[0] * dx[0]);
             Sy = RM<R>::sqrt((co.s11 * co.s11) * hE + dy[0] * dy[0]);
@@ -215,13 +219,17 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
             group_normal<R>(kind, nx, ny);
             const bool lep = refl_kind(kind, p.rmask) && (a.pp.rho <= 0.0 || d > -(R)a.pp.rho);
             R mx, my;
+            auto push = [&](R j0, R j1) {
+                const R ga = nx * co.s00, gb = ny * co.s11;
+                const R uc = (ga * j0 + gb * j1) + (nx * co.b0 + ny * co.b1) * h;
+                const R M = (R)0.5 * (uc + RM<R>::sqrt((ga * ga + gb * gb) * (((R)2.0 * h) * group_bcast<G, K>(E)) + uc * uc));
+                return RM<R>::fmax((R)0, M + d);
+            };
             if constexpr (VAR) {
                 const R j0 = group_bcast<G, K>(i0[0]), j1 = group_bcast<G, K>(i1[0]);
                 if (__any(lep)) {
-                    const R ga = nx * co.s00, gb = ny * co.s11;
-                    const R uc = (ga * j0 + gb * j1) + (nx * co.b0 + ny * co.b1) * h;
-                    const R M = (R)0.5 * (uc + RM<R>::sqrt((ga * ga + gb * gb) * (((R)2.0 * h) * group_bcast<G, K>(E)) + uc * uc));
-                    L = lep ? RM<R>::fmax((R)0, M + d) : (R)0;
+                    const R Lp = push(j0, j1);
+                    L = lep ? Lp : (R)0;
                 }
                 mx = em_move(co.b0, h, co.s00, j0);
                 my = em_move(co.b1, h, co.s11, j1);
@@ -232,6 +240,11 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
                 const R S = nx != (R)0 ? sx : sy;
                 const R M = (R)0.5 * (nx * mx + ny * my + S);
                 L = lep ? RM<R>::fmax((R)0, M + d) : (R)0;
+                if (__builtin_expect(corner, 0)) {
+                    const R Lp = push(group_bcast<G, K>(i0[0]), group_bcast<G, K>(i1[0]));
+                    L = lep && kind > 3 ? Lp : L;
+                    corner = false;
+                }
             }
             pd = me ? d : pd;
             pk = me ? kind : pk;
@@ -252,6 +265,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
                 const R d2 = group_dist<R>(p.rect, x, y, ex, ey, k2);
                 d = past ? d2 : d;
                 kind = past ? k2 : kind;
+                if constexpr (!VAR) corner = __any(past && kind > 3);
             }
             if constexpr (VAR) pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co);
             qx = me ? x : qx;
