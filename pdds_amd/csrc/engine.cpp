@@ -460,8 +460,10 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         if ((st = dbuf(e, B_PART, (size_t)std::max<int64_t>(part, 1) * sizeof(double), &p))) return st; dpart = (double *)p;
         if ((st = dbuf(e, B_KSTAT, (size_t)nk * sizeof(KnotStat), &p))) return st; dks = (KnotStat *)p;
         // patches of the batch: runs of equal tile among the ordered knots
+        // (a pass whose second step finds no lane left on a path still reads 4 texels of a tile for its idle
+        // lanes, PDE_TABLE and discs in FP32: the launch holds as many where no patch has a tile)
         std::vector<PatchDesc> patches;
-        size_t lds_bytes = 0;
+        size_t lds_bytes = 4 * sizeof(float4);
         if (tiled) {
             int64_t poff = 0;
             for (int q = 0; q < nk; ++q) {

@@ -1,0 +1,49 @@
+"""Tiled launches in which no stencil's tile fits in LDS: every patch reads its tables from global
+memory, also on a pass whose last paths stop in its first step (the FP32 kernels of two steps a
+pass).  Results are those of the persistent kernel, bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+SW, NE = (-1.0, -1.0), (1.0, 1.0)
+
+
+@pytest.fixture(scope="module")
+def eng():
+    from pdds_amd.engine import Engine
+    e = Engine(0)
+    yield e
+    e.close()
+
+
+def _equal(eng, mesh, problem, counts, **run):
+    from pdds_amd.engine import default_run
+    a, b = (eng.assemble(mesh, problem, default_run(lut_lds=lds, **run), 0, paths_per_knot=counts) for lds in (1, 0))
+    for k in ("G", "Gvar", "B", "BB"):
+        assert np.array_equal(a[k], b[k]), k
+    for k in ("path_steps", "exits", "paths"):
+        assert a["counters"][k] == b["counters"][k], k
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_table_without_tiles(eng, precision):
+    from pdds_amd.engine import Mesh
+    from pdds_amd.workloads import relative_fac, table_problem
+    # a segment's stencil covers 300 x 150 texels of 32 bytes
+    m = Mesh(SW, NE, 4, 8, relative_fac(SW, NE, 4, 8, 0.8))
+    counts = np.where(m.on_boundary, 1, 6000).astype(np.int64)
+    counts[70] = 5437
+    print("table 600", precision, flush=True)
+    _equal(eng, m, table_problem(eng, 600, SW + NE), counts, h=2e-3, seed=9, precision=precision)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_disc_without_tiles(eng, precision):
+    from pdds_amd.engine import Mesh, bvp
+    from pdds_amd.workloads import varcoef_lut
+    # a sector's box covers at least 150 x 150 texels of 16 bytes
+    m = Mesh.disc(1.0, 3, 8, 11, 6, 12, 1.0)
+    counts = np.where(m.on_boundary, 0, 700).astype(np.int64)
+    counts[5] = 321
+    print("disc 1024", precision, flush=True)
+    _equal(eng, m, bvp("varcoef_lut", lut=varcoef_lut(eng, 1024, SW + NE)), counts, h=1e-3, seed=4, precision=precision)
