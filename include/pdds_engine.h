@@ -201,7 +201,9 @@ typedef struct {
     double reduce_ms;       /* device time of the finalize kernel */
     double total_ms;        /* host wall time of the call */
     int64_t work_items;
-    int32_t grid_wgs, wg_size, item_paths, sub_batch;
+    int32_t grid_wgs, wg_size;  /* work-groups of the largest path launch; threads of a work-group of the
+                               path kernel that ran (of the call's first launch) */
+    int32_t item_paths, sub_batch;
 } pdds_counters;
 
 /* ---- per-path records (MCinCUDA shape) ----

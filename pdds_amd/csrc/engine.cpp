@@ -330,7 +330,6 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             rank[i] = it->second;
         }
         std::stable_sort(ord.begin(), ord.end(), [&](size_t a, size_t b) { return rank[a] < rank[b]; });
-        out.wg = path_tiled_wg(prob->pde, r->precision, r->step, geom);
     }
     // knots are processed in batches whose exit records fit the record budget
     const int64_t rec_bytes = (int64_t)sizeof(ExitRec);
@@ -517,11 +516,12 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         auto launched = [&](hipError_t lr) {
             return lr == hipSuccess ? PDDS_OK : fail(e, PDDS_ERR_DEVICE, std::string("path launch: ") + hipGetErrorString(lr));
         };
-        const int kwg = lanes ? 256 : wg;   // work-group of the path kernel (not the tiled one)
+        const int twg = path_tiled_wg(prob->pde, r->precision, r->step, geom);
+        const int kwg = use_tiles ? twg : lanes ? 256 : wg;   // work-group of the path kernel
+        if (k0 == 0) out.wg = kwg;
         int grid;
         pa.n_queues = 1;
         if (use_tiles) {
-            const int twg = path_tiled_wg(prob->pde, r->precision, r->step, geom);
             grid = r->grid_wgs > 0 ? r->grid_wgs
                                    : (int)std::max<int64_t>(1, std::min<int64_t>(e->n_cu, (tot + 8 * twg - 1) / (8 * twg)));
         } else if (persistent) {
