@@ -301,8 +301,10 @@ pdds_status pdds_solve_adaptive(pdds_engine *e, const pdds_mesh *m, const pdds_p
    Times trial assemblies of a sample of the mesh's knots (a contiguous run of at most max_knots
    Monte Carlo knots from the middle of the mesh, sample_paths paths each, so that the sample keeps
    the mesh's stencil and LUT-tile structure) over the launch shapes that do not change results
-   -- LDS tiling on or off, work-group size, work-groups per CU, paths per lane -- and writes into
-   *best the base run with the fastest shape (path-steps per second of the whole assembly). */
+   -- LDS tiling on or off, work-group size, work-groups per CU, paths per lane, of these the ones
+   that the problem's kernel reads -- and writes into *best the base run with the fastest shape
+   (path-steps per second of the whole assembly).  The sample runs the kernel of the largest
+   launches, also where it is small enough for another. */
 typedef struct {
     int64_t sample_paths;   /* paths per sampled knot (0: 16384) */
     int32_t max_knots;      /* sampled knots (0: 512) */

@@ -6,6 +6,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <string>
@@ -271,9 +272,31 @@ static int path_grid(int n_cu, int per_cu, int wg, int64_t slots, int64_t tot, i
     return grid;
 }
 
+// Whether a launch of that many paths takes the LDS-tiled kernel, unless the group kernel takes it:
+// coefficient LUT with a fifth-field quad plane, or the tabulated problem in launches that fill the
+// tiled grid, in rectangles (not its FP32 VR and VR + CV steps, whose rounding follows the
+// persistent kernel's code); not with reflecting sides, whose steps run in the persistent and
+// plain kernels.
+static bool takes_tiles(const pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const PdeParams &pp, int geom,
+                        int64_t paths) {
+    if (r->plain != 0 || r->lut_lds == 0 || pp.refl != 0) return false;
+    if (prob->pde == PDDS_PDE_VARCOEF_LUT) return pp.lut.nf == 5;
+    return prob->pde == PDDS_PDE_TABLE && geom == GeomRect &&
+           (r->precision == PDDS_FP64 || pp.step == STEP_CV || pp.step == STEP_PLAIN) &&
+           paths >= kTableTileLane * e->n_cu * (int64_t)path_tiled_wg(prob->pde, r->precision, r->step, geom);
+}
+
+// Lanes to a path of such a launch in the group kernel; 0: another kernel takes it.
+static int launch_lanes(const pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const PdeParams &pp, int geom,
+                        int64_t paths) {
+    if (r->plain != 0 || geom != GeomRect || pp.step != STEP_CV) return 0;
+    return group_lanes(prob->pde, r->precision, pp.refl != 0, e->n_cu, paths);
+}
+
 pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const double glob[4],
                          const std::vector<const DevTables *> &tabs, const std::vector<AsmKnot> &knots,
-                         int64_t n_vals, double *G_host, double *Gvar_host, AsmOut &out, const double *W_host) {
+                         int64_t n_vals, double *G_host, double *Gvar_host, AsmOut &out, const double *W_host,
+                         int64_t as_paths) {
     auto host_sd = [&](const AsmKnot &k) -> const StencilDesc & { return tabs[k.table]->host_sten[k.stencil]; };
     PdeParams pp;
     pdds_status st = make_params(e, prob, r, pp);
@@ -294,23 +317,17 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
     for (const DevTables *t : tabs)
         if (t->geom != geom) return fail(e, PDDS_ERR_INVALID, "one assembly mixes stencil geometries");
     if (pp.refl && geom != GeomRect) return fail(e, PDDS_ERR_UNSUPPORTED, "reflecting sides need rectangular stencils");
-    // LDS-tiled form (coefficient LUT with a fifth-field quad plane, persistent launch): knots
-    // are grouped into patches of equal tile, tiles that fit in LDS first, in first-seen order;
-    // not with reflecting sides, whose steps run in the persistent and plain kernels
+    // LDS-tiled form: knots are grouped into patches of equal tile, tiles that fit in LDS first, in
+    // first-seen order
     int64_t all_paths = 0;
     for (const AsmKnot &k : knots) all_paths += k.n;
-    const bool table = prob->pde == PDDS_PDE_TABLE;
     // the tabulated problem's tile holds its fields' two planes, and with a VR + CV step that of mu
-    // and F where its grid is the same and there is room; launches that fill the tiled grid, in
-    // rectangles (not the FP32 VR and VR + CV steps, whose rounding follows the persistent kernel's code)
+    // and F where its grid is the same and there is room
     const LutView &la = pp.lut, &lv = pp.vlut;
-    const int tile_planes = !table ? 1 : pp.step == STEP_VRCV && la.nx == lv.nx && la.ny == lv.ny && la.px == lv.px &&
-                                                 la.ox == lv.ox && la.oy == lv.oy && la.sx == lv.sx && la.sy == lv.sy ? 3 : 2;
-    const bool tiled =
-        persistent && r->lut_lds != 0 && pp.refl == 0 &&
-        ((prob->pde == PDDS_PDE_VARCOEF_LUT && pp.lut.nf == 5) ||
-         (table && geom == GeomRect && (r->precision == PDDS_FP64 || pp.step == STEP_CV || pp.step == STEP_PLAIN) &&
-          all_paths >= kTableTileLane * e->n_cu * (int64_t)path_tiled_wg(prob->pde, r->precision, r->step, geom)));
+    const int tile_planes = prob->pde != PDDS_PDE_TABLE ? 1
+                            : pp.step == STEP_VRCV && la.nx == lv.nx && la.ny == lv.ny && la.px == lv.px && la.ox == lv.ox &&
+                                      la.oy == lv.oy && la.sx == lv.sx && la.sy == lv.sy ? 3 : 2;
+    const bool tiled = takes_tiles(e, prob, r, pp, geom, std::max(all_paths, as_paths));
     const size_t tile_cap = e->lds_max > 1024 ? e->lds_max - 1024 : 0;
     std::vector<size_t> ord(knots.size());
     for (size_t i = 0; i < ord.size(); ++i) ord[i] = i;
@@ -505,8 +522,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         pa.patches = dpatch;
         pa.n_patches = (int32_t)patches.size();
         const bool fp64 = r->precision == PDDS_FP64;
-        const int lanes = persistent && geom == GeomRect && pp.step == STEP_CV
-                              ? group_lanes(prob->pde, r->precision, pp.refl != 0, e->n_cu, tot) : 0;
+        const int lanes = launch_lanes(e, prob, r, pp, geom, std::max(tot, as_paths));
         const bool use_tiles = tiled && !lanes;
         auto launch = [&](const PathLaunch &l) -> hipError_t {
             if (lanes) return fp64 ? launch_group_f64(prob->pde, mixed, lanes, l, pa) : launch_group_f32(prob->pde, mixed, lanes, l, pa);
@@ -1321,15 +1337,24 @@ pdds_status pdds_autotune(pdds_engine *e, const pdds_mesh *m, const pdds_problem
         r.plain = 0;
         cands.push_back(r);
     }
-    // LDS-tiled shapes: work-groups per CU, paths per lane and the tile's row pitch
-    const bool can_tile = p->pde == PDDS_PDE_VARCOEF_LUT && pp.lut.nf == 5;
-    if (can_tile)
-        for (int pad : {0, 1, 2, 3})
-            for (int g : {1, 2})
-                for (int ppl : {1, 2, 4, 8}) add(1, 0, g * e->n_cu, ppl, pad);
-    for (int wg : {64, 128, 256})
+    // shapes of the kernel that the largest launches take, which the sample runs whatever its own
+    // size; shapes differ in fields that this kernel reads
+    const int64_t large = std::numeric_limits<int64_t>::max();
+    pdds_run tile_run = cands[0];
+    tile_run.lut_lds = 1;
+    if (launch_lanes(e, p, &cands[0], pp, M.geom, large) > 0) {
         for (int g : {1, 2, 4, 8})
-            for (int ppl : {1, 4, 16}) add(0, wg, g * e->n_cu * 256 / wg, ppl, 0);
+            for (int ppl : {1, 4, 16}) add(base->lut_lds, base->wg_size, g * e->n_cu, ppl, base->lut_pad);
+    } else {
+        // LDS-tiled shapes: work-groups per CU, paths per lane and the tile's row pitch
+        if (takes_tiles(e, p, &tile_run, pp, M.geom, large))
+            for (int pad : {0, 1, 2, 3})
+                for (int g : {1, 2})
+                    for (int ppl : {1, 2, 4, 8}) add(1, 0, g * e->n_cu, ppl, pad);
+        for (int wg : {64, 128, 256})
+            for (int g : {1, 2, 4, 8})
+                for (int ppl : {1, 4, 16}) add(0, wg, g * e->n_cu * 256 / wg, ppl, 0);
+    }
     double best_rate = -1.0, base_rate = 0.0;
     size_t best_i = 0;
     for (size_t i = 0; i < cands.size(); ++i) {
@@ -1338,7 +1363,7 @@ pdds_status pdds_autotune(pdds_engine *e, const pdds_mesh *m, const pdds_problem
         for (int rep_i = 0; rep_i <= cfg.reps; ++rep_i) {
             AsmOut o;
             const double ts = now_ms();
-            if ((st = run_assembly(e, p, &cands[i], M.glob, {T}, knots, M.row_ptr.back(), nullptr, nullptr, o)))
+            if ((st = run_assembly(e, p, &cands[i], M.glob, {T}, knots, M.row_ptr.back(), nullptr, nullptr, o, nullptr, large)))
                 return st;
             const double dt = now_ms() - ts;
             if (rep_i == 0) continue;   // warm-up

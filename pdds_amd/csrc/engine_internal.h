@@ -150,10 +150,11 @@ pdds_status build_tables(pdds_engine *e, const std::vector<StencilDesc> &sten, c
                          const std::vector<double> &ipsi, DevTables &T);
 // W_host (optional, n_vals values): per CSR value the reference interface value of its column's
 // knot; the knots' equation means and variances then land in out.kstats[].Rm / Rv
+// as_paths: the path kernel is that of launches of at least so many paths (the autotuner's samples)
 pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const double glob[4],
                          const std::vector<const DevTables *> &tabs, const std::vector<AsmKnot> &knots,
                          int64_t n_vals, double *G_host, double *Gvar_host, AsmOut &out,
-                         const double *W_host = nullptr);
+                         const double *W_host = nullptr, int64_t as_paths = 0);
 void mesh_tables(const Mesh &m, int quirk, std::vector<StencilDesc> &sten, std::vector<double> &entx,
                  std::vector<double> &enty, std::vector<int8_t> &ents, std::vector<double> &entic2,
                  std::vector<int32_t> &e1,
