@@ -329,10 +329,12 @@ pdds_status pdds_point_eval(pdds_engine *e, const pdds_problem *p, const pdds_ru
    HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  Arguments, results
    and errors are those of pdds_point_eval (bit-identical results), but every device buffer the
    call needs (exit records, work items, reduction partials, statistics, queue counters and the
-   rectangle's stencil table) is taken from one fixed array of PDDS_NOALLOC_SCRATCH_BYTES that
-   each device holds from the library's load until the process ends; the call makes no hipMalloc
-   or hipFree.  It returns PDDS_ERR_FULL, before any device work, when its buffers would exceed
-   that array: about 32 bytes per path (some 2e6 paths per call in total).  Every call on one
+   rectangle's stencil table) is taken from one fixed array that each device holds from the
+   library's load until the process ends: PDDS_NOALLOC_SCRATCH_BYTES, which a call is counted
+   against, and 8 MiB for launch tables that are not counted.  The call makes no hipMalloc
+   or hipFree.  It returns PDDS_ERR_FULL when its buffers would exceed the counted bytes, before any
+   device work unless item_paths makes more than 17 work items of a point: about 32 bytes per path
+   (some 2e6 paths per call in total).  Every call on one
    device shares the array, which keeps the last call's contents (what must start at zero is
    cleared by each call); overlapping calls on one device would race, so the library serialises
    them with a per-device lock (they wait for each other, also across engines). */

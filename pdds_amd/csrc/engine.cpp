@@ -39,8 +39,18 @@ pdds_status fail(pdds_engine *e, pdds_status s, const std::string &msg) {
 // that address is ever handed to kernels or copies.
 // ---------------------------------------------------------------------------
 // Beside the bytes that callers may plan with, room for what a call's launch-side tables hold beyond
-// kKnotDescQuota (at most some 40,000 knots fit a call).
+// the quotas: of each knot its descriptor's copies and two entries of the block table, of each item
+// its descriptor's span, and the tables' alignment, queue counters and least block table.  A call has
+// at most as many knots as its estimate admits (point_eval_locked) and items of a path each as fit.
 static constexpr size_t kScratchSpare = (size_t)8 << 20;
+static constexpr int64_t kScratchKnotBytes =
+    kKnotDescQuota + (int64_t)sizeof(KnotStat) + 16 + 17 * (kItemDescQuota + (int64_t)sizeof(ItemStat));
+static_assert(PDDS_NOALLOC_SCRATCH_BYTES / (kScratchKnotBytes + (int64_t)sizeof(ExitRec)) *
+                          ((int64_t)sizeof(KnotDesc) - kKnotDescQuota + 2 * (int64_t)sizeof(int32_t)) +
+                      PDDS_NOALLOC_SCRATCH_BYTES / (kItemDescQuota + (int64_t)(sizeof(ItemStat) + sizeof(ExitRec))) *
+                          ((int64_t)sizeof(ItemDesc) - kItemDescQuota) +
+                      ((int64_t)64 << 10) <= (int64_t)kScratchSpare,
+              "the spare holds what a call takes beyond the quotas");
 static __device__ __align__(256) unsigned char scratch[PDDS_NOALLOC_SCRATCH_BYTES + kScratchSpare];
 
 namespace {
@@ -68,16 +78,19 @@ static hipError_t noalloc_scratch_of(int device, char **out) {
 
 // device buffer for slot i: grow-only and kept by the engine, or, while the engine has an arena
 // set, the next piece of the arena
-pdds_status dbuf(pdds_engine *e, int slot, size_t bytes, void **out) {
+pdds_status dbuf(pdds_engine *e, int slot, size_t bytes, void **out, size_t quota) {
     if (bytes == 0) bytes = 8;
     if (e->arena) {
         Arena &a = *e->arena;
-        const size_t off = (a.used + 255) & ~(size_t)255;
-        if (off > a.cap || bytes > a.cap - off)
+        if (quota == kAllBytes) quota = bytes;
+        const size_t limit = (size_t)PDDS_NOALLOC_SCRATCH_BYTES;
+        const size_t off = (a.used + 255) & ~(size_t)255, qoff = quota > 0 ? (a.quota + 255) & ~(size_t)255 : a.quota;
+        if (qoff > limit || quota > limit - qoff || off > a.cap || bytes > a.cap - off)
             return fail(e, PDDS_ERR_FULL, "the call needs more device memory than the " +
-                                              std::to_string(a.cap >> 20) + " MiB no-allocation scratch");
+                                              std::to_string(limit >> 20) + " MiB no-allocation scratch");
         *out = a.base + off;
         a.used = off + bytes;
+        a.quota = qoff + quota;
         return PDDS_OK;
     }
     DevBuf &b = e->bufs[slot];
@@ -463,9 +476,9 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
             kblk[b] = (int32_t)q;
         }
         KnotDesc *dk; ItemDesc *dit; int32_t *dkblk;
-        if ((st = upload(e, B_KNOTS, kd, &dk))) return st;
-        if ((st = upload(e, B_KBLK, kblk, &dkblk))) return st;
-        if ((st = upload(e, B_ITEMS, items, &dit))) return st;
+        if ((st = upload(e, B_KNOTS, kd, &dk, kKnotDescQuota))) return st;
+        if ((st = upload(e, B_KBLK, kblk, &dkblk, 0))) return st;
+        if ((st = upload(e, B_ITEMS, items, &dit, kItemDescQuota))) return st;
         Records rec;
         if ((st = dbuf(e, B_REC, (size_t)tot * sizeof(ExitRec), &p))) return st; rec.r = (ExitRec *)p;
         if ((st = dbuf(e, B_KACC, (size_t)nk * 2 * sizeof(unsigned long long), &p))) return st;
@@ -507,7 +520,7 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
         const size_t nctr = std::max<size_t>(kMaxQueues, patches.size());
         PatchDesc *dpatch = nullptr;
         if (tiled && (st = upload(e, B_PATCH, patches, &dpatch))) return st;
-        if ((st = dbuf(e, B_COUNTER, nctr * kQueueStride * sizeof(unsigned long long), &p))) return st;
+        if ((st = dbuf(e, B_COUNTER, nctr * kQueueStride * sizeof(unsigned long long), &p, nctr * sizeof(unsigned long long)))) return st;
         dctr = (unsigned long long *)p;
         HIPCHK(launch_fill_u64(dctr, (int64_t)nctr * kQueueStride, 0ULL, e->stream));
         // path kernel
@@ -1471,10 +1484,7 @@ static pdds_status point_eval_locked(pdds_engine *e, const pdds_problem *p, cons
         // exit records, and per point its descriptor, statistics, step counters and work items (at
         // most 17 of them, P >= N / 16, each with its descriptor and statistics), with room for
         // alignment
-        const int64_t need = paths * (int64_t)sizeof(ExitRec) +
-                             (int64_t)knots.size() * (int64_t)(kKnotDescQuota + sizeof(KnotStat) + 16 +
-                                                                17 * (kItemDescQuota + sizeof(ItemStat))) +
-                             ((int64_t)1 << 16);
+        const int64_t need = paths * (int64_t)sizeof(ExitRec) + (int64_t)knots.size() * kScratchKnotBytes + ((int64_t)1 << 16);
         if (need > (int64_t)PDDS_NOALLOC_SCRATCH_BYTES)
             return fail(e, PDDS_ERR_FULL, std::to_string(paths) + " paths at " + std::to_string(knots.size()) +
                                               " points need about " + std::to_string(need >> 20) +

@@ -43,9 +43,12 @@ struct DevTables {
 
 // A fixed region of device memory handed out front to back (256-byte aligned): while an engine
 // has one set, dbuf takes every buffer from it instead of allocating.
+// A call is refused by `quota`, the bytes that it takes as counted towards PDDS_NOALLOC_SCRATCH_BYTES
+// (kKnotDescQuota, kItemDescQuota; launch-side tables not at all); the region holds what it takes
+// beyond them (kScratchSpare).
 struct Arena {
     char *base = nullptr;
-    size_t cap = 0, used = 0;
+    size_t cap = 0, used = 0, quota = 0;
 };
 
 struct pdds_engine {
@@ -102,13 +105,14 @@ pdds_status fail(pdds_engine *e, pdds_status s, const std::string &msg);
             return fail(e, PDDS_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(_r));      \
     } while (0)
 
-// grow-only device buffer for slot i
-pdds_status dbuf(pdds_engine *e, int slot, size_t bytes, void **out);
+// grow-only device buffer for slot i; quota: what an arena counts of its bytes (all of them)
+constexpr size_t kAllBytes = ~(size_t)0;
+pdds_status dbuf(pdds_engine *e, int slot, size_t bytes, void **out, size_t quota = kAllBytes);
 
 template <class T>
-pdds_status upload(pdds_engine *e, int slot, const std::vector<T> &v, T **out) {
+pdds_status upload(pdds_engine *e, int slot, const std::vector<T> &v, T **out, size_t quota_each = sizeof(T)) {
     void *p;
-    pdds_status s = dbuf(e, slot, v.size() * sizeof(T), &p);
+    pdds_status s = dbuf(e, slot, v.size() * sizeof(T), &p, v.size() * quota_each);
     if (s) return s;
     if (!v.empty()) HIPCHK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, e->stream));
     *out = (T *)p;
