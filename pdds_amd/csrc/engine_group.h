@@ -93,7 +93,7 @@ template <class R> struct GroupState {
     uint32_t strm, st, poff, kid, g;
     int gmask;
     bool active;
-    KnotSteps ks;
+    LaneSteps ks;
     R s00, s11, b0, b1, c;  // varying motion: the coefficients at X that move it (and Y)
     R rd, lt;               // reflecting sides: distance of the nearest side at X, pending local time
     int rk, rmask;          //   that side, and the reflecting sides of the domain

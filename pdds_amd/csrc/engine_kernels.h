@@ -24,6 +24,7 @@
 //    items of each knot in item order.  Every sum has a fixed order: results do
 //    not depend on scheduling.
 #pragma once
+#include <type_traits>
 #include "pdds_pde.h"
 #include "engine_types.h"
 
@@ -444,13 +445,18 @@ __device__ __forceinline__ void write_exit(const PathKernelArgs &a, uint32_t g, 
 
 // Steps and step-cap stops of stopped paths of one knot, summed in a lane's registers and added
 // to the knot's counters (Records::kacc) when the lane moves to another knot and when it ends.
-struct KnotSteps {
+struct LaneSteps {
     int k;                    // knot of the sums
     unsigned long long st;    // steps
     uint32_t cap;             // paths stopped by the step cap while inside
+    static constexpr int words = 0;
 
-    __device__ __forceinline__ void init() { k = -1; st = 0ULL; cap = 0u; }
-    __device__ __forceinline__ void flush(const PathKernelArgs &a) {
+    __device__ __forceinline__ void init(unsigned long long * = nullptr, int = 0) { k = -1; st = 0ULL; cap = 0u; }
+    __device__ __forceinline__ void add(const PathKernelArgs &, uint32_t steps, bool capped) {
+        st += steps;
+        cap += capped ? 1u : 0u;
+    }
+    __device__ __forceinline__ void flush(const PathKernelArgs &a, int = 0) {
         if (st) {
             atomicAdd(a.rec.kacc + 2 * (int64_t)k, st);
             if (cap) atomicAdd(a.rec.kacc + 2 * (int64_t)k + 1, (unsigned long long)cap);
@@ -464,6 +470,68 @@ struct KnotSteps {
         k = kn;
     }
 };
+
+// Steps and step-cap stops of a wave's stopped paths, summed in its own words of LDS for the two
+// knots that its pool came to last, and added to their counters (Records::kacc) one atomic to a
+// wave and knot: when the pool comes to a third knot, and at the end.  A path of another knot (a long one, or
+// of knots of a few paths) adds its own.  Atomics of one address wait for each other and the loads
+// of a lane's next knot wait for them: with a sum per lane, 64 to a wave and knot, 2 10^6 FP32
+// paths of 16 points (plain step, some 150 steps each) took 4.7 ms, and take 1.8 so.  The kernels that
+// read a table, and the group kernel, keep LaneSteps: they wait for their reads more than for these atomics (2 10^6
+// paths of 16 or 2000 points, h = 1e-3, LUT or table: 28 to 37 ms either way), and with the wave's words the
+// compiler orders the table's FP32 plain step worse (2000 points: 39.8 ms, 34.7 so).
+struct KnotSteps {
+    static constexpr int words = 4;    // of LDS to a wave: steps and cap stops of two knots
+    unsigned long long *acc;     // the wave's words
+    int k;                       // the lane's knot
+    int kn, ko, sn;              // wave-uniform: the newer and the older knot, the newer one's slot
+
+    __device__ __forceinline__ void init(unsigned long long *lds, int lane) {
+        acc = lds + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * words;
+        if (lane < words) acc[lane] = 0ULL;
+        k = kn = ko = -1;
+        sn = 0;
+    }
+    __device__ __forceinline__ void add_global(const PathKernelArgs &a, int knot, unsigned long long st, unsigned long long cap) const {
+        if (st) atomicAdd(a.rec.kacc + 2 * (int64_t)knot, st);
+        if (cap) atomicAdd(a.rec.kacc + 2 * (int64_t)knot + 1, cap);
+    }
+    // the sums of one slot into its knot's counters (by the whole wave)
+    __device__ __forceinline__ void flush_slot(const PathKernelArgs &a, int slot, int knot, int lane) {
+        if (lane != 0 || knot < 0) return;
+        unsigned long long *w = acc + 2 * slot;
+        const unsigned long long st = __hip_atomic_exchange(w, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const unsigned long long cap = __hip_atomic_exchange(w + 1, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        add_global(a, knot, st, cap);
+    }
+    // the wave's pool comes to knot kk (wave-uniform; by the whole wave)
+    __device__ __forceinline__ void open(const PathKernelArgs &a, int kk, int lane) {
+        if (kk == kn || kk == ko) return;
+        sn ^= 1;
+        flush_slot(a, sn, ko, lane);
+        ko = kn;
+        kn = kk;
+    }
+    // the lane goes on to paths of knot kk
+    __device__ __forceinline__ void enter(const PathKernelArgs &, int kk) { k = kk; }
+    // a lane's path has stopped
+    __device__ __forceinline__ void add(const PathKernelArgs &a, uint32_t st, bool cap) const {
+        if (k == kn || k == ko) {
+            unsigned long long *w = acc + 2 * (k == kn ? sn : sn ^ 1);
+            (void)__hip_atomic_fetch_add(w, (unsigned long long)st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (cap) (void)__hip_atomic_fetch_add(w + 1, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else {
+            add_global(a, k, st, cap ? 1ULL : 0ULL);
+        }
+    }
+    __device__ __forceinline__ void flush(const PathKernelArgs &a, int lane) {
+        flush_slot(a, sn, kn, lane);
+        flush_slot(a, sn ^ 1, ko, lane);
+    }
+};
+
+template <int PDE>
+using PathSteps = std::conditional_t<PDE == PDE_VARCOEF_LUT || PDE == PDE_TABLE, LaneSteps, KnotSteps>;
 
 // Distance to a stencil's stopping domain: its rectangle, or its annular sector on a disc mesh.
 template <class R, int GEOM>
@@ -506,14 +574,14 @@ struct Walker {
     // local time
     int rmask, rk;
     R rd, rnx, rny, lt;
-    KnotSteps ks;          // the lane's knot, and the steps of its stopped paths not yet added to its counters
+    PathSteps<PDE> ks;     // the lane's knot, and the steps of stopped paths not yet added to their counters
 
-    __device__ __forceinline__ void init() {
+    __device__ __forceinline__ void init(unsigned long long *step_words = nullptr, int lane = 0) {
         // (a lane's first step, with zero coefficients, still takes the normals: they must be finite)
         pn1 = 0; pn2 = 0; s.pn1 = 0; s.pn2 = 0; kid = 0; kstream = 0; gmask = 0; g = 0; poff = 0; k2 = 0; hk = 0; sqhk = 0;
         active = false; fresh = false;
         rmask = 0; rk = 0; rd = 0; rnx = 0; rny = 0; lt = 0;
-        ks.init();
+        ks.init(step_words, lane);
     }
 
     // take path gg of the batch; k is its knot.  A lane's next path is mostly one of the same knot,
@@ -652,8 +720,7 @@ struct Walker {
                 (void)rect_dist<R>(dom, s.x, s.y, ex, ey, tx, ty, kind);
             }
             write_exit<R, PDE, GEOM>(a, g, s, gmask, ex, ey, kind);
-            ks.st += s.st;
-            ks.cap += capped && go ? 1u : 0u;
+            ks.add(a, s.st, capped && go);
             active = false;
         }
         fresh = false;
@@ -661,9 +728,8 @@ struct Walker {
 };
 
 // Wave-private pool of consecutive paths [next, end), taken a.pool_chunk at a time from one queue
-// (one atomic per chunk).  With it, the knot of the pool's first path and
-// where that knot ends, found once per chunk with wave-uniform values; a lane whose path
-// lies past that knot searches for its own.
+// (one atomic per chunk).  With it, the knot of its next path and where that knot ends, wave-uniform
+// values; a lane whose path lies past that knot searches for its own.
 struct WavePool {
     int64_t next = 0, end = 0;
     int ck = 0;
@@ -674,9 +740,20 @@ struct WavePool {
         if (s0 >= qe) return false;
         next = s0;
         end = s0 + n < qe ? s0 + n : qe;
-        ck = find_knot(a, s0);
-        ck_end = ck + 1 < a.n_knots ? a.knots[ck + 1].path_off : a.total;
+        find(a);
         return true;
+    }
+    __device__ __forceinline__ void find(const PathKernelArgs &a) {
+        ck = find_knot(a, next);
+        ck_end = ck + 1 < a.n_knots ? a.knots[ck + 1].path_off : a.total;
+    }
+    // the paths from `next` on are about to be handed out (by the whole wave)
+    template <class STEPS> __device__ __forceinline__ void come_to(const PathKernelArgs &a, STEPS &ks, int lane) {
+        if constexpr (STEPS::words > 0) {
+            if (next >= end) return;
+            if (next >= ck_end) find(a);
+            ks.open(a, __builtin_amdgcn_readfirstlane(ck), lane);
+        }
     }
     // a fresh chunk from counter over [qb, qe); false if that queue is drained
     __device__ __forceinline__ bool take(const PathKernelArgs &a, unsigned long long *counter, int64_t qb,
@@ -695,6 +772,7 @@ struct WavePool {
                                              bool drained, bool &done, int lane) {
         const int64_t avail = end > next ? end - next : 0;
         const int rank = __popcll(m & ((1ULL << lane) - 1ULL));
+        come_to(a, w.ks, lane);
         if (need) {
             if (rank < avail) {
                 const int64_t gg = next + rank;
@@ -755,7 +833,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(path_w
     const int lane = __lane_id();
     const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
     Walker<R, PDE, MIXED, GEOM, FAM, REFL> w;
-    w.init();
+    if constexpr (PathSteps<PDE>::words > 0) {
+        __shared__ unsigned long long step_words[4 * PathSteps<PDE>::words];
+        w.init(step_words, lane);
+    } else {
+        w.init();
+    }
     bool done = false;
     // The wave starts on its XCD's queue, so the paths (and LUT texels) of one XCD's L2
     // stay in one contiguous range of knots; a drained queue sends the wave on to the next.
@@ -777,7 +860,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(path_w
         }
         w.template step<false, false>(a, none, it);
     }
-    w.ks.flush(a);
+    w.ks.flush(a, lane);
 }
 
 // ----------------------------------------------------------------------------
@@ -1001,7 +1084,7 @@ path_kernel_tiled(PathKernelArgs a) {
         }
         __syncthreads();   // every wave is done with this tile
     }
-    w.ks.flush(a);
+    w.ks.flush(a, lane);
 }
 
 // ----------------------------------------------------------------------------

@@ -127,9 +127,9 @@ constexpr int64_t kItemDescQuota = 24;     // of a work item's, in the same esti
 // 32-byte record (a lane stores it with two 16-byte writes when its path stops, so a record
 // reaches memory as one 32-byte piece).  The exit side is not stored for FP64 paths: the
 // reduction classifies the exit point again, with the same test on the same doubles.  Step
-// counts are not stored per path: a lane sums the steps and step-cap stops of its stopped paths
-// in registers and adds them to its knot's counters kacc[2k] (steps) and kacc[2k + 1] (capped)
-// when it moves to a path of another knot and when it ends.
+// counts are not stored per path: a wave sums the steps and step-cap stops of its stopped paths
+// per knot (KnotSteps, LaneSteps) and adds them to the knot's counters kacc[2k] (steps) and
+// kacc[2k + 1] (capped).
 struct alignas(32) ExitRec {
     double x, y, Y, score;
 };

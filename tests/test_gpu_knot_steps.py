@@ -1,0 +1,45 @@
+"""Step and step-cap sums of the persistent path kernel (one lane to a path), which a wave holds for
+the two knots its pool came to last: knots of one path, of fewer than a wave takes at once and of
+many, one after another in one launch; a step cap that stops some paths.  Sums and results are
+the plain kernel's."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+GLOB = np.array([-1.0, -1.0, 1.0, 1.0])
+
+
+@pytest.fixture(scope="module")
+def eng():
+    from pdds_amd.engine import Engine
+    e = Engine(0)
+    yield e
+    e.close()
+
+
+def _counts(kind):
+    rng = np.random.default_rng(5)
+    return {"ones": np.ones(700, dtype=np.int64),
+            "few": rng.integers(1, 9, 3000),
+            "mixed": np.where(rng.random(400) < 0.7, rng.integers(1, 70, 400), rng.integers(2000, 4000, 400)),
+            "one": np.array([150001], dtype=np.int64)}[kind].astype(np.int64)
+
+
+@pytest.mark.parametrize("kind", ["ones", "few", "mixed", "one"])
+# (forms without several lanes to a path: the plain step, and FP32 paths with a reflecting side)
+@pytest.mark.parametrize("precision,pde,step,neumann,cap", [("fp64", "helmholtz", 1, 0, 0), ("fp32", "helmholtz", 1, 0, 0),
+                                                            ("fp64", "varcoef", 1, 0, 30), ("fp32", "varcoef", 1, 0, 30),
+                                                            ("fp32", "monegros", 1, 0, 0), ("fp32", "helmholtz", 0, 8, 0)])
+def test_step_sums_equal_plain(eng, kind, precision, pde, step, neumann, cap):
+    from pdds_amd.engine import bvp, default_run
+    n = _counts(kind)
+    x, y = np.linspace(-0.9, 0.8, len(n)), np.linspace(0.7, -0.6, len(n))
+    prob = bvp(pde, neumann=neumann)
+    run = dict(h=5e-3, seed=3, precision=precision, wg_size=128, step=step, max_steps=cap)
+    print(kind, precision, pde, step, neumann, cap, flush=True)
+    a, b = (eng.point_eval(prob, default_run(plain=p, **run), GLOB, x, y, n) for p in (0, 1))
+    assert a["counters"]["wg_size"] == 128
+    for k in ("path_steps", "paths", "exits", "capped"):
+        assert a["counters"][k] == b["counters"][k], k
+    assert np.array_equal(a["u"], b["u"]) and np.array_equal(a["u_var"], b["u_var"])
+    assert (a["counters"]["capped"] > 0) == (cap > 0)
