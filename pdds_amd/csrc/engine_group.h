@@ -156,6 +156,9 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
     const R beta = REC && p.second ? (R)0 : (R)a.beta;
     const R h = p.h, sqrth = p.sqrth;
     R x = p.x, y = p.y, Y = p.Y, Z = p.Z, xi = p.xi, nzc = p.nzc, nxc = p.nxc;
+    // (an FP64 group without a path reads one texel's lines of a table; with that test the compiler
+    // issues the FP32 reads one by one: 40 points x 30 paths of the LUT 0.7 ms, 1.7 so)
+    const bool live = sizeof(R) == 4 || p.active;
     // normals of the lane's steps, and the moves they make
     R n1[NS], n2[NS];
     const uint32_t st_l = p.st + (uint32_t)(sub * NS);
@@ -170,7 +173,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
     if constexpr (VAR) {
         co.s00 = p.s00; co.s11 = p.s11; co.b0 = p.b0; co.b1 = p.b1; co.c = p.c;
     } else {
-        pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co);   // sigma, b and c are constants
+        pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co, live);   // sigma, b and c are constants
     }
     R i0[NS], i1[NS], dx[NS], dy[NS];
 #pragma unroll
@@ -267,7 +270,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
                 kind = past ? k2 : kind;
                 if constexpr (!VAR) corner = __any(past && kind > 3);
             }
-            if constexpr (VAR) pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co);
+            if constexpr (VAR) pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co, live);
             qx = me ? x : qx;
             qy = me ? y : qy;
             qd = me ? d : qd;
@@ -288,7 +291,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
                     const R dY = co.c * Y * h;
                     Y = Y + dY;
                 }
-                if constexpr (VAR) pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co);
+                if constexpr (VAR) pde_coef_t<PDE, R, false>(x, y, a.pp, none, p.k2, co, live);
             }
         }
         if constexpr (VAR) {
@@ -302,7 +305,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
     R fY[NS], vi[NS], Yb[NS], ex[NS], ey[NS], eY[NS], lz = 0;
     bool stop[NS], cap[NS], go[NS];
     if constexpr (REFL) {
-        pde_coef_t<PDE, R, false>(px, py, a.pp, none, p.k2, co);
+        pde_coef_t<PDE, R, false>(px, py, a.pp, none, p.k2, co, live);
         vi[0] = em_dot(-(co.s11 * co.g1), i1[0], -(co.s00 * co.g0), i0[0]);
         // local time of the step: boundary data at X's projection, the growth factor of Y
         R psi = (R)0, w = (R)0;
@@ -343,7 +346,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
         R tx = px, ty = py, tY = pY;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            pde_coef_t<PDE, R, false>(tx, ty, a.pp, none, p.k2, co);
+            pde_coef_t<PDE, R, false>(tx, ty, a.pp, none, p.k2, co, live);
             const R v0 = -(co.s00 * co.g0);
             const R v1 = -(co.s11 * co.g1);
             vi[s] = em_dot(v1, i1[s], v0, i0[s]);
@@ -365,7 +368,7 @@ __device__ __forceinline__ void group_advance(const PathKernelArgs &a, const OUT
             if constexpr (VAR) {
                 if (s + 1 < NS) {
                     Coef<R> cm;
-                    pde_coef_t<PDE, R, false>(tx, ty, a.pp, none, p.k2, cm);
+                    pde_coef_t<PDE, R, false>(tx, ty, a.pp, none, p.k2, cm, live);
                     s00 = cm.s00; s11 = cm.s11;
                 } else {
                     s00 = qs00; s11 = qs11;

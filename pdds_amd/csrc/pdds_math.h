@@ -701,7 +701,7 @@ PDDS_HD void lut_accum(const LutView &L, const LutTile &T, lds_float4 *tp, bool 
             for (int a = 0; a < 4; ++a) A[a] = tp[b * T.pitch + a];
         } else {
 #pragma unroll
-            for (int a = 0; a < 4; ++a) A[a] = lut_at<float4>(L.a, (r0 + (uint32_t)a) * 16u);
+            for (int a = 0; a < 4; ++a) A[a] = (&lut_at<float4>(L.a, r0 * 16u))[a];
         }
         float row[NA];
 #pragma unroll
@@ -714,7 +714,7 @@ PDDS_HD void lut_accum(const LutView &L, const LutTile &T, lds_float4 *tp, bool 
             if constexpr (NF > 5) {
                 float4 q1;
                 if (SRC == 1 || (SRC == 2 && in)) q1 = tp[T.pb + b * T.pitch + a];
-                else q1 = lut_at<float4>(L.b, (r0 + (uint32_t)a) * 16u);
+                else q1 = (&lut_at<float4>(L.b, r0 * 16u))[a];
                 c[4] = q1.x; c[5] = q1.y; c[6] = q1.z; c[7] = q1.w;
             }
 #pragma unroll
@@ -745,7 +745,6 @@ PDDS_HD void lut_accum(const LutView &L, const LutTile &T, lds_float4 *tp, bool 
 // global loads.
 template <class R, int NF, bool TILED>
 PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF], bool live = true) {
-    (void)live;
     static_assert(NF <= 8, "at most 8 fields per texel");
     R t = (x - (R)L.ox) * (R)L.sx;
     R v = (y - (R)L.oy) * (R)L.sy;
@@ -757,7 +756,8 @@ PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF],
     bspline_wf((float)(v - fj), wy);
     // padded column / row of tap (a=0, b=0): i - 1 + kLutPad >= 0, j - 1 + kLutPad >= 0
     const int pc = (int)fi + (kLutPad - 1), pr = (int)fj + (kLutPad - 1);
-    const uint32_t t0 = (uint32_t)pr * (uint32_t)L.px + (uint32_t)pc;
+    // (lanes whose values nobody uses read one texel's lines: a gather costs about a cache line a cycle)
+    const uint32_t t0 = live ? (uint32_t)pr * (uint32_t)L.px + (uint32_t)pc : 0u;
     float acc[NF];
     if constexpr (TILED) {
         const int lc = pc - T.c0, lr = pr - T.r0;
@@ -777,9 +777,9 @@ PDDS_HD void lut_eval_t(const LutView &L, const LutTile &T, R x, R y, R out[NF],
 }
 
 template <class R, int NF>
-PDDS_HD void lut_eval(const LutView &L, R x, R y, R out[NF]) {
+PDDS_HD void lut_eval(const LutView &L, R x, R y, R out[NF], bool live = true) {
     const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
-    lut_eval_t<R, NF, false>(L, none, x, y, out);
+    lut_eval_t<R, NF, false>(L, none, x, y, out, live);
 }
 
 }  // namespace pdds

@@ -149,10 +149,10 @@ PDDS_HD void pde_coef_t(R x, R y, const PdeParams &P, const LutTile &T, R k2, Co
                     V.lds += T.pv;
                     lut_eval_t<R, 4, true>(P.vlut, V, x, y, w, live);
                 } else {
-                    lut_eval<R, 4>(P.vlut, x, y, w);
+                    lut_eval<R, 4>(P.vlut, x, y, w, live);
                 }
             } else {
-                lut_eval<R, 4>(P.vlut, x, y, w);
+                lut_eval<R, 4>(P.vlut, x, y, w, live);
             }
             co.m0 = w[0]; co.m1 = w[1]; co.F0 = w[2]; co.F1 = w[3];
         }
