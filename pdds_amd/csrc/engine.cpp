@@ -285,18 +285,46 @@ static int path_grid(int n_cu, int per_cu, int wg, int64_t slots, int64_t tot, i
     return grid;
 }
 
-// Whether a launch of that many paths takes the LDS-tiled kernel, unless the group kernel takes it:
-// coefficient LUT with a fifth-field quad plane, or the tabulated problem in launches that fill the
-// tiled grid, in rectangles (not its FP32 VR and VR + CV steps, whose rounding follows the
-// persistent kernel's code); not with reflecting sides, whose steps run in the persistent and
-// plain kernels.
-static bool takes_tiles(const pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const PdeParams &pp, int geom,
-                        int64_t paths) {
-    if (r->plain != 0 || r->lut_lds == 0 || pp.refl != 0) return false;
-    if (prob->pde == PDDS_PDE_VARCOEF_LUT) return pp.lut.nf == 5;
-    return prob->pde == PDDS_PDE_TABLE && geom == GeomRect &&
-           (r->precision == PDDS_FP64 || pp.step == STEP_CV || pp.step == STEP_PLAIN) &&
-           paths >= kTableTileLane * e->n_cu * (int64_t)path_tiled_wg(prob->pde, r->precision, r->step, geom);
+// The LDS tiles of a launch's knots (columns, rows, width, height, and the planes staged of it: 0 where
+// it does not fit), and whether the launch takes the tiled kernel, unless the group kernel takes it:
+// coefficient LUT with a fifth-field quad plane; the tabulated problem in rectangles by tabulated_tiles
+// (not its FP32 VR and VR + CV steps, whose rounding follows the persistent kernel's code).  Not with
+// reflecting sides, whose steps run in the persistent and plain kernels.  paths: the launch counts as
+// one of at least so many.
+struct TilePlan {
+    bool tiled = false;
+    std::vector<std::array<int, 5>> key;
+};
+static TilePlan plan_tiles(const pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const PdeParams &pp, int geom,
+                           const std::vector<const DevTables *> &tabs, const std::vector<AsmKnot> &knots, int64_t paths) {
+    TilePlan t;
+    const bool table = prob->pde == PDDS_PDE_TABLE;
+    if (r->plain != 0 || r->lut_lds == 0 || pp.refl != 0) return t;
+    if (table ? geom != GeomRect || !(r->precision == PDDS_FP64 || pp.step == STEP_CV || pp.step == STEP_PLAIN)
+              : prob->pde != PDDS_PDE_VARCOEF_LUT || pp.lut.nf != 5)
+        return t;
+    const int64_t lanes = (int64_t)e->n_cu * path_tiled_wg(prob->pde, r->precision, r->step, geom);
+    int64_t all = 0, fitting = 0;
+    for (const AsmKnot &k : knots) all += k.n;
+    if (table && !tabulated_tiles(std::max(all, paths), lanes, 1.0)) return t;
+    // the tabulated problem's tile holds its fields' two planes, and with a VR + CV step that of mu
+    // and F where its grid is the same and there is room
+    const LutView &la = pp.lut, &lv = pp.vlut;
+    const int planes = !table ? 1
+                       : pp.step == STEP_VRCV && la.nx == lv.nx && la.ny == lv.ny && la.px == lv.px && la.ox == lv.ox &&
+                                 la.oy == lv.oy && la.sx == lv.sx && la.sy == lv.sy ? 3 : 2;
+    const size_t cap = e->lds_max > 1024 ? e->lds_max - 1024 : 0;
+    t.key.resize(knots.size());
+    for (size_t i = 0; i < knots.size(); ++i) {
+        int c0, r0, tw, th;
+        lut_tile_of(pp.lut, tabs[knots[i].table]->host_sten[knots[i].stencil].bbox, c0, r0, tw, th);
+        const size_t plane = (size_t)(tw + r->lut_pad) * th * sizeof(float4);
+        const int fits = plane * planes <= cap ? planes : planes == 3 && plane * 2 <= cap ? 2 : 0;
+        t.key[i] = {c0, r0, tw, th, fits};
+        if (fits) fitting += knots[i].n;
+    }
+    t.tiled = !table || tabulated_tiles(std::max(all, paths), lanes, (double)fitting / (double)std::max<int64_t>(1, all));
+    return t;
 }
 
 // Lanes to a path of such a launch in the group kernel; 0: another kernel takes it.
@@ -332,29 +360,18 @@ pdds_status run_assembly(pdds_engine *e, const pdds_problem *prob, const pdds_ru
     if (pp.refl && geom != GeomRect) return fail(e, PDDS_ERR_UNSUPPORTED, "reflecting sides need rectangular stencils");
     // LDS-tiled form: knots are grouped into patches of equal tile, tiles that fit in LDS first, in
     // first-seen order
-    int64_t all_paths = 0;
-    for (const AsmKnot &k : knots) all_paths += k.n;
-    // the tabulated problem's tile holds its fields' two planes, and with a VR + CV step that of mu
-    // and F where its grid is the same and there is room
-    const LutView &la = pp.lut, &lv = pp.vlut;
-    const int tile_planes = prob->pde != PDDS_PDE_TABLE ? 1
-                            : pp.step == STEP_VRCV && la.nx == lv.nx && la.ny == lv.ny && la.px == lv.px && la.ox == lv.ox &&
-                                      la.oy == lv.oy && la.sx == lv.sx && la.sy == lv.sy ? 3 : 2;
-    const bool tiled = takes_tiles(e, prob, r, pp, geom, std::max(all_paths, as_paths));
-    const size_t tile_cap = e->lds_max > 1024 ? e->lds_max - 1024 : 0;
+    const TilePlan plan = plan_tiles(e, prob, r, pp, geom, tabs, knots, as_paths);
+    const bool tiled = plan.tiled;
+    const std::vector<std::array<int, 5>> &tkey = plan.key;
     std::vector<size_t> ord(knots.size());
     for (size_t i = 0; i < ord.size(); ++i) ord[i] = i;
-    std::vector<std::array<int, 5>> tkey(knots.size());   // c0, r0, tw, th, fits
     if (tiled) {
         std::map<std::array<int, 4>, int> first;
         std::vector<int> rank(knots.size());
         for (size_t i = 0; i < knots.size(); ++i) {
-            int c0, r0, tw, th;
-            lut_tile_of(pp.lut, host_sd(knots[i]).bbox, c0, r0, tw, th);
-            const size_t plane = (size_t)(tw + r->lut_pad) * th * sizeof(float4);
-            const int fits = plane * tile_planes <= tile_cap ? tile_planes : tile_planes == 3 && plane * 2 <= tile_cap ? 2 : 0;
-            tkey[i] = {c0, r0, tw, th, fits};
-            const std::array<int, 4> k4 = fits ? std::array<int, 4>{c0, r0, tw, th} : std::array<int, 4>{-1, -1, -1, -1};
+            const bool fits = tkey[i][4] != 0;
+            const std::array<int, 4> k4 = fits ? std::array<int, 4>{tkey[i][0], tkey[i][1], tkey[i][2], tkey[i][3]}
+                                               : std::array<int, 4>{-1, -1, -1, -1};
             auto it = first.find(k4);
             if (it == first.end()) it = first.emplace(k4, fits ? (int)i : (int)knots.size() + (int)i).first;
             rank[i] = it->second;
@@ -1360,7 +1377,7 @@ pdds_status pdds_autotune(pdds_engine *e, const pdds_mesh *m, const pdds_problem
             for (int ppl : {1, 4, 16}) add(base->lut_lds, base->wg_size, g * e->n_cu, ppl, base->lut_pad);
     } else {
         // LDS-tiled shapes: work-groups per CU, paths per lane and the tile's row pitch
-        if (takes_tiles(e, p, &tile_run, pp, M.geom, large))
+        if (plan_tiles(e, p, &tile_run, pp, M.geom, {T}, knots, large).tiled)
             for (int pad : {0, 1, 2, 3})
                 for (int g : {1, 2})
                     for (int ppl : {1, 2, 4, 8}) add(1, 0, g * e->n_cu, ppl, pad);

@@ -12,11 +12,16 @@ namespace pdds {
 // assembly (0.6 M) 3.4 and 3.5; FP64 Helmholtz assembly (1.9 M) 2.5 and 3.1, FP64 recorded run
 // (0.77 M) 4.0 and 3.6; with four and sixteen lanes: 140 k FP32 paths 1.25 and 1.16 ms, 5000 FP64
 // paths 0.73 and 0.58, 4000 0.34 and 0.29.
+// The tabulated problem's eight fields are 32 reads of 16 bytes a step, which each lane of a group
+// repeats (4 x 4 subdomains, 128 x 128 texels, h = 2e-4; by groups and by one lane in the persistent
+// kernel): FP64 6 10^4 paths 3.4 and 4.0 ms, 1.2 10^5 4.1 and 4.3, 2 10^5 5.7 and 5.1; FP32 2.65 and 3.1,
+// 4.8 and 5.1, 6.3 and 5.6, and with 512 x 512 texels on 8 x 8 3.6 and 3.1, 6.0 and 3.6, 7.9 and 4.6.
 int group_lanes(int pde, int precision, bool refl, int n_cu, int64_t paths) {
     const bool fp64 = precision == PDDS_FP64;
     const bool moves = pde == PDE_SINSIN || pde == PDE_HELMHOLTZ || pde == PDE_MONEGROS;   // const_motion
     if (!fp64 && (refl || pde == PDE_MONEGROS)) return 0;
     if ((!moves || refl) && paths > (int64_t)n_cu * 2048) return 0;
+    if (pde == PDE_TABLE && paths > (int64_t)n_cu * (fp64 ? 512 : 256)) return 0;
     if (!moves) return 4;
     if (refl) return paths > (int64_t)n_cu * 32 ? 4 : 16;
     if (paths >= (int64_t)n_cu * (fp64 ? 4096 : 2048)) return 1;

@@ -253,10 +253,17 @@ struct PathLaunch {
 // Launchers (defined in engine_f64.hip / engine_f32.hip)
 hipError_t launch_path_tiled_f64(int pde, int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
 hipError_t launch_path_tiled_f32(int pde, int geom, bool mixed, int grid, size_t lds, hipStream_t s, const PathKernelArgs &a);
-// The tabulated problem takes the LDS-tiled kernel from this many paths per lane of its grid (357 knots, a
-// table of 128 x 128, FP64, VR step: 285 10^3 paths 4.6 ms, 5.4 without; 1.4 10^6 6.7 ms and 11; at 142 10^3
-// the two are equal, 4.0 ms)
-constexpr int64_t kTableTileLane = 1;
+// Whether a launch of the tabulated problem takes the LDS-tiled kernel, by its paths, the lanes of the
+// tiled grid (131072 on 256 CUs) and the share of paths whose tile fits.  Where all fit, from four paths a
+// lane on: 357 knots of 8 x 8 or 4 x 4 subdomains, 128 x 128 texels, FP64, h = 2e-4 and 2e-3 of the
+// subdomain: 5.2 10^5 paths 9.2 and 1.13 ms, persistent kernel 8.4 and 1.07 (VR + CV 14.3 and 1.87,
+// 13.6 and 2.06; FP32 6.3 and 0.73, 8.2 and 1.0); 10^6 9.3 and 1.14, 11.3 and 1.4; 3 10^5 8.6 and 1.14,
+// 6.0 and 0.88.  The patch without a tile is worked on last, by all, with the tiled kernel's thin grid: where
+// 3 of 100 paths have none, 2.5 10^6 paths take 2.85 ms (2.58), 8 10^6 5.0 (6.6); where none fits (512 x 512
+// texels) 8 10^6 take 9.0 ms (8.1), 2 10^5 17.8 (5.4).
+inline bool tabulated_tiles(int64_t paths, int64_t lanes, double fitting) {
+    return fitting >= 1.0 ? paths >= 4 * lanes : fitting >= 0.9 && paths >= 32 * lanes;
+}
 int path_tiled_wg(int pde, int precision, int step, int geom);   // block size of the LDS-tiled kernel
 hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);

@@ -1,6 +1,6 @@
-"""Tiled launches in which no stencil's tile fits in LDS: every patch reads its tables from global
-memory, also on a pass whose last paths stop in its first step (the FP32 kernels of two steps a
-pass).  Results are those of the persistent kernel, bit for bit."""
+"""Tiled launches in which some or all stencils' tiles do not fit in LDS: their patch reads its tables
+from global memory, also on a pass whose last paths stop in its first step (the FP32 kernels of
+two steps a pass).  Results are those of the persistent kernel, bit for bit."""
 import numpy as np
 import pytest
 
@@ -16,9 +16,10 @@ def eng():
     e.close()
 
 
-def _equal(eng, mesh, problem, counts, **run):
+def _equal(eng, mesh, problem, counts, wg, **run):
     from pdds_amd.engine import default_run
-    a, b = (eng.assemble(mesh, problem, default_run(lut_lds=lds, **run), 0, paths_per_knot=counts) for lds in (1, 0))
+    a, b = (eng.assemble(mesh, problem, default_run(lut_lds=lds, wg_size=128, **run), 0, paths_per_knot=counts) for lds in (1, 0))
+    assert a["counters"]["wg_size"] == wg and b["counters"]["wg_size"] == 128
     for k in ("G", "Gvar", "B", "BB"):
         assert np.array_equal(a[k], b[k]), k
     for k in ("path_steps", "exits", "paths"):
@@ -26,15 +27,15 @@ def _equal(eng, mesh, problem, counts, **run):
 
 
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
-def test_table_without_tiles(eng, precision):
+def test_table_with_some_tiles(eng, precision):
     from pdds_amd.engine import Mesh
     from pdds_amd.workloads import relative_fac, table_problem
-    # a segment's stencil covers 300 x 150 texels of 32 bytes
-    m = Mesh(SW, NE, 4, 8, relative_fac(SW, NE, 4, 8, 0.8))
-    counts = np.where(m.on_boundary, 1, 6000).astype(np.int64)
+    # the crossing's stencil does not fit, the others' do: 4.3 10^6 paths
+    m = Mesh(SW, NE, 4, 16, relative_fac(SW, NE, 4, 16, 0.8))
+    counts = np.where(m.on_boundary, 0, 12500).astype(np.int64)
     counts[70] = 5437
-    print("table 600", precision, flush=True)
-    _equal(eng, m, table_problem(eng, 600, SW + NE), counts, h=2e-3, seed=9, precision=precision)
+    print("table 160", precision, flush=True)
+    _equal(eng, m, table_problem(eng, 160, SW + NE), counts, 512, h=8e-3, seed=9, precision=precision)
 
 
 @pytest.mark.parametrize("precision", ["fp32", "fp64"])
@@ -46,4 +47,4 @@ def test_disc_without_tiles(eng, precision):
     counts = np.where(m.on_boundary, 0, 700).astype(np.int64)
     counts[5] = 321
     print("disc 1024", precision, flush=True)
-    _equal(eng, m, bvp("varcoef_lut", lut=varcoef_lut(eng, 1024, SW + NE)), counts, h=1e-3, seed=4, precision=precision)
+    _equal(eng, m, bvp("varcoef_lut", lut=varcoef_lut(eng, 1024, SW + NE)), counts, 512, h=1e-3, seed=4, precision=precision)
