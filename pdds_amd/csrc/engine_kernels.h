@@ -127,11 +127,14 @@ PDDS_HD void rbf_tab4(double px, double py, const double x[4], const double y[4]
 // stays 0).  Two exponentials per chunk instead of one per entry; the values equal the direct ones
 // to about 1e-13 relative (those below about 1e-180 may come out as 0).  Each value phi_k is added
 // as acc[k] = fma(Y, phi_k, acc[k]); the sums for k past the side's end are formed and not used.
+// BRANCH: r_0 by dexp_fast, the same bits with a branch for the exponents far from 0.
+template <bool BRANCH = false>
 PDDS_HD void rbf_side_chunk(const double *px, const double *py, int j0, double sx, double sy, double ss, double q,
                             double x, double y, double inv_c2, const double *T, double Y, double acc[kRbfChunk]) {
     const double dx = px[j0] - x, dy = py[j0] - y;
     double p = dexp_tab_nonpos(-(dx * dx + dy * dy) * inv_c2, T);
-    double r = dexp_le700(__builtin_fmin(-(2.0 * (dx * sx + dy * sy) + ss) * inv_c2, 700.0));
+    const double xr = __builtin_fmin(-(2.0 * (dx * sx + dy * sy) + ss) * inv_c2, 700.0);
+    double r = BRANCH ? dexp_fast(xr) : dexp_le700(xr);
     acc[0] = __builtin_fma(Y, p, acc[0]);
 #pragma unroll
     for (int k = 1; k < kRbfChunk; ++k) {
