@@ -327,6 +327,20 @@ static TilePlan plan_tiles(const pdds_engine *e, const pdds_problem *prob, const
     return t;
 }
 
+// Paths up to which a call for records takes the group kernel rather than a lane to a path.  A LUT's or
+// table's reads are repeated by the lanes of a path, which pays while the card waits for the
+// longest paths (groups and one lane to a path, h = 1e-2 and 3e-4 on the square, 512 x 512 samples): FP64
+// LUT 10^5 paths 1.5 and 1.2 ms, 37 and 36 (64 x 64 1.0 and 1.1, 26 and 32), 3 10^5 2.7 and 2.0, 71 and
+// 63, with a second phase 3.5 and 2.8, 73 and 77; FP64 table 3 10^5 2.5 and 3.1, 71 and 98, 10^6 7.4 and
+// 7.4, 205 and 234 (64 x 64 5.0 and 4.2, 113 and 130).  FP32, h = 1e-2 and 1e-3: LUT 300 paths 0.50 and 0.37, 5.5
+// and 3.4, 10^5 1.4 and 0.67, 14 and 7.5; table 2 10^4 0.60 and 0.66, 5.7 and 6.8, 10^5 1.7 and 1.2, 15 and 13.
+static int64_t records_by_groups(const pdds_engine *e, const pdds_problem *prob, bool fp64, bool phase2) {
+    const int64_t cu = e->n_cu;
+    if (prob->pde == PDDS_PDE_VARCOEF_LUT) return !fp64 ? 0 : cu * (phase2 ? 1024 : 512);
+    if (prob->pde == PDDS_PDE_TABLE) return cu * (fp64 ? 2048 : 256);
+    return ((int64_t)1 << 32) - 1;    // its indices have 32 bits
+}
+
 // Lanes to a path of such a launch in the group kernel; 0: another kernel takes it.
 static int launch_lanes(const pdds_engine *e, const pdds_problem *prob, const pdds_run *r, const PdeParams &pp, int geom,
                         int64_t paths) {
@@ -1624,7 +1638,7 @@ pdds_status pdds_paths(pdds_engine *e, const pdds_problem *p, const pdds_run *r,
     // the control-variate step as a group launch of one knot, whose lanes take up new paths where one
     // per lane would wait for its wave's longest; not the FP32 forms that the group kernel lacks (a
     // second phase starts at any step count, half a Philox call) nor counts past its 32-bit indices
-    const bool group = pp.step == STEP_CV && n < ((int64_t)1 << 32) && a.max_steps < ((int64_t)1 << 27) &&
+    const bool group = pp.step == STEP_CV && n <= records_by_groups(e, p, fp64, phase2 != 0) && a.max_steps < ((int64_t)1 << 27) &&
                        (fp64 || (!phase2 && !pp.refl && p->pde != PDDS_PDE_MONEGROS));
     PathKernelArgs ga;
     PathOut go;
@@ -1658,6 +1672,10 @@ pdds_status pdds_paths(pdds_engine *e, const pdds_problem *p, const pdds_run *r,
         int per_cu = 0;
         HIPCHK(launch(PathLaunch{0, wg, e->stream, &per_cu}));
         grid = path_grid(e->n_cu, per_cu, wg, 64 / 4, n, 0, 0, ga);
+        // (larger chunks in launches of many, so that paths of few steps do not wait for their queue's
+        // counter, which takes 0.1 us to a chunk: 10^6 FP32 paths of 25 steps 0.70 ms with chunks of
+        // 20 paths, 0.27 with 64; of 250 steps 1.40 and 1.45)
+        ga.pool_chunk = std::max<int64_t>(ga.pool_chunk, std::min<int64_t>(64, n / (32 * (int64_t)e->n_cu)));
         HIPCHK(hipEventRecord(e->ev[0], e->stream));
         HIPCHK(launch(PathLaunch{(int)grid, wg, e->stream, nullptr}));
     } else {

@@ -30,13 +30,12 @@ template <int PDE> static hipError_t group_records_f32(const PathLaunch &l, cons
     return l.go(group_kernel<float, PDE, false, 4, false, PathOut>, a, o);
 }
 
-// one phase, without reflecting sides
+// one phase, without reflecting sides; not the coefficient LUT, whose records take one lane to a path
 hipError_t launch_group_records_f32(int pde, const PathLaunch &l, const PathKernelArgs &a, const PathOut &o) {
     if (a.pp.refl || o.phase2) return hipErrorInvalidValue;
     switch (pde) {
         case PDE_SINSIN: return group_records_f32<PDE_SINSIN>(l, a, o);
         case PDE_VARCOEF: return group_records_f32<PDE_VARCOEF>(l, a, o);
-        case PDE_VARCOEF_LUT: return group_records_f32<PDE_VARCOEF_LUT>(l, a, o);
         case PDE_HELMHOLTZ: return group_records_f32<PDE_HELMHOLTZ>(l, a, o);
         case PDE_TABLE: return group_records_f32<PDE_TABLE>(l, a, o);
         default: return hipErrorInvalidValue;
