@@ -120,13 +120,16 @@ typedef struct {
     int64_t max_steps;      /* per-path step cap (0: 2^26) */
     int32_t sub_batch;      /* paths per variance batch S (0: 32) */
     int32_t item_paths;     /* paths per work item P, multiple of S (0: chosen from the path count) */
-    int32_t wg_size;        /* work-group size (0: 256) */
-    int32_t grid_wgs;       /* persistent work-groups (0: 2 per CU) */
-    int32_t lut_lds;        /* 1: stage LUT tiles in LDS when they fit (default 1) */
+    int32_t wg_size;        /* work-group size of the persistent and plain kernels (0: 256); launches of
+                               several lanes to a path and LDS-tiled ones have their own */
+    int32_t grid_wgs;       /* work-groups of a persistent or tiled launch (0: chosen from the path count) */
+    int32_t lut_lds;        /* 1: large launches stage LUT tiles in LDS where they fit (default 1); launches
+                               of several lanes to a path do not read it */
     int32_t plain;          /* 1: plain launch -- one path per lane, one work-group per item of wg_size
                                paths, no lane recycling, no persistent queue (the baseline GPU form) */
-    int32_t paths_per_lane; /* persistent launches: a wave takes 64 x this many paths from its queue
-                               at once (0: 4); results do not depend on it */
+    int32_t paths_per_lane; /* persistent launches: a wave takes as many paths from its queue at once
+                               as this many passes of its lanes need (0: chosen from the path count);
+                               results do not depend on it */
     int32_t step;           /* step family (PDDS_STEP_*, default 0) */
     int32_t adaptive_h;     /* 1: each knot's paths step with h_k = min(h, (d / (2 |beta| |N^T sigma(X0)|))^2),
                                d the knot's signed distance to its stopping domain and N that side's

@@ -19,11 +19,12 @@
 // cheapest per step (FP32 Helmholtz: about 280 VALU instructions for two steps of 64 paths, 377 for
 // eight steps of 16) and one of 16 has the shortest step (a path of the FP64 recorded run: 1.9 us a
 // step with one path per lane, 0.15 us here).  A launch starts as wide as its path count asks for
-// (group_lanes) and widens where a wave's last paths leave room.  Measured against one path per
-// lane: 4 points x 1000 paths 1.9 -> 0.29 ms, one knot of the recorded run 4.7 -> 0.58, the whole
-// run 8.0 -> 3.6, Poisson FP32 (0.6 M paths) 8.2 -> 3.4, server burst 139 -> 83 ms; per-path records
-// of 1e5 two-phase paths 9.5 -> 5.4, 16 Robin points x 4096 paths 8.5 -> 4.0, 390 k paths of a LUT
-// assembly 7.3 -> 5.6 (FP64) and 8.9 -> 4.0 ms (FP32).
+// (group_lanes) and widens where a wave's last paths leave room.  Against one path per lane, whole
+// calls: 4 points x 1000 paths 2.4 -> 0.29 ms, one knot of the recorded run 7.0 -> 0.55, the whole
+// run 11.2 -> 3.4, Poisson FP32 (0.6 M paths) 13.0 -> 3.4, server burst 129 -> 73; per-path records
+// of 1e5 two-phase paths 10.9 -> 4.3, 16 Robin points x 4096 paths 10.6 -> 4.2.  Lanes that read a
+// table repeat its reads: at the limit of 2048 paths per CU the LUT's launches are no faster than with
+// a lane per path (5.2 10^5 paths of points on the whole square, 64 x 64 samples: FP64 8.9 ms, 7.8 so).
 #pragma once
 #include <type_traits>
 #include <utility>

@@ -65,7 +65,6 @@ struct pdds_engine {
     DevTables dom;              // one-stencil table of the rectangle point evaluations stop on
     double dom_rect[4] = {0, 0, 0, 0};
     int64_t record_budget = (int64_t)24 << 30;   // bytes of exit records per assembly batch
-    int path_wgs_per_cu = 8;                      // persistent path-kernel work-groups per CU
     size_t lds_max = 64 * 1024;                   // LDS bytes a work-group may use
     Arena *arena = nullptr;     // set only inside pdds_point_eval_noalloc
     char *scratch = nullptr;    // device address of this device's no-allocation scratch array

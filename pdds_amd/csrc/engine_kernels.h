@@ -13,8 +13,8 @@
 //    and its exit record (projection, Y, score) is written at its global path
 //    index; steps are summed per knot.  The plain form launches one lane per path,
 //    no refill; path_kernel_tiled reads its tables from LDS tiles; small launches
-//    and those of constant-motion problems run in engine_group.h's group_kernel,
-//    several lanes per path.
+//    of the control-variate step in rectangles, and those of constant-motion
+//    problems at any size, run in engine_group.h's group_kernel, several lanes per path.
 //  * reduce16_kernel (reduce_kernel for what it does not take): work items of P
 //    paths of one knot per work-group.  Per
 //    sub-batch of S paths it forms the per-side RBF moments Phi_j = sum Y phi_j(X)
@@ -963,8 +963,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_
 // outside the tile go to the vector L1.  The tabulated problem holds both planes of its eight
 // fields, and with a VR + CV step that of mu and F if its grid is the same and there is room.
 // Without the tile its step waits for 32 (48) scattered 16-byte reads of the vector L1, about a cache
-// line a cycle: 357 knots, 1.4 10^6 paths, a table of 128 x 128, FP64, h = 5e-4: VR + CV step 15.5 ms
-// persistent, 9.4 ms tiled; control variates 10.0 and 6.4 ms (FP32 9.3 and 4.9).
+// line a cycle: 357 knots, 1.4 10^6 paths, a table of 128 x 128, FP64, h = 5e-4: VR + CV step 8.9 ms
+// persistent, 7.2 ms tiled; control variates 6.0 and 4.7 ms (FP32 5.1 and 3.1).
 // ----------------------------------------------------------------------------
 // one work-group per CU holding every wave the register budget allows (the run-time step-family
 // variants one wave less, as in path_kernel, and so the FP32 annular-sector kernels, whose
