@@ -287,8 +287,8 @@ static int path_grid(int n_cu, int per_cu, int wg, int64_t slots, int64_t tot, i
 
 // The LDS tiles of a launch's knots (columns, rows, width, height, and the planes staged of it: 0 where
 // it does not fit), and whether the launch takes the tiled kernel, unless the group kernel takes it:
-// coefficient LUT with a fifth-field quad plane; the tabulated problem in rectangles by tabulated_tiles
-// (not its FP32 VR and VR + CV steps, whose rounding follows the persistent kernel's code).  Not with
+// coefficient LUT with a fifth-field quad plane by lut_tiles; the tabulated problem in rectangles by
+// tabulated_tiles (not its FP32 VR and VR + CV steps, whose rounding follows the persistent kernel's code).  Not with
 // reflecting sides, whose steps run in the persistent and plain kernels.  paths: the launch counts as
 // one of at least so many.
 struct TilePlan {
@@ -306,7 +306,11 @@ static TilePlan plan_tiles(const pdds_engine *e, const pdds_problem *prob, const
     const int64_t lanes = (int64_t)e->n_cu * path_tiled_wg(prob->pde, r->precision, r->step, geom);
     int64_t all = 0, fitting = 0;
     for (const AsmKnot &k : knots) all += k.n;
-    if (table && !tabulated_tiles(std::max(all, paths), lanes, 1.0)) return t;
+    auto takes = [&](double share) {
+        return table ? tabulated_tiles(std::max(all, paths), lanes, share)
+                     : lut_tiles(r->precision == PDDS_FP64, geom == GeomRect, std::max(all, paths), lanes, share);
+    };
+    if (!takes(1.0)) return t;
     // the tabulated problem's tile holds its fields' two planes, and with a VR + CV step that of mu
     // and F where its grid is the same and there is room
     const LutView &la = pp.lut, &lv = pp.vlut;
@@ -323,7 +327,7 @@ static TilePlan plan_tiles(const pdds_engine *e, const pdds_problem *prob, const
         t.key[i] = {c0, r0, tw, th, fits};
         if (fits) fitting += knots[i].n;
     }
-    t.tiled = !table || tabulated_tiles(std::max(all, paths), lanes, (double)fitting / (double)std::max<int64_t>(1, all));
+    t.tiled = takes((double)fitting / (double)std::max<int64_t>(1, all));
     return t;
 }
 

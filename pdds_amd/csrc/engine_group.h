@@ -22,9 +22,7 @@
 // (group_lanes) and widens where a wave's last paths leave room.  Against one path per lane, whole
 // calls: 4 points x 1000 paths 2.4 -> 0.29 ms, one knot of the recorded run 7.0 -> 0.55, the whole
 // run 11.2 -> 3.4, Poisson FP32 (0.6 M paths) 13.0 -> 3.4, server burst 129 -> 73; per-path records
-// of 1e5 two-phase paths 10.9 -> 4.3, 16 Robin points x 4096 paths 10.6 -> 4.2.  Lanes that read a
-// table repeat its reads: at the limit of 2048 paths per CU the LUT's launches are no faster than with
-// a lane per path (5.2 10^5 paths of points on the whole square, 64 x 64 samples: FP64 8.9 ms, 7.8 so).
+// of 1e5 two-phase paths 10.9 -> 4.3, 16 Robin points x 4096 paths 10.6 -> 4.2.
 #pragma once
 #include <type_traits>
 #include <utility>

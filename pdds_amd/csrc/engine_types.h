@@ -264,6 +264,19 @@ hipError_t launch_path_tiled_f32(int pde, int geom, bool mixed, int grid, size_t
 inline bool tabulated_tiles(int64_t paths, int64_t lanes, double fitting) {
     return fitting >= 1.0 ? paths >= 4 * lanes : fitting >= 0.9 && paths >= 32 * lanes;
 }
+// The same of the coefficient LUT (lanes: 131072, FP32 rectangles 196608).  Each pair: tiled and persistent
+// kernel, at h = 1e-2 of the subdomain's size squared, and where two follow, at 1e-3.  FP64: 2 10^6 paths
+// 4.8 and 4.7 ms, 46 and 42 (8 x 8 subdomains of 32 knots, 256 x 256 samples, all tiles fit), 6.8 and 5.9,
+// 59 and 62 (512 x 512, a few tiles do not); 6 10^6 paths 9.7 and 10.1, 10.9 and 12.9 (64 x 64: 9.8 and 9.1);
+// 1.5 10^7 18.9 and 21.9, 18.8 and 28.2; where none fits (4 x 4) 6 10^6 take 14.4 and 14.7, 1.5 10^7 32.7 and
+// 34.3.  FP32: 5 10^5 paths 2.3 and 1.7, 25 and 20 (128 x 128 on 4 x 4), 10^6 2.1 and 3.1, 21 and 27 (256 x 256
+// on 8 x 8); where a few tiles do not fit 2 10^6 6.7 and 5.5, 58 and 48, 6 10^6 8.6 and 12.2; where none
+// fits 15.9 and 13.6 (6 10^6), 34.8 and 32.1 (1.5 10^7).  Discs of 24 to 144 sectors, FP32: 2 10^6 paths 1.0
+// and 1.5, 1.5 and 1.3, 6 10^6 1.9 and 3.1, 2.0 and 2.2.
+inline bool lut_tiles(bool fp64, bool rect, int64_t paths, int64_t lanes, double fitting) {
+    if (fp64) return paths >= 24 * lanes;
+    return fitting >= 0.75 && paths >= (rect && fitting >= 1.0 ? 6 : 16) * lanes;
+}
 int path_tiled_wg(int pde, int precision, int step, int geom);   // block size of the LDS-tiled kernel
 hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);
 hipError_t launch_path_f32(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);

@@ -28,8 +28,8 @@ def mesh():
 
 
 def _many(eng, mesh):
-    """Paths per knot with which a launch has more than 2048 paths per CU."""
-    return int(eng.info()["n_cu"]) * 2048 // int(np.sum(~mesh.on_boundary)) + 200
+    """Paths per knot with which a launch takes the tiled kernel, if three of its tiles in four fit."""
+    return int(eng.info()["n_cu"]) * 24 * 512 // int(np.sum(~mesh.on_boundary)) + 200
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
@@ -94,14 +94,17 @@ def test_lut_assembly_is_the_same_in_every_kernel(eng, mesh, mode, n, precision)
     assert ref["counters"]["wg_size"] == 128
     for pad in (0, 1, 3, 7):
         got = eng.assemble(mesh, prob, default_run(lut_pad=pad, wg_size=128, **run), 0, paths_per_knot=counts)
-        assert got["counters"]["wg_size"] == TILED[precision], pad
+        # (of 256 samples most tiles with 7 spare texels a row do not fit)
+        assert got["counters"]["wg_size"] == (128 if pad == 7 and n == 256 and precision == "fp32" else TILED[precision]), pad
         _same(got, ref)
-    few = np.where(np.arange(mesh.n_knots) % 5 == 43 % 5, counts, 0)
+    few = np.where(np.arange(mesh.n_knots) == 42, 30011, np.where(np.arange(mesh.n_knots) == 43, 1500, 0))
     got = eng.assemble(mesh, prob, default_run(wg_size=128, **run), 0, paths_per_knot=few)
     assert got["counters"]["wg_size"] == 256
+    ref2 = eng.assemble(mesh, prob, default_run(lut_lds=0, wg_size=128, **run), 0, paths_per_knot=np.where(few > 0, few, counts))
+    assert ref2["counters"]["wg_size"] == 128
     for k in np.flatnonzero(few):
         r = slice(mesh.row_ptr[k], mesh.row_ptr[k + 1])
-        assert np.array_equal(got["G"][r], ref["G"][r]) and got["B"][k] == ref["B"][k], k
+        assert np.array_equal(got["G"][r], ref2["G"][r]) and got["B"][k] == ref2["B"][k], k
     if precision == "fp64":
         _same(eng.assemble(mesh, prob, default_run(plain=1, **run), 0, paths_per_knot=counts), ref)
         _knot_equals_oracle(ref, mesh, olut, 43, 1500, h, 5)
@@ -135,7 +138,7 @@ def test_tiled_shards_are_bit_identical(eng, mesh):
     assembly's bits."""
     from pdds_amd.engine import bvp, default_run
     samples, _ = _table(0, 256)
-    prob, many = bvp("varcoef_lut", lut=eng.lut(samples, BOX)), 3 * _many(eng, mesh)
+    prob, many = bvp("varcoef_lut", lut=eng.lut(samples, BOX)), 4 * _many(eng, mesh)
     run = default_run(h=8e-3, seed=29, sub_batch=32, item_paths=640)
     full = eng.assemble(mesh, prob, run, many)
     assert full["counters"]["wg_size"] == 512

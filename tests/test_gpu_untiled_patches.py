@@ -38,13 +38,13 @@ def test_table_with_some_tiles(eng, precision):
     _equal(eng, m, table_problem(eng, 160, SW + NE), counts, 512, h=8e-3, seed=9, precision=precision)
 
 
-@pytest.mark.parametrize("precision", ["fp32", "fp64"])
-def test_disc_without_tiles(eng, precision):
+# 1024: a sector's box covers at least 150 x 150 texels of 16 bytes, no tile fits; 256: a fifth do not
+@pytest.mark.parametrize("precision,n", [("fp64", 1024), ("fp64", 256), ("fp32", 256)])
+def test_disc_without_tiles(eng, precision, n):
     from pdds_amd.engine import Mesh, bvp
     from pdds_amd.workloads import varcoef_lut
-    # a sector's box covers at least 150 x 150 texels of 16 bytes
     m = Mesh.disc(1.0, 3, 8, 11, 6, 12, 1.0)
-    counts = np.where(m.on_boundary, 0, 700).astype(np.int64)
+    counts = np.where(m.on_boundary, 0, 8000).astype(np.int64)
     counts[5] = 321
-    print("disc 1024", precision, flush=True)
-    _equal(eng, m, bvp("varcoef_lut", lut=varcoef_lut(eng, 1024, SW + NE)), counts, 512, h=1e-3, seed=4, precision=precision)
+    print("disc", n, precision, flush=True)
+    _equal(eng, m, bvp("varcoef_lut", lut=varcoef_lut(eng, n, SW + NE)), counts, 512, h=1e-3, seed=4, precision=precision)
