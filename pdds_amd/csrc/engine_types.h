@@ -269,13 +269,13 @@ inline bool tabulated_tiles(int64_t paths, int64_t lanes, double fitting) {
 // 4.8 and 4.7 ms, 46 and 42 (8 x 8 subdomains of 32 knots, 256 x 256 samples, all tiles fit), 6.8 and 5.9,
 // 59 and 62 (512 x 512, a few tiles do not); 6 10^6 paths 9.7 and 10.1, 10.9 and 12.9 (64 x 64: 9.8 and 9.1);
 // 1.5 10^7 18.9 and 21.9, 18.8 and 28.2; where none fits (4 x 4) 6 10^6 take 14.4 and 14.7, 1.5 10^7 32.7 and
-// 34.3.  FP32: 5 10^5 paths 2.3 and 1.7, 25 and 20 (128 x 128 on 4 x 4), 10^6 2.1 and 3.1, 21 and 27 (256 x 256
-// on 8 x 8); where a few tiles do not fit 2 10^6 6.7 and 5.5, 58 and 48, 6 10^6 8.6 and 12.2; where none
+// 34.3.  FP32 (4 x 4, 128 x 128, at 5e-3 and 1e-3): 5.4 10^5 paths 4.6 and 3.8, 24 and 21, 7.7 10^5 4.7 and
+// 4.5, 24 and 23, 10^6 4.5 and 5.5, 21 and 25 (256 x 256 on 8 x 8 4.3 and 5.4, 21 and 27); where a few tiles do not fit 2 10^6 6.7 and 5.5, 58 and 48, 6 10^6 8.6 and 12.2; where none
 // fits 15.9 and 13.6 (6 10^6), 34.8 and 32.1 (1.5 10^7).  Discs of 24 to 144 sectors, FP32: 2 10^6 paths 1.0
 // and 1.5, 1.5 and 1.3, 6 10^6 1.9 and 3.1, 2.0 and 2.2.
 inline bool lut_tiles(bool fp64, bool rect, int64_t paths, int64_t lanes, double fitting) {
     if (fp64) return paths >= 24 * lanes;
-    return fitting >= 0.75 && paths >= (rect && fitting >= 1.0 ? 6 : 16) * lanes;
+    return fitting >= 0.75 && paths >= (rect && fitting >= 1.0 ? 4 : 16) * lanes;
 }
 int path_tiled_wg(int pde, int precision, int step, int geom);   // block size of the LDS-tiled kernel
 hipError_t launch_path_f64(int pde, int geom, bool persistent, bool mixed, const PathLaunch &l, const PathKernelArgs &a);

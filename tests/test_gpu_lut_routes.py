@@ -28,7 +28,7 @@ def _counts(mesh, total):
 
 # samples per side: 64 every tile fits, 256 the crossing's does not, 512 none; paths per CU at the limit
 @pytest.mark.parametrize("precision,n,per_cu,wg", [("fp64", 64, 24 * 512, 512), ("fp64", 512, 24 * 512, 512),
-                                                   ("fp32", 64, 6 * 768, 768), ("fp32", 256, 16 * 768, 768),
+                                                   ("fp32", 64, 4 * 768, 768), ("fp32", 256, 16 * 768, 768),
                                                    ("fp32", 512, 16 * 768, 128)])
 def test_tiles_by_paths_and_fit(eng, precision, n, per_cu, wg):
     from pdds_amd.engine import Mesh, bvp, default_run
