@@ -474,62 +474,64 @@ struct LaneSteps {
     }
 };
 
-// Steps and step-cap stops of a wave's stopped paths, summed in its own words of LDS for the two
+// Steps and step-cap stops of a wave's stopped paths, summed in its own words of LDS for the eight
 // knots that its pool came to last, and added to their counters (Records::kacc) one atomic to a
-// wave and knot: when the pool comes to a third knot, and at the end.  A path of another knot (a long one, or
+// wave and knot: when the pool comes to a ninth knot, and at the end.  A path of another knot (a long one, or
 // of knots of a few paths) adds its own.  Atomics of one address wait for each other and the loads
 // of a lane's next knot wait for them: with a sum per lane, 64 to a wave and knot, 2 10^6 FP32
-// paths of 16 points (plain step, some 150 steps each) took 4.7 ms, and take 1.8 so.  The kernels that
-// read a table, and the group kernel, keep LaneSteps: they wait for their reads more than for these atomics (2 10^6
-// paths of 16 or 2000 points, h = 1e-3, LUT or table: 28 to 37 ms either way), and with the wave's words the
-// compiler orders the table's FP32 plain step worse (2000 points: 39.8 ms, 34.7 so).
+// paths of 16 points (plain step, some 50 and 250 steps each) took 5.0 and 5.8 ms, and take 1.05 and 3.0 so.
+// A wave's lanes are on paths of several chunks, each of other knots where knots have a few thousand paths:
+// with words for two knots the same launch took 1.5 and 3.1 ms, and 1.4 10^6 paths of 340 knots 1.97 (1.67 so).
+// The kernels that read a table, and the group kernel, keep LaneSteps: they wait for their reads more
+// than for these atomics (2 10^6 paths of 16 or 2000 points, h = 1e-3, LUT or table: 28 to 37 ms either way),
+// and with the wave's words the compiler orders the table's FP32 plain step worse (2000 points: 39.8 ms,
+// 34.7 so).
 struct KnotSteps {
-    static constexpr int words = 4;    // of LDS to a wave: steps and cap stops of two knots
+    static constexpr int slots = 8;
+    static constexpr int words = 3 * slots;    // of LDS to a wave: a knot, its steps and cap stops
     unsigned long long *acc;     // the wave's words
-    int k;                       // the lane's knot
-    int kn, ko, sn;              // wave-uniform: the newer and the older knot, the newer one's slot
+    int k, slot;                 // the lane's knot, and its slot when the lane came to it (-1: it had none)
+    int kn, sn;                  // wave-uniform: the newest knot and its slot
 
     __device__ __forceinline__ void init(unsigned long long *lds, int lane) {
         acc = lds + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * words;
-        if (lane < words) acc[lane] = 0ULL;
-        k = kn = ko = -1;
+        if (lane < words) __hip_atomic_store(acc + lane, lane < slots ? ~0ULL : 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        k = kn = -1;
+        slot = -1;
         sn = 0;
     }
     __device__ __forceinline__ void add_global(const PathKernelArgs &a, int knot, unsigned long long st, unsigned long long cap) const {
         if (st) atomicAdd(a.rec.kacc + 2 * (int64_t)knot, st);
         if (cap) atomicAdd(a.rec.kacc + 2 * (int64_t)knot + 1, cap);
     }
-    // the sums of one slot into its knot's counters (by the whole wave)
-    __device__ __forceinline__ void flush_slot(const PathKernelArgs &a, int slot, int knot, int lane) {
-        if (lane != 0 || knot < 0) return;
-        unsigned long long *w = acc + 2 * slot;
-        const unsigned long long st = __hip_atomic_exchange(w, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const unsigned long long cap = __hip_atomic_exchange(w + 1, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        add_global(a, knot, st, cap);
+    // a slot's sums into its knot's counters; kk takes the slot (one lane)
+    __device__ __forceinline__ void flush_slot(const PathKernelArgs &a, int s, unsigned long long kk) {
+        const unsigned long long knot = __hip_atomic_exchange(acc + s, kk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const unsigned long long st = __hip_atomic_exchange(acc + slots + s, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const unsigned long long cap = __hip_atomic_exchange(acc + 2 * slots + s, 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        add_global(a, (int)knot, st, cap);
     }
     // the wave's pool comes to knot kk (wave-uniform; by the whole wave)
     __device__ __forceinline__ void open(const PathKernelArgs &a, int kk, int lane) {
-        if (kk == kn || kk == ko) return;
-        sn ^= 1;
-        flush_slot(a, sn, ko, lane);
-        ko = kn;
+        if (kk == kn) return;
+        sn = (sn + 1) & (slots - 1);
         kn = kk;
+        if (lane == 0) flush_slot(a, sn, (unsigned long long)kk);
     }
     // the lane goes on to paths of knot kk
-    __device__ __forceinline__ void enter(const PathKernelArgs &, int kk) { k = kk; }
+    __device__ __forceinline__ void enter(const PathKernelArgs &, int kk) { k = kk; slot = kk == kn ? sn : -1; }
     // a lane's path has stopped
     __device__ __forceinline__ void add(const PathKernelArgs &a, uint32_t st, bool cap) const {
-        if (k == kn || k == ko) {
-            unsigned long long *w = acc + 2 * (k == kn ? sn : sn ^ 1);
-            (void)__hip_atomic_fetch_add(w, (unsigned long long)st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (cap) (void)__hip_atomic_fetch_add(w + 1, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const int s = k == kn ? sn : slot;
+        if (s >= 0 && (int)__hip_atomic_load(acc + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == k) {
+            (void)__hip_atomic_fetch_add(acc + slots + s, (unsigned long long)st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (cap) (void)__hip_atomic_fetch_add(acc + 2 * slots + s, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         } else {
             add_global(a, k, st, cap ? 1ULL : 0ULL);
         }
     }
     __device__ __forceinline__ void flush(const PathKernelArgs &a, int lane) {
-        flush_slot(a, sn, kn, lane);
-        flush_slot(a, sn ^ 1, ko, lane);
+        if (lane < slots) flush_slot(a, lane, ~0ULL);
     }
 };
 

@@ -1,5 +1,5 @@
 """Step and step-cap sums of the persistent path kernel (one lane to a path), which a wave holds for
-the two knots its pool came to last: knots of one path, of fewer than a wave takes at once and of
+the eight knots its pool came to last: knots of one path, of fewer than a wave takes at once and of
 many, one after another in one launch; a step cap that stops some paths.  Sums and results are
 the plain kernel's."""
 import numpy as np
