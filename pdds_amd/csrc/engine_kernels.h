@@ -24,7 +24,6 @@
 //    items of each knot in item order.  Every sum has a fixed order: results do
 //    not depend on scheduling.
 #pragma once
-#include <type_traits>
 #include "pdds_pde.h"
 #include "engine_types.h"
 
@@ -482,10 +481,8 @@ struct LaneSteps {
 // paths of 16 points (plain step, some 50 and 250 steps each) took 5.0 and 5.8 ms, and take 1.05 and 3.0 so.
 // A wave's lanes are on paths of several chunks, each of other knots where knots have a few thousand paths:
 // with words for two knots the same launch took 1.5 and 3.1 ms, and 1.4 10^6 paths of 340 knots 1.97 (1.67 so).
-// The kernels that read a table, and the group kernel, keep LaneSteps: they wait for their reads more
-// than for these atomics (2 10^6 paths of 16 or 2000 points, h = 1e-3, LUT or table: 28 to 37 ms either way),
-// and with the wave's words the compiler orders the table's FP32 plain step worse (2000 points: 39.8 ms,
-// 34.7 so).
+// 9.6 10^5 FP32 paths of 16 points of the LUT problem, 25 steps each: 2.65 ms and 1.34 so.  The tiled kernel has
+// no LDS to spare for these words, and the group kernel's waves hold fewer paths: they keep LaneSteps.
 struct KnotSteps {
     static constexpr int slots = 8;
     static constexpr int words = 3 * slots;    // of LDS to a wave: a knot, its steps and cap stops
@@ -535,9 +532,6 @@ struct KnotSteps {
     }
 };
 
-template <int PDE>
-using PathSteps = std::conditional_t<PDE == PDE_VARCOEF_LUT || PDE == PDE_TABLE, LaneSteps, KnotSteps>;
-
 // Distance to a stencil's stopping domain: its rectangle, or its annular sector on a disc mesh.
 template <class R, int GEOM>
 __device__ __forceinline__ R domain_dist(const R *dom, R x, R y, R &ex, R &ey, R &nx, R &ny, int &kind) {
@@ -555,7 +549,8 @@ template <int GEOM> constexpr int domain_len() { return GEOM == GeomDisc ? 6 : 4
 // REFL: some global sides reflect (rectangles only): the path carries its nearest side (distance,
 // kind, outward normal) and the local time of a projection, and steps with refl_step while that
 // side reflects; only absorbing sides stop it.
-template <class R, int PDE, bool MIXED, int GEOM, int FAM, bool REFL = false>
+// STEPS: how the steps of stopped paths are summed (LaneSteps, KnotSteps).
+template <class R, int PDE, bool MIXED, int GEOM, int FAM, bool REFL = false, class STEPS = LaneSteps>
 struct Walker {
     // rectangles without reflecting sides: the stopping test without branches, the exit projection
     // and side formed by the stopping lanes alone; fast: also lanes that are not stepping kept out by
@@ -579,7 +574,7 @@ struct Walker {
     // local time
     int rmask, rk;
     R rd, rnx, rny, lt;
-    PathSteps<PDE> ks;     // the lane's knot, and the steps of stopped paths not yet added to their counters
+    STEPS ks;              // the lane's knot, and the steps of stopped paths not yet added to their counters
 
     __device__ __forceinline__ void init(unsigned long long *step_words = nullptr, int lane = 0) {
         // (a lane's first step, with zero coefficients, still takes the normals: they must be finite)
@@ -837,13 +832,9 @@ template <class R, int PDE, bool MIXED, int GEOM, int FAM, bool REFL = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(path_waves_f<R, PDE, FAM>()))) path_kernel(PathKernelArgs a) {
     const int lane = __lane_id();
     const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
-    Walker<R, PDE, MIXED, GEOM, FAM, REFL> w;
-    if constexpr (PathSteps<PDE>::words > 0) {
-        __shared__ unsigned long long step_words[4 * PathSteps<PDE>::words];
-        w.init(step_words, lane);
-    } else {
-        w.init();
-    }
+    Walker<R, PDE, MIXED, GEOM, FAM, REFL, KnotSteps> w;
+    __shared__ unsigned long long step_words[4 * KnotSteps::words];
+    w.init(step_words, lane);
     bool done = false;
     // The wave starts on its XCD's queue, so the paths (and LUT texels) of one XCD's L2
     // stay in one contiguous range of knots; a drained queue sends the wave on to the next.

@@ -29,12 +29,16 @@ def _counts(kind):
 # (forms without several lanes to a path: the plain step, and FP32 paths with a reflecting side)
 @pytest.mark.parametrize("precision,pde,step,neumann,cap", [("fp64", "helmholtz", 1, 0, 0), ("fp32", "helmholtz", 1, 0, 0),
                                                             ("fp64", "varcoef", 1, 0, 30), ("fp32", "varcoef", 1, 0, 30),
-                                                            ("fp32", "monegros", 1, 0, 0), ("fp32", "helmholtz", 0, 8, 0)])
+                                                            ("fp32", "monegros", 1, 0, 0), ("fp32", "helmholtz", 0, 8, 0),
+                                                            ("fp64", "varcoef_lut", 1, 0, 0), ("fp32", "varcoef_lut", 1, 0, 25),
+                                                            ("fp64", "table", 1, 0, 25), ("fp64", "table", 2, 0, 0)])
 def test_step_sums_equal_plain(eng, kind, precision, pde, step, neumann, cap):
     from pdds_amd.engine import bvp, default_run
     n = _counts(kind)
     x, y = np.linspace(-0.9, 0.8, len(n)), np.linspace(0.7, -0.6, len(n))
-    prob = bvp(pde, neumann=neumann)
+    from pdds_amd.workloads import table_problem, varcoef_lut
+    prob = {"varcoef_lut": lambda: bvp(pde, lut=varcoef_lut(eng, 64, tuple(GLOB))),
+            "table": lambda: table_problem(eng, 64, tuple(GLOB))}.get(pde, lambda: bvp(pde, neumann=neumann))()
     run = dict(h=5e-3, seed=3, precision=precision, wg_size=128, step=step, max_steps=cap)
     print(kind, precision, pde, step, neumann, cap, flush=True)
     a, b = (eng.point_eval(prob, default_run(plain=p, **run), GLOB, x, y, n) for p in (0, 1))
