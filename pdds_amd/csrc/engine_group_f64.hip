@@ -14,13 +14,13 @@ namespace pdds {
 // paths 0.73 and 0.58, 4000 0.34 and 0.29.
 // Lanes that read a table repeat the reads of their path's other lanes, which pays while a launch lasts as
 // long as its longest path.  By groups and by one lane in the persistent kernel: the tabulated problem's
-// 32 reads of 16 bytes a step (4 x 4 subdomains, 128 x 128 texels, h = 2e-4) FP64 6 10^4 paths 3.4 and 4.0 ms,
-// 1.2 10^5 4.1 and 4.3, 2 10^5 5.7 and 5.1; FP32 2.65 and 3.1, 4.8 and 5.1, 6.3 and 5.6, and with 512 x 512
-// texels on 8 x 8 3.6 and 3.1, 6.0 and 3.6, 7.9 and 4.6.  The LUT's 20 reads (4 x 4 subdomains and points
-// on the whole square, 64 x 64 samples, h = 1e-3 of the domain): FP64 6.5 10^4 paths 14.1 and 17.1, 5.2 and
-// 5.1, 10^5 15.4 and 17.1, 6.5 and 6.8, 1.3 10^5 17.5 and 19.5, 6.5 and 6.9, 5 10^5 27 and 23, 13.8 and 10.5;
-// FP32 11.4 and 14.5, 2.7 and 3.0, 11.8 and 14.6, 4.0 and 3.0, 13.5 and 14.7, 4.2 and 3.1, 21 and 19, 9.5 and
-// 6.6; with 512 x 512 samples 10^5 FP64 17.7 and 17.5, 8.1 and 7.1, FP32 13.5 and 15.6, 6.3 and 3.6.
+// 32 reads of 16 bytes a step (h = 2e-4; 4 x 4 subdomains, 128 x 128 texels) FP64 6 10^4 paths 3.4 and 4.0 ms,
+// 1.2 10^5 4.3 and 4.4, 2 10^5 5.2 and 5.2; FP32 2.7 and 3.0, 5.1 and 5.1, 6.2 and 5.6, and with 512 x 512
+// texels on 8 x 8 1.0 and 0.73, 1.6 and 0.96, 2.2 and 1.15.  The LUT's 20 reads (4 x 4 subdomains and points
+// on the whole square, 64 x 64 samples, h = 1e-3 of the domain): FP64 6.5 10^4 paths 14.5 and 16.8, 5.2 and
+// 5.1, 10^5 15.9 and 16.9, 6.7 and 6.7, 1.3 10^5 17.1 and 19.3, 6.6 and 6.8, 5 10^5 27 and 23, 13.5 and 10.2;
+// FP32 11.5 and 15.0, 2.7 and 3.0, 12.5 and 14.9, 4.0 and 3.1, 13.7 and 15.2, 4.2 and 3.2, 20 and 19, 9.1 and
+// 6.6; with 512 x 512 samples 10^5 FP64 17.4 and 17.3, 8.3 and 7.0, FP32 13.7 and 15.4, 6.4 and 3.7.
 int group_lanes(int pde, int precision, bool refl, int n_cu, int64_t paths) {
     const bool fp64 = precision == PDDS_FP64;
     const bool moves = pde == PDE_SINSIN || pde == PDE_HELMHOLTZ || pde == PDE_MONEGROS;   // const_motion

@@ -256,23 +256,25 @@ hipError_t launch_path_tiled_f32(int pde, int geom, bool mixed, int grid, size_t
 // Whether a launch of the tabulated problem takes the LDS-tiled kernel, by its paths, the lanes of the
 // tiled grid (131072 on 256 CUs) and the share of paths whose tile fits.  Where all fit, from four paths a
 // lane on: 357 knots of 8 x 8 or 4 x 4 subdomains, 128 x 128 texels, FP64, h = 2e-4 and 2e-3 of the
-// subdomain: 5.2 10^5 paths 9.2 and 1.13 ms, persistent kernel 8.4 and 1.07 (VR + CV 14.3 and 1.87,
-// 13.6 and 2.06; FP32 6.3 and 0.73, 8.2 and 1.0); 10^6 9.3 and 1.14, 11.3 and 1.4; 3 10^5 8.6 and 1.14,
-// 6.0 and 0.88.  The patch without a tile is worked on last, by all, with the tiled kernel's thin grid: where
-// 3 of 100 paths have none, 2.5 10^6 paths take 2.85 ms (2.58), 8 10^6 5.0 (6.6); where none fits (512 x 512
-// texels) 8 10^6 take 9.0 ms (8.1), 2 10^5 17.8 (5.4).
+// subdomain: 5.2 10^5 paths 9.2 and 1.15 ms, persistent kernel 8.7 and 1.08 (VR + CV 14.4 and 1.83,
+// 13.7 and 2.02; FP32 6.4 and 0.73, 8.1 and 1.0); 10^6 10.0 and 1.18, 11.1 and 1.33; 3 10^5 8.6 and 1.14,
+// 6.3 and 0.85.  The patch without a tile is worked on last, by all, with the tiled kernel's thin grid: where
+// 3 of 100 paths have none, 2.5 10^6 paths take 2.9 ms (2.7), 8 10^6 5.1 (6.9); where none fits (512 x 512
+// texels) 4.7 (3.0) and 11.0 (8.8).
 inline bool tabulated_tiles(int64_t paths, int64_t lanes, double fitting) {
     return fitting >= 1.0 ? paths >= 4 * lanes : fitting >= 0.9 && paths >= 32 * lanes;
 }
 // The same of the coefficient LUT (lanes: 131072, FP32 rectangles 196608).  Each pair: tiled and persistent
 // kernel, at h = 1e-2 of the subdomain's size squared, and where two follow, at 1e-3.  FP64: 2 10^6 paths
-// 4.8 and 4.7 ms, 46 and 42 (8 x 8 subdomains of 32 knots, 256 x 256 samples, all tiles fit), 6.8 and 5.9,
-// 59 and 62 (512 x 512, a few tiles do not); 6 10^6 paths 9.7 and 10.1, 10.9 and 12.9 (64 x 64: 9.8 and 9.1);
-// 1.5 10^7 18.9 and 21.9, 18.8 and 28.2; where none fits (4 x 4) 6 10^6 take 14.4 and 14.7, 1.5 10^7 32.7 and
-// 34.3.  FP32 (4 x 4, 128 x 128, at 5e-3 and 1e-3): 5.4 10^5 paths 4.6 and 3.8, 24 and 21, 7.7 10^5 4.7 and
-// 4.5, 24 and 23, 10^6 4.5 and 5.5, 21 and 25 (256 x 256 on 8 x 8 4.3 and 5.4, 21 and 27); where a few tiles do not fit 2 10^6 6.7 and 5.5, 58 and 48, 6 10^6 8.6 and 12.2; where none
-// fits 15.9 and 13.6 (6 10^6), 34.8 and 32.1 (1.5 10^7).  Discs of 24 to 144 sectors, FP32: 2 10^6 paths 1.0
-// and 1.5, 1.5 and 1.3, 6 10^6 1.9 and 3.1, 2.0 and 2.2.
+// 4.9 and 4.8 ms, 47 and 44 (8 x 8 subdomains of 32 knots, 256 x 256 samples, all tiles fit), 7.0 and 5.8,
+// 60 and 59 (512 x 512, a few tiles do not); 6 10^6 paths 9.8 and 9.7, 11.4 and 13.0 (64 x 64: 9.8 and 8.9);
+// 1.5 10^7 18.3 and 21.5, 18.5 and 27.4; where none fits (4 x 4) 6 10^6 take 14.1 and 14.2, 1.5 10^7 32.0 and
+// 33.3.  FP32 (4 x 4, 128 x 128, at 5e-3 and 1e-3): 5.4 10^5 paths 4.6 and 3.7, 23 and 21, 7.7 10^5 4.8 and
+// 4.8, 24 and 24, 10^6 4.5 and 5.0, 20 and 26 (256 x 256 on 8 x 8 4.3 and 5.5, 22 and 24); where a few tiles
+// do not fit 2 10^6 7.0 and 5.2, 55 and 47, 6 10^6 8.5 and 12.1; where none fits 15.5 and 13.1 (6 10^6), 34.1
+// and 31.2 (1.5 10^7).  Discs of 24 and 144 sectors, 64 x 64: FP32 2 10^6 paths 1.0 and 1.4, 1.6 and 1.2, 6 10^6
+// 1.9 and 2.6, 2.0 and 2.1; FP64 2 10^6 2.2 and 2.0, 2.2 and 1.7, 6 10^6 3.9 and 3.6, 3.4 and 2.9, 1.5 10^7 7.8
+// and 6.9, 6.1 and 5.8.
 inline bool lut_tiles(bool fp64, bool rect, int64_t paths, int64_t lanes, double fitting) {
     if (fp64) return paths >= 24 * lanes;
     return fitting >= 0.75 && paths >= (rect && fitting >= 1.0 ? 4 : 16) * lanes;
