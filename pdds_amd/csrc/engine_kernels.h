@@ -24,6 +24,7 @@
 //    items of each knot in item order.  Every sum has a fixed order: results do
 //    not depend on scheduling.
 #pragma once
+#include <type_traits>
 #include "pdds_pde.h"
 #include "engine_types.h"
 
@@ -473,18 +474,19 @@ struct LaneSteps {
     }
 };
 
-// Steps and step-cap stops of a wave's stopped paths, summed in its own words of LDS for the eight
-// knots that its pool came to last, and added to their counters (Records::kacc) one atomic to a
-// wave and knot: when the pool comes to a ninth knot, and at the end.  A path of another knot (a long one, or
+// Steps and step-cap stops of a wave's stopped paths, summed in its own words of LDS for the SLOTS (a power
+// of two) knots that its pool came to last, and added to their counters (Records::kacc) one atomic to a
+// wave and knot: when the pool comes to one more, and at the end.  A path of another knot (a long one, or
 // of knots of a few paths) adds its own.  Atomics of one address wait for each other and the loads
 // of a lane's next knot wait for them: with a sum per lane, 64 to a wave and knot, 2 10^6 FP32
 // paths of 16 points (plain step, some 50 and 250 steps each) took 5.0 and 5.8 ms, and take 1.05 and 3.0 so.
 // A wave's lanes are on paths of several chunks, each of other knots where knots have a few thousand paths:
 // with words for two knots the same launch took 1.5 and 3.1 ms, and 1.4 10^6 paths of 340 knots 1.97 (1.67 so).
 // 9.6 10^5 FP32 paths of 16 points of the LUT problem, 25 steps each: 2.65 ms and 1.34 so.  The tiled kernel has
-// no LDS to spare for these words, and the group kernel's waves hold fewer paths: they keep LaneSteps.
+// LDS to spare for two knots a wave (TiledSteps).  The group kernel's waves hold fewer paths: LaneSteps.
+template <int SLOTS>
 struct KnotSteps {
-    static constexpr int slots = 8;
+    static constexpr int slots = SLOTS;
     static constexpr int words = 3 * slots;    // of LDS to a wave: a knot, its steps and cap stops
     unsigned long long *acc;     // the wave's words
     int k, slot;                 // the lane's knot, and its slot when the lane came to it (-1: it had none)
@@ -832,8 +834,8 @@ template <class R, int PDE, bool MIXED, int GEOM, int FAM, bool REFL = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(path_waves_f<R, PDE, FAM>()))) path_kernel(PathKernelArgs a) {
     const int lane = __lane_id();
     const LutTile none{nullptr, 0, 0, 0, 0, 0, 0, 0};
-    Walker<R, PDE, MIXED, GEOM, FAM, REFL, KnotSteps> w;
-    __shared__ unsigned long long step_words[4 * KnotSteps::words];
+    Walker<R, PDE, MIXED, GEOM, FAM, REFL, KnotSteps<8>> w;
+    __shared__ unsigned long long step_words[4 * KnotSteps<8>::words];
     w.init(step_words, lane);
     bool done = false;
     // The wave starts on its XCD's queue, so the paths (and LUT texels) of one XCD's L2
@@ -968,6 +970,13 @@ template <class R, int PDE, int FAM, int GEOM> constexpr int tiled_waves() {
 }
 template <class R, int PDE, int FAM, int GEOM> constexpr int tiled_wg() { return 64 * 4 * tiled_waves<R, PDE, FAM, GEOM>(); }
 
+// How the tiled kernel sums steps: FP32 control-variate launches of the LUT problem by wave (3.2 10^6 paths of 16
+// points, 25 and 250 steps each, 8.2 and 12.8 ms with a sum per lane, 1.4 and 10.6 so; 3437 knots the same
+// either way), the others by lane (FP64 control variates lose 2 % of 3437 knots with the wave's sums,
+// and gain on few knots alone).
+template <class R, int PDE, int FAM>
+using TiledSteps = std::conditional_t<sizeof(R) == 4 && PDE == PDE_VARCOEF_LUT && FAM == STEP_CV, KnotSteps<2>, LaneSteps>;
+
 __device__ __forceinline__ int find_patch(const PatchDesc *p, int n, int64_t g) {
     int lo = 0, hi = n;
     while (hi - lo > 1) {
@@ -984,8 +993,17 @@ path_kernel_tiled(PathKernelArgs a) {
     extern __shared__ float4 tile[];
     __shared__ int s_patch;
     const int lane = __lane_id();
-    Walker<R, PDE, MIXED, GEOM, FAM> w;
-    w.init();
+    using Steps = TiledSteps<R, PDE, FAM>;
+    Walker<R, PDE, MIXED, GEOM, FAM, false, Steps> w;
+    if constexpr (Steps::words > 0) {
+        // (with s_patch within the KiB that plan_tiles leaves)
+        constexpr int n_words = tiled_wg<R, PDE, FAM, GEOM>() / 64 * Steps::words;
+        static_assert(n_words * sizeof(unsigned long long) <= 1000, "step sums past the LDS that the tiles leave");
+        __shared__ unsigned long long step_words[n_words];
+        w.init(step_words, lane);
+    } else {
+        w.init();
+    }
     // first patch: the one holding this work-group's share of the batch's path range
     int p = find_patch(a.patches, a.n_patches, (int64_t)blockIdx.x * a.total / (int64_t)gridDim.x);
     bool first = true;

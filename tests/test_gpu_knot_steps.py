@@ -1,5 +1,5 @@
-"""Step and step-cap sums of the persistent path kernel (one lane to a path), which a wave holds for
-the eight knots its pool came to last: knots of one path, of fewer than a wave takes at once and of
+"""Step and step-cap sums of the persistent and tiled path kernels (one lane to a path), which a wave holds for
+the knots its pool came to last: knots of one path, of fewer than a wave takes at once and of
 many, one after another in one launch; a step cap that stops some paths.  Sums and results are
 the plain kernel's."""
 import numpy as np
@@ -43,6 +43,27 @@ def test_step_sums_equal_plain(eng, kind, precision, pde, step, neumann, cap):
     print(kind, precision, pde, step, neumann, cap, flush=True)
     a, b = (eng.point_eval(prob, default_run(plain=p, **run), GLOB, x, y, n) for p in (0, 1))
     assert a["counters"]["wg_size"] == 128
+    for k in ("path_steps", "paths", "exits", "capped"):
+        assert a["counters"][k] == b["counters"][k], k
+    assert np.array_equal(a["u"], b["u"]) and np.array_equal(a["u_var"], b["u_var"])
+    assert (a["counters"]["capped"] > 0) == (cap > 0)
+
+
+@pytest.mark.parametrize("kind", ["ones", "mixed", "one"])
+@pytest.mark.parametrize("cap", [0, 25])
+def test_tiled_step_sums_equal_persistent(eng, kind, cap):
+    """The tiled kernel's FP32 sums, for the two knots a wave came to last."""
+    from pdds_amd.engine import bvp, default_run
+    from pdds_amd.workloads import varcoef_lut
+    # above four paths a lane of the tiled grid
+    extra = eng.info()["n_cu"] * 768 * 4
+    n = np.append(_counts(kind), [extra // 3, 7, extra])
+    x, y = np.linspace(-0.9, 0.8, len(n)), np.linspace(0.7, -0.6, len(n))
+    prob = bvp("varcoef_lut", lut=varcoef_lut(eng, 64, tuple(GLOB)))
+    print(kind, cap, flush=True)
+    a, b = (eng.point_eval(prob, default_run(h=1e-2, seed=3, precision="fp32", wg_size=128, lut_lds=lds, max_steps=cap),
+                           GLOB, x, y, n) for lds in (1, 0))
+    assert a["counters"]["wg_size"] == 768 and b["counters"]["wg_size"] == 128
     for k in ("path_steps", "paths", "exits", "capped"):
         assert a["counters"][k] == b["counters"][k], k
     assert np.array_equal(a["u"], b["u"]) and np.array_equal(a["u_var"], b["u_var"])
